@@ -82,6 +82,48 @@ __device__ __forceinline__ float activate(float v, int act) {
   return v * sg;
 }
 
+// Four result columns n .. n + 3 of one row (row_at: element offset of the row) through the bias /
+// activation epilogue, stored as f32 or in the storage dtype.  vec: the row takes one vector store;
+// otherwise (a row on any boundary, N not a multiple of 4) element by element inside N.
+template <class T, int EPI>
+__device__ __forceinline__ void store_quad(void* __restrict__ D, long row_at, int n, int N, float4 v,
+                                           const float* __restrict__ bias, int act, int vec) {
+  if (n >= N) return;
+  float e[4] = {v.x, v.y, v.z, v.w};
+  if (bias) {
+    if (vec) {
+      const float4 bv = *reinterpret_cast<const float4*>(bias + n);
+      e[0] += bv.x; e[1] += bv.y; e[2] += bv.z; e[3] += bv.w;
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e[u] += bias[n + u < N ? n + u : n];
+    }
+  }
+  if (act != ACT_NONE) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) e[u] = activate(e[u], act);
+  }
+  if constexpr (EPI == EPI_F32) {
+    float* d = reinterpret_cast<float*>(D) + row_at + n;
+    if (vec) {
+      *reinterpret_cast<float4*>(d) = make_float4(e[0], e[1], e[2], e[3]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (n + u < N) d[u] = e[u];
+    }
+  } else {
+    uint16_t* d = reinterpret_cast<uint16_t*>(D) + row_at + n;
+    if (vec) {
+      *reinterpret_cast<uint2*>(d) = make_uint2(pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3]));
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (n + u < N) d[u] = to_storage<T>(e[u]);
+    }
+  }
+}
+
 struct Gemm16Params {
   const uint16_t* A;
   const uint16_t* B;

@@ -98,16 +98,16 @@ int launch_gemm16_tile(Gemm16Params p, hipStream_t s, int wg_limit = 0) {
   return launch_status();
 }
 
-// D[m][n] = sum over splits (in split order) of the f32 partials, stored as f32 or in
-// the storage dtype; four columns per thread (N % 8 == 0 on this path).
+// D[m][n] = sum over splits (in split order) of the f32 partials ws[splits][M][ldw], then bias and activation,
+// stored as f32 or in the storage dtype; four columns per thread.
 template <class T, int EPI>
-__global__ void splitk_reduce_kernel(const float* __restrict__ ws, void* __restrict__ D, int M, int N, long ldd,
-                                     int splits, const float* __restrict__ bias, int act) {
+__global__ void splitk_reduce_kernel(const float* __restrict__ ws, void* __restrict__ D, int M, int N, long ldw, long ldd,
+                                     int splits, const float* __restrict__ bias, int act, int vec) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int nq = N / 4;
+  const int nq = (N + 3) / 4;
   if (i >= (long)M * nq) return;
   const int m = (int)(i / nq), n = (int)(i % nq) * 4;
-  const size_t mn = (size_t)M * N;
+  const size_t slice = (size_t)M * ldw;
   // (the partials of four splits are fetched together: they were written by other
   // XCDs, so every one of these loads pays a trip to memory)
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -115,25 +115,19 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ ws, void* __restr
     float4 v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      v[u] = z0 + u < splits ? *reinterpret_cast<const float4*>(ws + (z0 + u) * mn + (size_t)m * N + n)
+      v[u] = z0 + u < splits ? *reinterpret_cast<const float4*>(ws + (z0 + u) * slice + (size_t)m * ldw + n)
                              : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int u = 0; u < 4; ++u) { acc.x += v[u].x; acc.y += v[u].y; acc.z += v[u].z; acc.w += v[u].w; }
   }
-  if (bias) {
-    const float4 bv = *reinterpret_cast<const float4*>(bias + n);
-    acc.x += bv.x; acc.y += bv.y; acc.z += bv.z; acc.w += bv.w;
-  }
-  acc.x = activate(acc.x, act); acc.y = activate(acc.y, act);
-  acc.z = activate(acc.z, act); acc.w = activate(acc.w, act);
-  if constexpr (EPI == EPI_F32) {
-    *reinterpret_cast<float4*>(reinterpret_cast<float*>(D) + (long)m * ldd + n) = acc;
-  } else {
-    uint2 pk;
-    pk.x = pack2<T>(acc.x, acc.y);
-    pk.y = pack2<T>(acc.z, acc.w);
-    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(D) + (long)m * ldd + n) = pk;
-  }
+  store_quad<T, EPI>(D, (long)m * ldd, n, N, acc, bias, act, vec);
+}
+template <class T, int EPI>
+int launch_splitk_reduce(const float* ws, long ldw, const Gemm16Params& p, int splits, int vec, hipStream_t s) {
+  const long quads = (long)p.M * ((p.N + 3) / 4);
+  hipLaunchKernelGGL((splitk_reduce_kernel<T, EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, ws, p.D, p.M,
+                     p.N, ldw, p.ldd, splits, p.bias, p.act, vec);
+  return launch_status();
 }
 
 // Tile and split-K choice of the dense 16-bit GEMM for an aligned problem — the one
@@ -142,11 +136,13 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ ws, void* __restr
 struct Gemm16Schedule {
   int tile;      // workgroup tile edge: 256, 128 or 64 (square unless tile_m says otherwise)
   int split_k;   // number of K splits (1 = none)
-  bool skinny;   // M <= 8: the streaming kernel (32 x 64 workgroup tile, K slices of 32)
+  bool skinny;   // the few-row streaming kernel (32 x 64 workgroup tile up to 8 rows, 32 x 128 above; K slices of 32)
   int rest_split = 1;   // 256 tiles, split_k 1: K splits of the tiles beyond the last full round of 256
   int tile_m = 0;       // 128 with tile 256: the 128 x 256 tile (tile rows x tile columns); 0: square
 };
-constexpr int kSkinnyMaxM = 8;
+constexpr int kSkinnyMaxM = 8;           // 64-column strips up to here,
+constexpr int kSkinnyWideMaxM = 32;      // 128-column strips up to here
+constexpr int kLooseMaxM = 64;           // and for rows of B on any boundary up to here
 constexpr long kSplitTargetWgs = 768;
 constexpr int kWeightStreamMaxM = 128;   // up to here a product is bound by reading B once
 
@@ -200,6 +196,27 @@ inline double est_few_rows_us(const FewRowTile& t, int M, int N, int K, int spli
   const double stream = bytes / (t.tbs * 1e6 * std::min(1.0, wgs / 185.0));
   const double sum = splits > 1 ? 3.4 + (double)M * N * splits * 1.6e-6 : 0.0;
   return t.launch + std::max(compute, stream) + sum;
+}
+
+// Workgroups of the few-row kernel on 128-column strips with K in as many parts as keep it within one workgroup
+// per compute unit (a second round would be nearly empty), every wave with at least one slice.
+inline int skinny_wide_splits(int N, int K) {
+  return std::max(1, std::min(256 / ceil_div(N, 128), K / 256));
+}
+// K splits for rows of B on any boundary, where the streaming kernel is the only one that reads B in place:
+// the fewest microseconds by an estimate fitted to forced splits over 512 to 16384 columns and 256 to
+// 14336 rows of B (a workgroup streams a 256-byte row in 7.5 ns, the chip 5.6 TB/s; a split adds a launch
+// and a sum, 3.6 us).
+inline int skinny_loose_splits(int N, int K) {
+  const int strips = ceil_div(N, 128), most = skinny_wide_splits(N, K);
+  int best = 1;
+  double best_us = 1e30;
+  for (int splits = 1; splits <= most; ++splits) {
+    const double rounds = ceil_div(strips * splits, 256) * 256.0 / std::max(256, strips * splits);
+    const double us = std::max(7.5e-3 * K / splits, 2.0 * K * N / 5.6e6) * rounds + (splits > 1 ? 3.6 : 0.0);
+    if (us < best_us) { best_us = us; best = splits; }
+  }
+  return best;
 }
 
 inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
@@ -289,24 +306,78 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     // splits keep that under about 0.4 of the operand traffic
     splits = (int)std::min<long>(splits, std::max<long>(2, (long)K * (M + N) / (10L * M * N)));
     while (splits > 1 && K % (splits * G16_BK) != 0) --splits;
+    // 9 to 32 rows: the streaming kernel on 128-column strips instead where its workgroups come out at
+    // nearly one per compute unit and B is more than a launch's worth of streaming (M = 16: 8192 x 8192
+    // 31.4 -> 28.1 us, 14336 x 4096 28.5 -> 25.8, 4096 x 4096 13.3 -> 11.4; level at 17 MB; at 186
+    // workgroups, 11840 columns, 20.9 against 22.8; with K ranges under 512, 16 x 2048 x 7168, 11.5 against
+    // 12.2), and where K has no even split that would give the tiles
+    // enough workgroups (27 x 3520 x 5312: 32.7 -> 13.7).
+    if (M <= kSkinnyWideMaxM && N >= 128) {
+      const int wide = skinny_wide_splits(N, K);
+      const long wgs = (long)ceil_div(N, 128) * wide;
+      if ((2.0 * K * N >= 2.4e7 && wgs >= 216 && wgs <= 256 && K >= 2048 && K / wide >= 512) || (K >= 2048 && tiles * splits < 128 && wgs > 2 * tiles * splits))
+        return {128, wide, true};
+    }
   }
   return {t128 ? 128 : 64, splits, false};
 }
 
-template <class T, int EPI>
-int launch_gemm16_skinny(const Gemm16Params& p, int kps, int splits, hipStream_t s) {
-  constexpr int MI = 1, NW = 8, NJ = 2, KS = 2;
-  auto kern = gemm16_skinny_kernel<T, MI, NW, NJ, KS, EPI>;
-  constexpr int lds = skinny_lds_bytes<MI, NW, NJ, KS>();
+template <class T, int MI, int NW, int NJ, int EPI, bool NT, bool LOOSE>
+int launch_gemm16_skinny_as(const Gemm16Params& p, int kps, int splits, float* part, int d_vec, hipStream_t s) {
+  auto kern = gemm16_skinny_kernel<T, MI, NW, NJ, EPI, NT, LOOSE>;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
-    attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   skinny_lds_bytes<NW, NJ>(32));
   });
   if (attr_err != hipSuccess) return kDeviceFailed;
-  hipLaunchKernelGGL(kern, dim3(ceil_div(p.N, 32 * NJ), splits), dim3(NW * 64), lds, s, p, kps);
+  hipLaunchKernelGGL(kern, dim3(ceil_div(p.N, 32 * NJ), splits), dim3(NW * 64), (skinny_lds_bytes<NW, NJ>(std::min(p.M, 32))), s, p,
+                     kps, part, d_vec);
   return launch_status();
+}
+
+// The few-row streaming kernel with K in `splits` parts.  loose: see the kernel; A is then copied into
+// rows padded with zeros to a multiple of 8 where its own cannot be read 16 bytes at a time.
+template <class T, int EPI>
+int launch_gemm16_skinny(Gemm16Params p, int splits, bool loose, hipStream_t s) {
+  const int cols = p.M <= kSkinnyMaxM && !loose ? 64 : 128;
+  const int kps = ceil_div(ceil_div(p.K, splits), 32) * 32;
+  splits = ceil_div(p.K, kps);
+  const long ldw = (long)ceil_div(p.N, cols) * cols;
+  const int K8 = (p.K + 7) & ~7;
+  const bool a_copy = loose && (p.K % 8 != 0 || p.lda % 8 != 0 || !aligned16(p.A));
+  const size_t a_bytes = a_copy ? (((size_t)p.M * K8 * 2 + 255) & ~size_t(255)) : 0;
+  const size_t part_bytes = splits > 1 ? (size_t)splits * p.M * ldw * 4 : 0;
+  char* ws = nullptr;
+  if (a_bytes + part_bytes) {
+    ws = static_cast<char*>(stream_workspace(s, a_bytes + part_bytes));
+    if (!ws) return kDeviceFailed;
+  }
+  float* part = splits > 1 ? reinterpret_cast<float*>(ws + a_bytes) : nullptr;
+  constexpr int dsz = EPI == EPI_F32 ? 4 : 2;
+  const int d_vec = p.N % 4 == 0 && (p.ldd * dsz) % (4 * dsz) == 0 && aligned16(p.D) && (!p.bias || aligned16(p.bias));
+  Gemm16Params q = p;
+  if (a_copy) {
+    hipLaunchKernelGGL(pad_rows_kernel<uint16_t>, copy_grid(p.M, K8, 8, 1), copy_block(), 0, s, reinterpret_cast<uint16_t*>(ws),
+                       (long)K8, 0L, p.A, p.lda, 0L, p.M, p.K, p.M);
+    if (int rc = launch_status(); rc != kOk) return rc;
+    q.A = reinterpret_cast<const uint16_t*>(ws);
+    q.lda = K8;
+  }
+  const bool nt = 2.0 * p.K * p.N >= kStreamOnceBytes;
+  int rc;
+  if (loose)
+    rc = p.M <= 32 ? launch_gemm16_skinny_as<T, 1, 8, 4, EPI, false, true>(q, kps, splits, part, d_vec, s)
+                   : launch_gemm16_skinny_as<T, 2, 4, 4, EPI, false, true>(q, kps, splits, part, d_vec, s);
+  else if (cols == 64)
+    rc = nt ? launch_gemm16_skinny_as<T, 1, 8, 2, EPI, true, false>(q, kps, splits, part, d_vec, s)
+            : launch_gemm16_skinny_as<T, 1, 8, 2, EPI, false, false>(q, kps, splits, part, d_vec, s);
+  else
+    rc = nt ? launch_gemm16_skinny_as<T, 1, 8, 4, EPI, true, false>(q, kps, splits, part, d_vec, s)
+            : launch_gemm16_skinny_as<T, 1, 8, 4, EPI, false, false>(q, kps, splits, part, d_vec, s);
+  if (rc != kOk || !part) return rc;
+  return launch_splitk_reduce<T, EPI>(part, ldw, p, splits, d_vec, s);
 }
 
 template <class T, int EPI>
@@ -416,6 +487,9 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
                    ((p.strideD * dsz) % 16 == 0) && aligned16(p.A) && aligned16(p.B) && aligned16(p.D) &&
                    (!p.bias || aligned16(p.bias));
   if (!vec) {
+    // few rows: the streaming kernel reads B where it lies
+    if (p.groups == 1 && p.M <= kLooseMaxM && p.N >= 8)
+      return launch_gemm16_skinny<T, EPI>(p, skinny_loose_splits(p.N, p.K), true, s);
     // small products go one thread per output element; above about 2^24 multiply-adds the
     // copies into aligned buffers cost less than that kernel loses
     if ((double)p.M * p.N * p.K * p.groups >= (double)(1L << 24) && p.M >= 16 && p.N >= 16 &&
@@ -451,7 +525,7 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
     return launch_gemm16_rest<T, EPI>(p, main_wgs, tiles - main_wgs, sch.rest_split, s);
   }
   const bool t128 = sch.tile == 128;
-  if (sch.skinny && sch.split_k == 1) return launch_gemm16_skinny<T, EPI>(p, p.K, 1, s);
+  if (sch.skinny) return launch_gemm16_skinny<T, EPI>(p, sch.split_k, false, s);
   // Every K split is one "batch" of the same kernel writing f32 partials, summed in
   // split order by a second kernel, so the result does not depend on scheduling.
   {
@@ -470,23 +544,12 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
       q.act = ACT_NONE;
       q.ldd = p.N;
       q.strideD = (long)mn;
-      int rc;
-      if (sch.skinny) {
-        // the skinny kernel takes the whole problem and splits K by blockIdx.y itself
-        q.K = p.K;
-        rc = launch_gemm16_skinny<T, EPI_F32>(q, ceil_div(ceil_div(p.K, splits), 32) * 32, splits, s);
-      } else {
-        rc = sch.tile == 256 && sch.tile_m == 128 ? launch_gemm16_tile<T, 128, 256, 2, 2, EPI_F32, false, kBigTileMfma>(q, s)
-             : sch.tile == 256 ? launch_gemm16_tile<T, 256, 256, 2, 2, EPI_F32, false, kBigTileMfma>(q, s)
-             : t128      ? launch_gemm16_tile<T, 128, 128, 2, 2, EPI_F32, false>(q, s)
-                         : launch_gemm16_tile<T, 64, 64, 2, 2, EPI_F32, false>(q, s);
-      }
-      if (rc == kOk) {
-        const long quads = (long)p.M * (p.N / 4);
-        hipLaunchKernelGGL((splitk_reduce_kernel<T, EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s,
-                           ws, p.D, p.M, p.N, p.ldd, splits, p.bias, p.act);
-        rc = launch_status();
-      }
+      const int rc =
+          sch.tile == 256 && sch.tile_m == 128 ? launch_gemm16_tile<T, 128, 256, 2, 2, EPI_F32, false, kBigTileMfma>(q, s)
+          : sch.tile == 256 ? launch_gemm16_tile<T, 256, 256, 2, 2, EPI_F32, false, kBigTileMfma>(q, s)
+          : t128      ? launch_gemm16_tile<T, 128, 128, 2, 2, EPI_F32, false>(q, s)
+                      : launch_gemm16_tile<T, 64, 64, 2, 2, EPI_F32, false>(q, s);
+      if (rc == kOk) return launch_splitk_reduce<T, EPI>(ws, p.N, p, splits, 1, s);
       return rc;
     }
   }

@@ -17,7 +17,7 @@
 // consecutive 32-byte k groups rather than one contiguous run.
 #pragma once
 #include <type_traits>
-#include "common.h"
+#include "host_util.h"
 
 namespace tsr950 {
 
@@ -435,64 +435,90 @@ template <class T> __device__ __forceinline__ float f8_to_f32(uint8_t c) {
   else return e4m3_to_f32(c);
 }
 
+// Raw accumulators of columns n .. n + 3 of row m through the product's epilogue.  vec: the rows of D (and
+// acc_out, col_scale) take vector accesses, otherwise element by element inside N.
+template <class T> using g8_elem = typename std::conditional<std::is_same<T, I8>::value, int32_t, float>::type;
+template <class T> using g8_quad = typename std::conditional<std::is_same<T, I8>::value, i32x4, f32x4>::type;
+template <class T, int EPI>
+__device__ __forceinline__ void gemm8_store_quad(const Gemm8Params& p, int m, int n, const g8_quad<T>& acc, int vec) {
+  if (n >= p.N) return;
+  const long o = (long)m * p.N + n;
+  auto store4 = [&](auto* d, auto e0, auto e1, auto e2, auto e3) __attribute__((always_inline)) {
+    using E = std::remove_pointer_t<decltype(d)>;
+    typedef E out4 __attribute__((ext_vector_type(4)));
+    if (vec) {
+      *reinterpret_cast<out4*>(d) = out4{e0, e1, e2, e3};
+    } else {
+      d[0] = e0;
+      if (n + 1 < p.N) d[1] = e1;
+      if (n + 2 < p.N) d[2] = e2;
+      if (n + 3 < p.N) d[3] = e3;
+    }
+  };
+  float v[4];
+  if constexpr (std::is_same<T, I8>::value) {
+    if constexpr (EPI == EPI8_I32) {
+      store4(reinterpret_cast<int32_t*>(p.D) + o, acc[0], acc[1], acc[2], acc[3]);
+      return;
+    } else {
+      if (p.acc_out) store4(p.acc_out + o, acc[0], acc[1], acc[2], acc[3]);
+      const float rs = p.row_scale[m];
+      float cs[4];
+      if (vec) {
+        const float4 t = *reinterpret_cast<const float4*>(p.col_scale + n);
+        cs[0] = t.x; cs[1] = t.y; cs[2] = t.z; cs[3] = t.w;
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) cs[u] = p.col_scale[n + u < p.N ? n + u : n];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = ((float)acc[u] * rs) * cs[u];
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = (acc[u] * p.scale_a) * p.scale_b;
+  }
+  if constexpr (EPI == EPI8_SCALED_BF16) {
+    uint16_t* d = reinterpret_cast<uint16_t*>(p.D) + o;
+    store4(d, f32_to_bf16_bits(v[0]), f32_to_bf16_bits(v[1]), f32_to_bf16_bits(v[2]), f32_to_bf16_bits(v[3]));
+  } else if constexpr (EPI != EPI8_I32) {
+    store4(reinterpret_cast<float*>(p.D) + o, v[0], v[1], v[2], v[3]);
+  }
+}
+
 // A product split along K: the slices' partial results (int32 accumulators, or f32 ones of the fp8
-// form computed with unit scales), [splits][M][N], are summed in slice order and passed through
+// form computed with unit scales), [splits][M][ldw], are summed in slice order and passed through
 // the product's epilogue.  int32 sums are exact, so the int8 forms give the bits of the unsplit
 // kernel; the f32 sum of the fp8 form is one fixed order.  Four columns per thread.
 template <class T, int EPI>
-__global__ __launch_bounds__(256) void gemm8_split_sum_kernel(const void* __restrict__ part, int splits, const Gemm8Params p) {
-  constexpr bool IS_I8 = std::is_same<T, I8>::value;
+__global__ __launch_bounds__(256) void gemm8_split_sum_kernel(const void* __restrict__ part, int splits, long ldw, int vec,
+                                                              const Gemm8Params p) {
+  using quad_t = g8_quad<T>;
   const long quad = (long)blockIdx.x * 256 + threadIdx.x;
-  const int nq = p.N / 4;
+  const int nq = (p.N + 3) / 4;
   if (quad >= (long)p.M * nq) return;
   const int m = (int)(quad / nq), n = (int)(quad - (long)m * nq) * 4;
-  const long o = (long)m * p.N + n, mn = (long)p.M * p.N;
-  float v[4];
-  if constexpr (IS_I8) {
-    // (the partials of four slices are fetched together: they were written by other XCDs, so every
-    // one of these loads pays a trip to memory)
-    int4 acc = make_int4(0, 0, 0, 0);
-    for (int z0 = 0; z0 < splits; z0 += 4) {
-      int4 a[4];
+  const g8_elem<T>* src = reinterpret_cast<const g8_elem<T>*>(part) + (long)m * ldw + n;
+  const long slice = (long)p.M * ldw;
+  // (the partials of four slices are fetched together: they were written by other XCDs, so every
+  // one of these loads pays a trip to memory)
+  quad_t acc = {0, 0, 0, 0};
+  for (int z0 = 0; z0 < splits; z0 += 4) {
+    quad_t a[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        a[u] = z0 + u < splits ? *reinterpret_cast<const int4*>(reinterpret_cast<const int32_t*>(part) + (z0 + u) * mn + o)
-                               : make_int4(0, 0, 0, 0);
+    for (int u = 0; u < 4; ++u)
+      a[u] = z0 + u < splits ? *reinterpret_cast<const quad_t*>(src + (z0 + u) * slice) : quad_t{0, 0, 0, 0};
 #pragma unroll
-      for (int u = 0; u < 4; ++u) { acc.x += a[u].x; acc.y += a[u].y; acc.z += a[u].z; acc.w += a[u].w; }
-    }
-    if constexpr (EPI == EPI8_I32) {
-      *reinterpret_cast<int4*>(reinterpret_cast<int32_t*>(p.D) + o) = acc;
-      return;
-    } else {
-      if (p.acc_out) *reinterpret_cast<int4*>(p.acc_out + o) = acc;
-      const float rs = p.row_scale[m];
-      const float4 cs = *reinterpret_cast<const float4*>(p.col_scale + n);
-      v[0] = ((float)acc.x * rs) * cs.x; v[1] = ((float)acc.y * rs) * cs.y;
-      v[2] = ((float)acc.z * rs) * cs.z; v[3] = ((float)acc.w * rs) * cs.w;
-    }
-  } else {
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int z0 = 0; z0 < splits; z0 += 4) {
-      float4 a[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        a[u] = z0 + u < splits ? *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(part) + (z0 + u) * mn + o)
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) { acc.x += a[u].x; acc.y += a[u].y; acc.z += a[u].z; acc.w += a[u].w; }   // slice order
-    }
-    v[0] = (acc.x * p.scale_a) * p.scale_b; v[1] = (acc.y * p.scale_a) * p.scale_b;
-    v[2] = (acc.z * p.scale_a) * p.scale_b; v[3] = (acc.w * p.scale_a) * p.scale_b;
+    for (int u = 0; u < 4; ++u) acc += a[u];           // slice order
   }
-  if constexpr (EPI == EPI8_SCALED_BF16) {
-    uint2 pk;
-    pk.x = pack2<BF16>(v[0], v[1]);
-    pk.y = pack2<BF16>(v[2], v[3]);
-    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.D) + o) = pk;
-  } else if constexpr (EPI != EPI8_I32) {
-    *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.D) + o) = make_float4(v[0], v[1], v[2], v[3]);
-  }
+  gemm8_store_quad<T, EPI>(p, m, n, acc, vec);
+}
+template <class T, int EPI>
+int launch_gemm8_split_sum(const void* part, int splits, long ldw, int vec, const Gemm8Params& p, hipStream_t s) {
+  const long quads = (long)p.M * ((p.N + 3) / 4);
+  hipLaunchKernelGGL((gemm8_split_sum_kernel<T, EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, part, splits, ldw, vec,
+                     p);
+  return launch_status();
 }
 
 // Any-shape fallback, one thread per output element, k in order.

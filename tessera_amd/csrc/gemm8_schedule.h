@@ -10,7 +10,7 @@ struct Gemm8Schedule {
   int tile_m;    // rows of the workgroup tile: 256 or 128 (tile kernel), 32 or 64 (few-row streaming kernel)
   int tile_n;    // columns: 256 (tile kernel) or 128 (streaming kernel's strip)
   int tile_k;    // bytes of K per step: 128 (tile kernel) or 64 (a streaming slice)
-  int split_k;   // K slices summed by the split-sum kernel (1 = none; the streaming kernel always goes through it)
+  int split_k;   // K slices summed by the split-sum kernel (1 = none)
   bool skinny;   // the few-row streaming kernel
 };
 
@@ -35,7 +35,7 @@ inline double est_tiles8_us(int bm, long tiles, int ksteps) {
 // compute unit's K steps (its first workgroup at `step`, every further one sharing the unit at
 // `shared` per step) and the time to stream the tile columns of B at `tbs` TB/s, which takes about
 // 155 workgroups in flight to reach (256 for the streaming kernel) and is stretched by a last, partly filled round; the sum over
-// K parts (always there behind the streaming kernel) adds 2 us and 1.4 us per million partials.
+// K parts adds 2 us and 1.4 us per million partials.
 struct Gemm8Fit { double launch, step, shared, tbs; };
 constexpr Gemm8Fit kGemm8Fit[3] = {{5.23, 0.731, 1.265, 5.44},     // the streaming kernel (a step = one 64-row slice of a wave)
                                    {6.51, 0.780, 1.121, 6.52},     // 128 x 256 tiles (a step = 128 of K)
@@ -56,22 +56,35 @@ inline double est_gemm8_fit_us(int kind, int M, int N, int K, int splits) {
   // out 5 % faster with it)
   const double sat = kind == 0 ? 256.0 : 155.0;
   const double stream = bytes / (f.tbs * 1e6 * std::min(1.0, wgs / sat)) * (wgs > 256 ? busiest * 256.0 / wgs : 1.0);
-  const double sum = (splits > 1 || kind == 0) ? 2.06 + (double)M * N * splits * 1.43e-6 : 0.0;
+  const double sum = splits > 1 ? 2.06 + (double)M * N * splits * 1.43e-6 : 0.0;
   return f.launch + std::max(compute, stream) + sum;
+}
+
+// K splits of the streaming kernel: never over one workgroup per compute unit (the second round would be
+// nearly empty), at least one 64-row slice for each of its waves (8 waves up to 32 rows, 4 above: twice the
+// accumulators), and within that the fewest microseconds by an estimate: a workgroup streams a 128-byte row
+// in 3.75 ns, the chip 5.6 TB/s; a split adds a launch and a sum, 3.6 us.
+inline int gemm8_skinny_splits(int M, int N, int K) {
+  const int strips = (N + 127) / 128;
+  const int most = std::max(1, std::min(256 / strips, K / ((M <= 32 ? 8 : 4) * 64)));
+  int best = 1;
+  double best_us = 1e30;
+  for (int splits = 1; splits <= most; ++splits) {
+    const int wgs = strips * splits;
+    const double rounds = wgs > 256 ? (wgs + 255) / 256 * 256.0 / wgs : 1.0;
+    const double us = std::max(3.75e-3 * K / splits, (double)K * N / 5.6e6) * rounds + (splits > 1 ? 3.6 : 0.0);
+    if (us <= best_us) { best_us = us; best = splits; }
+  }
+  return best;
 }
 
 // The rule: the streaming kernel for few rows, else tile rows and a power-of-two K split by est_tiles8_us.
 inline Gemm8Schedule select_gemm8_rule(int M, int N, int K) {
   auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
-  // At most 64 rows against a long K (quantised decode): the streaming kernel, one workgroup per
-  // 128-column strip and K range, about one workgroup per compute unit and at least two 64-row
-  // slices for each of its waves (8 waves up to 32 rows, 4 above: twice the accumulators).
-  if (M <= kGemm8SkinnyMaxM && K % 64 == 0 && K >= 2048) {
-    const int nw = M <= 32 ? 8 : 4;
-    const int strips = (int)cdiv(N, 128);
-    // (never a little over one workgroup per compute unit: the second round would be nearly empty)
-    int splits = std::max(1, std::min(256 / strips, K / (2 * nw * 64)));
-    const int kps = (int)cdiv(cdiv(K, splits), 64) * 64;
+  // At most 64 rows (quantised decode): the streaming kernel.  (Below 1024 rows of B the tiles are as good:
+  // 48 x 4096 x 512 10.2 us against 12.3.)
+  if (M <= kGemm8SkinnyMaxM && K % 16 == 0 && K >= 1024) {
+    const int kps = (int)cdiv(cdiv(K, gemm8_skinny_splits(M, N, K)), 64) * 64;
     return {M <= 32 ? 32 : 64, 128, 64, (int)cdiv(K, kps), true};
   }
   // Tile rows (256 or 128) and K slices by estimated time.  Few tiles and a long K (few rows against a

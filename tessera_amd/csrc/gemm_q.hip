@@ -95,6 +95,58 @@ int gemm8_repitched(const Gemm8Params& p, hipStream_t s) {
   return rc;
 }
 
+// The few-row streaming kernel with K in `splits` parts (more than one: then the sum).  loose: rows of B on any boundary; A is
+// then copied into rows padded with zeros to a multiple of 16 where its own cannot be read 16 bytes at a time.
+// (8 waves and about 256 workgroups measured best for up to 32 rows: 4-wave workgroups, two per
+// compute unit, and 384 or 512 workgroups were level or slower on M = 1 ... 32 against 4096 ...
+// 28672 columns.  33 to 64 rows double the accumulators: 4 waves, one per SIMD.)
+template <class T, int EPI>
+int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
+  const bool one = p.M <= 32;
+  const int nw = one ? 8 : 4;
+  using Kernel = void (*)(const Gemm8Params, int, int, void*, int);
+  static const Kernel kernels[2][2] = {{gemm8_skinny_kernel<T, 4, 2, EPI, false>, gemm8_skinny_kernel<T, 4, 2, EPI, true>},
+                                       {gemm8_skinny_kernel<T, 8, 1, EPI, false>, gemm8_skinny_kernel<T, 8, 1, EPI, true>}};
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  std::call_once(once, [&] {
+    for (int o = 0; o < 2; ++o)
+      for (Kernel k : kernels[o])
+        if (attr_err == hipSuccess)
+          attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         g8s_smem(o ? 8 : 4, 32));
+  });
+  if (attr_err != hipSuccess) return kDeviceFailed;
+  const int strips = ceil_div(p.N, G8S_COLS);
+  const int kps = ceil_div(ceil_div(p.K, splits), G8S_ROWS) * G8S_ROWS;
+  splits = ceil_div(p.K, kps);
+  const long ldw = (long)strips * G8S_COLS;
+  const int K16 = (p.K + 15) & ~15;
+  const bool a_copy = loose && (p.K % 16 != 0 || !aligned16(p.A));
+  const size_t a_bytes = a_copy ? (((size_t)p.M * K16 + 255) & ~size_t(255)) : 0;
+  const size_t part_bytes = splits > 1 ? (size_t)splits * p.M * ldw * 4 : 0;
+  char* ws = nullptr;
+  if (a_bytes + part_bytes) {
+    ws = static_cast<char*>(stream_workspace(s, a_bytes + part_bytes));
+    if (!ws) return kDeviceFailed;
+  }
+  Gemm8Params q = p;
+  int lda = p.K;
+  if (a_copy) {
+    hipLaunchKernelGGL(pad_rows_kernel<uint8_t>, copy_grid(p.M, K16, 16, 1), copy_block(), 0, s, reinterpret_cast<uint8_t*>(ws),
+                       (long)K16, 0L, p.A, (long)p.K, 0L, p.M, p.K, p.M);
+    if (int rc = launch_status(); rc != kOk) return rc;
+    q.A = reinterpret_cast<const uint8_t*>(ws);
+    lda = K16;
+  }
+  void* part = splits > 1 ? ws + a_bytes : nullptr;
+  const int vec = p.N % 4 == 0 && aligned16(p.D) && (!p.acc_out || aligned16(p.acc_out)) && (!p.col_scale || aligned16(p.col_scale));
+  hipLaunchKernelGGL(kernels[one][loose], dim3(strips, splits), dim3(nw * 64), g8s_smem(nw, std::min(p.M, 32)), s, q, lda, kps, part,
+                     vec);
+  if (int rc = launch_status(); rc != kOk || !part) return rc;
+  return launch_gemm8_split_sum<T, EPI>(part, splits, ldw, vec, p, s);
+}
+
 template <class T, int EPI>
 int gemm8_dev(Gemm8Params p, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0 || p.K <= 0 || !p.A || !p.B || !p.D) return kBadShape;
@@ -104,6 +156,9 @@ int gemm8_dev(Gemm8Params p, hipStream_t s) {
   const bool vec = (p.K % 16 == 0) && (p.N % 16 == 0) && (p.K < (1 << 22)) && (p.N < (1 << 22)) && aligned16(p.A) && aligned16(p.B) && aligned16(p.D) &&
                    (!p.acc_out || aligned16(p.acc_out)) && (!p.col_scale || aligned16(p.col_scale));
   if (!vec) {
+    // few rows: the streaming kernel reads B where it lies
+    if (p.M <= kGemm8SkinnyMaxM && p.N >= 16 && p.N < (1 << 25) && p.K < (1 << 24))
+      return gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(p.M, p.N, p.K), true, s);
     // small products go one thread per output element; above about 2^24 multiply-adds the copies
     // into aligned, zero-padded buffers cost less than that kernel loses
     if ((double)p.M * p.N * p.K >= (double)(1L << 24) && p.M >= 16 && p.N >= 16 && p.K + 16 < (1 << 22) && p.N + 16 < (1 << 22))
@@ -113,39 +168,7 @@ int gemm8_dev(Gemm8Params p, hipStream_t s) {
     return launch_status();
   }
   const Gemm8Schedule sch = select_gemm8_schedule(p.M, p.N, p.K);
-  if (sch.skinny) {
-    // (8 waves and about 256 workgroups measured best for up to 32 rows: 4-wave workgroups, two per
-    // compute unit, and 384 or 512 workgroups were level or slower on M = 1 ... 32 against 4096 ...
-    // 28672 columns.  33 to 64 rows double the accumulators: 4 waves, one per SIMD.)
-    const int nw = p.M <= 32 ? 8 : 4;
-    const int smem = p.M <= 32 ? g8s_smem(8, 1) : g8s_smem(4, 2);
-    const void* kern = p.M <= 32 ? reinterpret_cast<const void*>(gemm8_skinny_kernel<T, 8, 1>)
-                                 : reinterpret_cast<const void*>(gemm8_skinny_kernel<T, 4, 2>);
-    static std::once_flag once;
-    static hipError_t attr_err = hipSuccess;
-    std::call_once(once, [&] {
-      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm8_skinny_kernel<T, 8, 1>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, g8s_smem(8, 1));
-      if (attr_err == hipSuccess)
-        attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm8_skinny_kernel<T, 4, 2>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, g8s_smem(4, 2));
-    });
-    if (attr_err != hipSuccess) return kDeviceFailed;
-    const int strips = ceil_div(p.N, G8S_COLS);
-    const int splits = sch.split_k;
-    const int kps = ceil_div(ceil_div(p.K, splits), G8S_ROWS) * G8S_ROWS;
-    void* ws = stream_workspace(s, (size_t)splits * p.M * p.N * 4);
-    if (!ws) return kDeviceFailed;
-    void* args[] = {(void*)&p.A, (void*)&p.B, (void*)&ws, (void*)&p.M, (void*)&p.N, (void*)&p.K, (void*)&kps};
-    if (hipLaunchKernel(kern, dim3(strips, splits), dim3(nw * 64), args, smem, s) != hipSuccess) {
-      (void)hipGetLastError();
-      return kDeviceFailed;
-    }
-    const long quads = (long)p.M * (p.N / 4);
-    hipLaunchKernelGGL((gemm8_split_sum_kernel<T, EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, ws,
-                       splits, p);
-    return launch_status();
-  }
+  if (sch.skinny) return gemm8_skinny<T, EPI>(p, sch.split_k, false, s);
   const int bm = sch.tile_m, splits = sch.split_k;
   p.tiles_m = ceil_div(p.M, bm);
   p.tiles_n = ceil_div(p.N, G8_BN);
@@ -166,10 +189,7 @@ int gemm8_dev(Gemm8Params p, hipStream_t s) {
       q.ksplit = ceil_div(ceil_div(p.K, G8_BK), splits) * G8_BK;
       hipLaunchKernelGGL((gemm8_kernel<T, RAW_EPI, BM>), dim3(tiles, splits), dim3(256), g8_smem(BM), s, q);
       if (int rc = launch_status(); rc != kOk) return rc;
-      const long quads = (long)p.M * (p.N / 4);
-      hipLaunchKernelGGL((gemm8_split_sum_kernel<T, EPI>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, ws,
-                         splits, p);
-      return launch_status();
+      return launch_gemm8_split_sum<T, EPI>(ws, splits, p.N, 1, p, s);
     }
     if (int rc = gemm8_attr<T, EPI, BM>(); rc != kOk) return rc;
     hipLaunchKernelGGL((gemm8_kernel<T, EPI, BM>), dim3(tiles), dim3(256), g8_smem(BM), s, p);
