@@ -141,9 +141,15 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {
 // does not serialise later LDS reads of OTHER stages behind it; the kernel waits
 // for these loads itself (fa_wait_loads) before the barrier that publishes the
 // stage.
+// (NT: the non-temporal hint, for data read once; see buffer_load_b128.)
+template <bool NT = false>
 __device__ __forceinline__ void load16_to_lds(const void* base, uint32_t byte_off, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds_base), "v"(byte_off), "s"(base) : "memory");
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 :: "s"(lds_base), "v"(byte_off), "s"(base) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(lds_base), "v"(byte_off), "s"(base) : "memory");
 }
 __device__ __forceinline__ void fa_wait_loads() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -42,7 +42,9 @@ struct FlashDecodeParams {
   int tiles_per_split;
 };
 
-template <class T, int DP, int NQ>
+// PAD: the head dimension p.D < DP (a multiple of 16): the missing columns of Q are zero registers, those of K and
+// V zeros that are written to LDS once and never loaded over.  NT: K and V with the non-temporal hint.
+template <class T, int DP, int NQ, bool PAD, bool NT>
 __global__ __launch_bounds__(DecodeGeom<DP>::THREADS) void flash_decode_kernel(const FlashDecodeParams dp) {
   using G = DecodeGeom<DP>;
   const FlashParams& p = dp.f;
@@ -77,7 +79,7 @@ __global__ __launch_bounds__(DecodeGeom<DP>::THREADS) void flash_decode_kernel(c
     const uint16_t* src = p.Q + batch * p.qs.batch + (hkv * p.ratio + hsel) * p.qs.head + (long)qi * p.qs.row + 8 * lh;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
-      qf[qt][ks] = valid ? *reinterpret_cast<const uint4*>(src + 16 * ks) : make_uint4(0u, 0u, 0u, 0u);
+      qf[qt][ks] = valid && (!PAD || 16 * ks < p.D) ? *reinterpret_cast<const uint4*>(src + 16 * ks) : make_uint4(0u, 0u, 0u, 0u);
     klo[qt] = 0;
     khi[qt] = -1;
     if (valid) key_bounds(qi, p.Sq, p.Sk, p.causal, p.window, klo[qt], khi[qt]);
@@ -90,6 +92,7 @@ __global__ __launch_bounds__(DecodeGeom<DP>::THREADS) void flash_decode_kernel(c
   // chunk P % CHUNKS) and holds the row's logical chunk (physical ^ swizzle(row)).
   int ld_row[LD];
   uint32_t ld_koff[LD], ld_voff[LD];
+  bool ld_kok[LD], ld_vok[LD];                         // the slot's column exists
   const uint32_t krow_bytes = (uint32_t)p.ks.row * 2, vrow_bytes = (uint32_t)p.vs.row * 2;
 #pragma unroll
   for (int q = 0; q < LD; ++q) {
@@ -98,6 +101,16 @@ __global__ __launch_bounds__(DecodeGeom<DP>::THREADS) void flash_decode_kernel(c
     ld_row[q] = row;
     ld_koff[q] = row * krow_bytes + ((chp ^ kswz(row)) << 4);
     ld_voff[q] = row * vrow_bytes + ((chp ^ vswz(row)) << 4);
+    ld_kok[q] = !PAD || (chp ^ kswz(row)) * 8 < p.D;
+    ld_vok[q] = !PAD || (chp ^ vswz(row)) * 8 < p.D;
+    if constexpr (PAD) {
+      const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        if (!ld_kok[q]) lds_write_b128(wsm, st * TILE + P * 16, zero);
+        if (!ld_vok[q]) lds_write_b128(wsm, (2 + st) * TILE + P * 16, zero);
+      }
+    }
   }
   auto load_tile = [&](int tile, int stage) {
     const uint16_t* kt = Kb + (long)tile * G::BK * p.ks.row;
@@ -110,8 +123,11 @@ __global__ __launch_bounds__(DecodeGeom<DP>::THREADS) void flash_decode_kernel(c
         ko -= (uint32_t)(ld_row[q] - last) * krow_bytes;
         vo -= (uint32_t)(ld_row[q] - last) * vrow_bytes;
       }
-      load16_to_lds(kt, ko, wlds + stage * TILE + q * 1024);
-      load16_to_lds(vt, vo, wlds + (2 + stage) * TILE + q * 1024);
+      // (every instruction covers whole rows, so some lane always loads: the counts waited for hold)
+      const uint32_t k_lds = __builtin_amdgcn_readfirstlane(wlds + stage * TILE + q * 1024);
+      const uint32_t v_lds = k_lds + 2 * TILE;
+      if (!PAD || ld_kok[q]) load16_to_lds<NT>(kt, ko, k_lds);
+      if (!PAD || ld_vok[q]) load16_to_lds<NT>(vt, vo, v_lds);
     }
   };
 
@@ -266,6 +282,7 @@ __global__ __launch_bounds__(DecodeGeom<DP>::THREADS) void flash_decode_kernel(c
     const int rows_here = min(32, dp.rows - 32 * qt);
     for (int idx = tid; idx < rows_here * (D / 4); idx += G::THREADS) {
       const int il = idx / (D / 4), d = (idx - il * (D / 4)) * 4;
+      if (PAD && d >= p.D) continue;
       float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int w = 0; w < G::WAVES; ++w) {
@@ -292,7 +309,7 @@ __global__ __launch_bounds__(DecodeGeom<DP>::THREADS) void flash_decode_kernel(c
         }
         if (p.LSE && d == 0) p.LSE[rowlin] = lse;
       } else {
-        *reinterpret_cast<float4*>(dp.part_o + ((long)split * total_rows + rowlin) * D + d) = acc;
+        *reinterpret_cast<float4*>(dp.part_o + ((long)split * total_rows + rowlin) * p.D + d) = acc;
         if (d == 0) dp.part_lse[(long)split * total_rows + rowlin] = lse;
       }
     }

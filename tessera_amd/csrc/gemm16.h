@@ -189,7 +189,8 @@ __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n,
 // One BM x BN output tile: rows [m_begin, min(m_begin + BM, m_end)), column tile tn, of
 // the product whose operand and output bases are Ab / Bb / B2b / Db.  All threads of the
 // workgroup call it with the same arguments.
-template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32>
+// NTB: B with the non-temporal hint (see buffer_load_b128).
+template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32, bool NTB = false>
 __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, const int m_begin, const int m_end,
                                             const int tn, const uint16_t* Ab, const uint16_t* Bb,
                                             const uint16_t* B2b, char* Db, const bool paced = false) {
@@ -306,7 +307,7 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, c
       const int qb = q - A_CHUNKS;
       uint32_t off = b_off0;
       if constexpr (GUARD) off = (k0 + b_krow(qb) < K) ? off : kOutOfRange;
-      return buffer_load_b128(b_base[qb / B_PER] + (long)(k0 + (qb % B_PER) * B_KSTRIDE) * p.ldb, off);
+      return buffer_load_b128<NTB>(b_base[qb / B_PER] + (long)(k0 + (qb % B_PER) * B_KSTRIDE) * p.ldb, off);
     }
   };
   auto gload1 = [&](int q, int k0, auto guarded_c) { st[q] = gfetch(q, k0, guarded_c); };
@@ -678,7 +679,7 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, c
 // MID (grouped 256-row tiles only): a last row tile of 65 to 128 rows runs on the 128-row tile
 // body.  A separate instantiation, for launches whose groups average at most a tile of rows: the
 // kernel that serves large groups keeps its two bodies.
-template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32, bool MID = false>
+template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32, bool MID = false, bool NTB = false>
 __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Params p) {
   constexpr bool SWIGLU = (EPI == EPI_SWIGLU16 || EPI == EPI_GATED_F32);
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -775,17 +776,17 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Par
     // full tile, whose other 192 rows would be computed and thrown away.
     if (m_end - m_begin <= 64) {
       // (paced when full tiles of the same group and column run beside it; 16-wide step only)
-      gemm16_tile<T, 64, BN, 1, 4, EPI, GROUPED, MS>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db, MS == 16 && tm > 0);
+      gemm16_tile<T, 64, BN, 1, 4, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db, MS == 16 && tm > 0);
       return;
     }
     // (up to 128 rows left — a group of about a hundred rows, a chunk of a thousand tokens over
     // 64 experts — the 128-row tile: half the matrix work)
     if (MID && m_end - m_begin <= 128) {
-      gemm16_tile<T, 128, BN, 2, 2, EPI, GROUPED, MS>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
+      gemm16_tile<T, 128, BN, 2, 2, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
       return;
     }
   }
-  gemm16_tile<T, BM, BN, WM, WN, EPI, GROUPED, MS>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
+  gemm16_tile<T, BM, BN, WM, WN, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
 }
 
 // The tiles that are left when the tile count is not a multiple of the 256 compute units would

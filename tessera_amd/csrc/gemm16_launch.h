@@ -71,10 +71,10 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // wg_limit > 0: only the first wg_limit workgroups of a dense product's tile order are launched
 // (the caller serves the remaining tiles itself).
-template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32, bool MID = false>
+template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32, bool MID = false, bool NTB = false>
 int launch_gemm16_tile(Gemm16Params p, hipStream_t s, int wg_limit = 0) {
   using S = Gemm16Smem<BM, BN>;
-  auto kern = gemm16_kernel<T, BM, BN, WM, WN, EPI, GROUPED, MS, MID>;
+  auto kern = gemm16_kernel<T, BM, BN, WM, WN, EPI, GROUPED, MS, MID, NTB>;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
@@ -638,11 +638,21 @@ int launch_gemm16_grouped(Gemm16Params p, hipStream_t s) {
   // groups that average at most a tile of rows (a chunk of a thousand tokens over 64 experts): the
   // instantiation whose last row tile also comes in a 128-row form
   const bool mid = (long)p.M <= 256L * p.groups;
+  // Weights that outgrow the memory-side cache are streamed past it: each panel is read by one row tile, or by
+  // a few running side by side on one XCD, whose L2 still serves them (64 experts of 4096 x 1408, the
+  // whole layer: 8 tokens 285 -> 256 us, 64 408 -> 378, 512 447 -> 423, 1024 539 -> 524, 1900 660 -> 654).
+  const bool nt = (long)p.M <= 256L * p.groups &&
+                  (EPI == EPI_SWIGLU16 ? 4.0 : 2.0) * p.K * p.N * p.groups >= kStreamOnceBytes;
   if constexpr (EPI == EPI_SWIGLU16) {
+    if (mid && nt) return launch_gemm16_tile<T, 256, 256, 2, 2, EPI, true, kGroupedTileMfma, true, true>(p, s);
     if (mid) return launch_gemm16_tile<T, 256, 256, 2, 2, EPI, true, kGroupedTileMfma, true>(p, s);
     return launch_gemm16_tile<T, 256, 256, 2, 2, EPI, true, kGroupedTileMfma>(p, s);
   } else {
-    if ((long)p.M < 64L * p.groups) return launch_gemm16_tile<T, 128, 128, 2, 2, EPI, true>(p, s);
+    if ((long)p.M < 64L * p.groups) {
+      if (nt) return launch_gemm16_tile<T, 128, 128, 2, 2, EPI, true, 32, false, true>(p, s);
+      return launch_gemm16_tile<T, 128, 128, 2, 2, EPI, true>(p, s);
+    }
+    if (mid && nt) return launch_gemm16_tile<T, 256, 256, 2, 2, EPI, true, kGroupedTileMfma, true, true>(p, s);
     if (mid) return launch_gemm16_tile<T, 256, 256, 2, 2, EPI, true, kGroupedTileMfma, true>(p, s);
     return launch_gemm16_tile<T, 256, 256, 2, 2, EPI, true, kGroupedTileMfma>(p, s);
   }
