@@ -67,6 +67,9 @@ _SIGNATURES = {
     "tessera_gfx950_device_cus": [_P(_c_int)],
     "tessera_gfx950_malloc": [_P(_c_vp), _c_sz],
     "tessera_gfx950_free": [_c_vp],
+    "tessera_gfx950_pool_malloc": [_P(_c_vp), _c_sz],
+    "tessera_gfx950_pool_free": [_c_vp, _c_int],
+    "tessera_gfx950_pool_trim": [],
     "tessera_gfx950_memcpy_h2d": [_c_vp, _c_vp, _c_sz],
     "tessera_gfx950_memcpy_d2h": [_c_vp, _c_vp, _c_sz],
     "tessera_gfx950_memset": [_c_vp, _c_int, _c_sz],
@@ -279,6 +282,10 @@ class DeviceBuffer:
         check(load().tessera_gfx950_malloc(ctypes.byref(p), self.nbytes), "malloc")
         self.ptr = p.value
 
+    @property
+    def address(self) -> Optional[int]:
+        return self.ptr
+
     @classmethod
     def from_host(cls, a: np.ndarray) -> "DeviceBuffer":
         a = np.ascontiguousarray(a)
@@ -308,6 +315,57 @@ class DeviceBuffer:
                 load().tessera_gfx950_free(self.ptr)
             finally:
                 self.ptr = None
+
+    def __del__(self):  # pragma: no cover - best effort
+        try:
+            self.close()
+        except Exception:
+            pass
+
+
+class PooledBuffer:
+    """A device allocation from the library's pool, for results of calls on the default stream.
+
+    ``address`` is for such calls.  Reading ``ptr`` marks the buffer as shared: its memory may then be in use in
+    other streams, and is not handed out again before the device has been synchronised."""
+
+    __slots__ = ("nbytes", "address", "_shared", "_free", "__weakref__")
+
+    def __init__(self, nbytes: int):
+        self.address = None
+        self.nbytes = int(nbytes)
+        self._shared = 0
+        lib = load()
+        self._free = lib.tessera_gfx950_pool_free
+        p = _c_vp()
+        check(lib.tessera_gfx950_pool_malloc(ctypes.byref(p), self.nbytes), "malloc")
+        self.address = p.value
+
+    @property
+    def ptr(self) -> Optional[int]:
+        self._shared = 1
+        return self.address
+
+    def upload(self, a: np.ndarray) -> None:
+        a = np.ascontiguousarray(a)
+        if a.nbytes > self.nbytes:
+            raise ValueError("upload larger than the device buffer")
+        check(load().tessera_gfx950_memcpy_h2d(self.address, a.ctypes.data, a.nbytes), "memcpy_h2d")
+
+    def download(self, shape, dtype) -> np.ndarray:
+        out = np.empty(shape, dtype)
+        if out.nbytes > self.nbytes:
+            raise ValueError("download larger than the device buffer")
+        check(load().tessera_gfx950_memcpy_d2h(out.ctypes.data, self.address, out.nbytes), "memcpy_d2h")
+        return out
+
+    def zero(self) -> None:
+        check(load().tessera_gfx950_memset(self.address, 0, self.nbytes), "memset")
+
+    def close(self) -> None:
+        p, self.address = self.address, None
+        if p:
+            self._free(p, self._shared)
 
     def __del__(self):  # pragma: no cover - best effort
         try:
