@@ -95,8 +95,11 @@ constexpr int FA_BKV = 64;             // keys per LDS tile
 // Per padded head dimension: waves per workgroup (always two per SIMD), how many waves share
 // one 32-row block by output columns, query rows per workgroup, 16-byte chunks per LDS row,
 // bytes of one K (or V) stage, LDS bytes.
-template <int DP> struct FlashGeom {
-  static constexpr int WAVES = 8;
+// W = 4: the same body as workgroups of 128 query rows, two of them on a compute unit (67 KB of LDS
+// each at DP = 128), for launches whose 256-row workgroups would leave compute units idle or half
+// of their only row block empty; the launcher has the rule and both sides' times.
+template <int DP, int W = 8> struct FlashGeom {
+  static constexpr int WAVES = W;
   static constexpr int THREADS = WAVES * 64;
   // DP = 256: a wave's 32 rows x 256 output columns would be 128 accumulator registers, which
   // does not fit next to 64 Q and 64 score registers in the 256 a wave has at two per SIMD.
@@ -166,9 +169,9 @@ __device__ __forceinline__ float scale_acc(float acc, float corr) {
   return acc;
 }
 
-template <class T, int DP, bool EXT, bool PAD>
-__global__ __launch_bounds__(FlashGeom<DP>::THREADS, 1) void flash_fwd_kernel(const FlashParams p) {
-  using G = FlashGeom<DP>;
+template <class T, int DP, bool EXT, bool PAD, int W>
+__global__ __launch_bounds__((FlashGeom<DP, W>::THREADS), 2) void flash_fwd_kernel(const FlashParams p) {
+  using G = FlashGeom<DP, W>;
   constexpr int D = DP;                  // extent the loops are unrolled for
   constexpr int FA_WAVES = G::WAVES, FA_THREADS = G::THREADS, FA_BQ = G::BQ;
   constexpr int FA_KT = FA_BKV / 32;     // 32-key MFMA tiles per LDS tile
@@ -209,13 +212,19 @@ __global__ __launch_bounds__(FlashGeom<DP>::THREADS, 1) void flash_fwd_kernel(co
   // the grid is (B * Hq, query blocks, 1), heaviest blocks first.  No index needs a
   // division either way.
   // qlin / kvlin: linear (batch, head) index of the query head / of its KV head.
+  // Workgroups of 4 waves serve short sequences, whose K and V stay in the L2 in any order, two to a compute
+  // unit: their query blocks come last in the grid, so that the heavy blocks of all heads are dealt out first
+  // and share a unit with light ones (with the order above B 2 x S 1024 put two heavy ones on one unit).
   const int nsplit = p.nsplit > 1 ? p.nsplit : 1;
-  const int split = p.nsplit > 1 ? (int)blockIdx.y % nsplit : 0;
-  const int qb = (int)gridDim.y / nsplit - 1 - (int)blockIdx.y / nsplit;
+  const bool grouped = gridDim.z > 1 || (int)gridDim.x == 8 * p.ratio;
+  const bool blocks_last = W == 4 && grouped;
+  const int yblocks = blocks_last ? gridDim.z : gridDim.y, yblock = blocks_last ? blockIdx.z : blockIdx.y;
+  const int split = p.nsplit > 1 ? yblock % nsplit : 0;
+  const int qb = yblocks / nsplit - 1 - yblock / nsplit;
   int qlin, kvlin;
-  if (gridDim.z > 1 || (int)gridDim.x == 8 * p.ratio) {
+  if (grouped) {
     const int w = blockIdx.x;
-    kvlin = blockIdx.z * 8 + (w & 7);
+    kvlin = (blocks_last ? blockIdx.y : blockIdx.z) * 8 + (w & 7);
     qlin = kvlin * p.ratio + (w >> 3);
   } else {
     qlin = blockIdx.x;
