@@ -308,8 +308,49 @@ int flash_host(const void* Q, const void* K, const void* V, void* O, void* LSE, 
   return kOk;
 }
 
+// How many workgroups share each walk of the backward's two kernels.
+struct BwdSplits { int dq = 1, dkv = 1; };
+
+// The split with the least estimated time of one kernel: a walk of `longest` steps is shared by n
+// workgroups (one per compute unit: registers and LDS), the kernel takes the longer of one share and
+// the whole work over 256 compute units, and the n partial results are written and read once more
+// at about 4 TB/s, behind one more launch.  Taken only if it saves a tenth.
+inline int best_bwd_split(double longest, double total, double step_us, double part_bytes) {
+  const double chip = total / 256.0;
+  auto at = [&](int n) {
+    return step_us * std::max(std::ceil(longest / n), chip) + (n > 1 ? 4.0 + n * part_bytes * 2.0 / 4.0e6 : 0.0);
+  };
+  int best = 1;
+  for (int n = 2; n <= 64 && n <= longest; ++n)
+    if (at(n) < 0.9 * at(1) && at(n) < at(best)) best = n;
+  return best;
+}
+
+// Both walks in steps: 64 keys of a 256-row query block (dQ), 64 query rows of one head against 128 keys (dK, dV).
+inline BwdSplits plan_bwd_splits(int B, int Hq, int Hkv, int Sq, int Sk, int D, int causal) {
+  const int off = Sk > Sq ? Sk - Sq : 0;
+  double dq_long = 0, dq_total = 0, dkv_long = 0, dkv_total = 0;
+  for (int q0 = 0; q0 < Sq; q0 += FB_BQ) {
+    const int end = causal ? std::min(Sk, std::min(q0 + FB_BQ, Sq) + off) : Sk;
+    const double n = ceil_div(end, FB_BKV);
+    dq_long = std::max(dq_long, n);
+    dq_total += n;
+  }
+  for (int k0 = 0; k0 < Sk; k0 += FB_BK) {
+    const int first = causal ? std::max(0, k0 - off) / FB_BQT : 0;
+    const double n = (double)std::max(ceil_div(Sq, FB_BQT) - first, 0) * (Hq / Hkv);
+    dkv_long = std::max(dkv_long, n);
+    dkv_total += n;
+  }
+  BwdSplits r;
+  const double width = D / 128.0;
+  r.dq = best_bwd_split(dq_long, dq_total * B * Hq, 2.6 * width + 0.2, 4.0 * B * Hq * Sq * D);
+  r.dkv = best_bwd_split(dkv_long, dkv_total * B * Hkv, 1.5 * width + 0.3, 8.0 * B * Hkv * Sk * D);
+  return r;
+}
+
 template <class T, int D>
-int launch_bwd(const FlashBwdParams& p, hipStream_t s) {
+int launch_bwd(const FlashBwdParams& p, const BwdSplits& sp, hipStream_t s) {
   constexpr int kDqSmem = 4 * FB_BKV * D * 2;
   constexpr int kDkvSmem = flash_bwd_dkdv_lds_bytes<D>();
   auto dq_kern = flash_bwd_dq_kernel<T, D>;
@@ -324,9 +365,17 @@ int launch_bwd(const FlashBwdParams& p, hipStream_t s) {
                                      hipFuncAttributeMaxDynamicSharedMemorySize, kDkvSmem);
   });
   if (attr_err != hipSuccess) return kDeviceFailed;
-  hipLaunchKernelGGL(dq_kern, dim3(ceil_div(p.Sq, FB_BQ) * p.B * p.Hq), dim3(FB_DQ_THREADS), kDqSmem, s, p);
+  hipLaunchKernelGGL(dq_kern, dim3(ceil_div(p.Sq, FB_BQ) * p.B * p.Hq, sp.dq), dim3(FB_DQ_THREADS), kDqSmem, s, p);
   if (int rc = launch_status(); rc != kOk) return rc;
-  hipLaunchKernelGGL(dkv_kern, dim3(ceil_div(p.Sk, FB_BK) * p.B * p.Hkv), dim3(FB_DKV_THREADS), kDkvSmem, s, p);
+  hipLaunchKernelGGL(dkv_kern, dim3(ceil_div(p.Sk, FB_BK) * p.B * p.Hkv, sp.dkv), dim3(FB_DKV_THREADS), kDkvSmem, s,
+                     p);
+  if (sp.dq > 1 || sp.dkv > 1) {
+    if (int rc = launch_status(); rc != kOk) return rc;
+    const long qn4 = (long)p.B * p.Hq * p.Sq * D / 4, kvn4 = (long)p.B * p.Hkv * p.Sk * D / 4;
+    const long blocks = (std::max(sp.dq > 1 ? qn4 : 0, sp.dkv > 1 ? kvn4 : 0) + 255) / 256;
+    hipLaunchKernelGGL(flash_bwd_sum_kernel, dim3((unsigned)std::min<long>(blocks, 4096), 3), dim3(256), 0, s, p, sp.dq,
+                       sp.dkv, qn4, kvn4);
+  }
   return launch_status();
 }
 
@@ -557,7 +606,17 @@ int flash_bwd_dev(const void* dO, const void* Q, const void* K, const void* V, c
     if (al_in && scale_ok && D < 128 && D != 64)
       return flash_bwd_padded_dev<T>(dO, Q, K, V, O, LSE, dQ, dK, dV, B, Hq, Hkv, Sq, Sk, D, scale, causal, s);
   }
-  const size_t ws_floats = 2 * rows + (recompute ? rows * D + rows : 0);
+  const bool mfma = scale_ok && (D == 128 || D == 64) &&
+                    ((reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) | reinterpret_cast<uintptr_t>(V) |
+                      reinterpret_cast<uintptr_t>(dO) | reinterpret_cast<uintptr_t>(dQ) | reinterpret_cast<uintptr_t>(dK) |
+                      reinterpret_cast<uintptr_t>(dV)) & 15) == 0;
+  BwdSplits splits;
+  if (mfma) splits = plan_bwd_splits(B, Hq, Hkv, Sq, Sk, D, causal);
+  const size_t kvrows_all = (size_t)B * Hkv * Sk;
+  // Delta | LSE2 [| O | LSE], each a whole number of 16 bytes, then the partial gradients
+  const size_t head_floats = (2 * rows + (recompute ? rows * D + rows : 0) + 3) / 4 * 4;
+  const size_t dq_part = splits.dq > 1 ? splits.dq * rows * D : 0;
+  const size_t ws_floats = head_floats + dq_part + (splits.dkv > 1 ? splits.dkv * 2 * kvrows_all * D : 0);
   if (hipMallocAsync(reinterpret_cast<void**>(&ws), ws_floats * sizeof(float), s) != hipSuccess) {
     (void)hipGetLastError();
     return kDeviceFailed;
@@ -579,6 +638,8 @@ int flash_bwd_dev(const void* dO, const void* Q, const void* K, const void* V, c
     p.dO = static_cast<const uint16_t*>(dO);
     p.O = O; p.LSE = LSE; p.Delta = delta; p.LSE2 = ws + rows;
     p.dQ = dQ; p.dK = dK; p.dV = dV;
+    p.dq_part = splits.dq > 1 ? ws + head_floats : nullptr;
+    p.dkv_part = splits.dkv > 1 ? ws + head_floats + dq_part : nullptr;
     p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.Sq = Sq; p.Sk = Sk;
     p.scale = scale;
     p.causal = causal ? 1 : 0;
@@ -586,14 +647,13 @@ int flash_bwd_dev(const void* dO, const void* Q, const void* K, const void* V, c
                       reinterpret_cast<uintptr_t>(V) | reinterpret_cast<uintptr_t>(dO) |
                       reinterpret_cast<uintptr_t>(dQ) | reinterpret_cast<uintptr_t>(dK) |
                       reinterpret_cast<uintptr_t>(dV)) & 15) == 0;
-    const bool mfma = al && scale_ok && (D == 128 || D == 64);
     hipLaunchKernelGGL((flash_bwd_delta_kernel<T>), dim3((unsigned)((rows * 16 + 255) / 256)), dim3(256), 0, s,
                        p.dO, p.O, p.LSE, delta, p.LSE2, (long)rows, D, mfma ? -1.f : 1.f,
                        mfma ? -1.f / scale : 1.f);
     rc = launch_status();
     if (rc == kOk) {
-      if (mfma && D == 128) rc = launch_bwd<T, 128>(p, s);
-      else if (mfma) rc = launch_bwd<T, 64>(p, s);
+      if (mfma && D == 128) rc = launch_bwd<T, 128>(p, splits, s);
+      else if (mfma) rc = launch_bwd<T, 64>(p, splits, s);
       else if (al && D > 128 && std::isfinite(scale) && (long)(Hq / Hkv) * Sq * Sk <= (1L << 33))   // (else: 112 GiB of scratch a group)
         rc = flash_bwd_dense_dev<T>(dO, Q, K, V, LSE, delta, dQ, dK, dV, B, Hq, Hkv, Sq, Sk, D, scale, causal, s);
       else {

@@ -39,6 +39,11 @@ struct FlashBwdParams {
   int B, Hq, Hkv, Sq, Sk;
   float scale;
   int causal;
+  // Few workgroups: the walk of each one is shared by gridDim.y workgroups, which write f32 partial
+  // gradients here instead: dq_part [split][B Hq Sq D], dkv_part [split][dK | dV][B Hkv Sk D]; null
+  // without a split.  flash_bwd_sum_kernel adds them in split order.
+  float* dq_part;
+  float* dkv_part;
 };
 
 constexpr float kLog2e = 1.44269504088896340736f;
@@ -96,6 +101,29 @@ __global__ void flash_bwd_delta_kernel(const uint16_t* __restrict__ dO, const fl
   }
 }
 
+// dst[i] = sum over the splits of part[split][i], in split order; blockIdx.y picks dQ, dK or dV.
+// One pass of 16-byte loads, four splits in flight per thread.
+__global__ __launch_bounds__(256) void flash_bwd_sum_kernel(const FlashBwdParams p, int dq_splits, int dkv_splits,
+                                                            long qn4, long kvn4) {
+  const int which = blockIdx.y;
+  const int ns = which == 0 ? dq_splits : dkv_splits;
+  if (ns <= 1) return;
+  const float4* part = reinterpret_cast<const float4*>(which == 0 ? p.dq_part : p.dkv_part) + (which == 2 ? kvn4 : 0);
+  float4* dst = reinterpret_cast<float4*>(which == 0 ? p.dQ : which == 1 ? p.dK : p.dV);
+  const long n = which == 0 ? qn4 : kvn4, stride = which == 0 ? qn4 : 2 * kvn4;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
+    float4 acc = part[i];
+    for (int s0 = 1; s0 < ns; s0 += 4) {
+      float4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = s0 + u < ns ? part[(s0 + u) * stride + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { acc.x += v[u].x; acc.y += v[u].y; acc.z += v[u].z; acc.w += v[u].w; }
+    }
+    dst[i] = acc;
+  }
+}
+
 // ---------------------------------------------------------------------------------
 // dQ: 8 waves x 32 query rows; K/V tiles of 64 keys stream global -> LDS.
 // ---------------------------------------------------------------------------------
@@ -137,7 +165,9 @@ __global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const Fl
 
   int kv_end = p.Sk;
   if (p.causal) kv_end = min(p.Sk, min(q0 + FB_BQ, p.Sq) - 1 + off + 1);
-  const int ntiles = (kv_end + FB_BKV - 1) / FB_BKV;
+  const int all_tiles = (kv_end + FB_BKV - 1) / FB_BKV;
+  const int share = (all_tiles + (int)gridDim.y - 1) / (int)gridDim.y;     // key tiles of a split
+  const int t0 = min((int)blockIdx.y * share, all_tiles), ntiles = min(t0 + share, all_tiles);
   int nt_w = 0;
   if (qw < p.Sq) {
     int e = kv_end;
@@ -202,14 +232,14 @@ __global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const Fl
 #pragma unroll
     for (int r = 0; r < 16; ++r) dq[dt][r] = 0.f;
 
-  if (ntiles > 0) {
-    load_tile(Kb, 0, 0);
-    load_tile(Vb, 0, 2);
+  if (ntiles > t0) {
+    load_tile(Kb, t0, 0);
+    load_tile(Vb, t0, 2);
   }
   fa_wait_loads();
   __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const int st = t & 1;
+  for (int t = t0; t < ntiles; ++t) {
+    const int st = (t - t0) & 1;
     if (t + 1 < ntiles) {
       load_tile(Kb, t + 1, st ^ 1);
       load_tile(Vb, t + 1, 2 + (st ^ 1));
@@ -272,12 +302,13 @@ __global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const Fl
     __syncthreads();
   }
   if (qi >= p.Sq) return;
+  float* out = p.dq_part ? p.dq_part + (long)blockIdx.y * p.B * p.Hq * p.Sq * D : p.dQ;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       const int d = dt * 32 + 8 * a + 4 * lh;
-      *reinterpret_cast<float4*>(p.dQ + (qrow0 + qi) * D + d) =
+      *reinterpret_cast<float4*>(out + (qrow0 + qi) * D + d) =
           make_float4(dq[dt][4 * a] * p.scale, dq[dt][4 * a + 1] * p.scale, dq[dt][4 * a + 2] * p.scale,
                       dq[dt][4 * a + 3] * p.scale);
     }
@@ -344,7 +375,12 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
   const int t_first = q_first / FB_BQT;
   const int qtiles = (p.Sq + FB_BQT - 1) / FB_BQT;
   const int steps_per_head = max(qtiles - t_first, 0);
-  const int nsteps = steps_per_head * ratio;
+  // this split's share of the walk: steps [step0, step0 + nsteps), step j being head j % ratio of the
+  // tile j / ratio from the last one down
+  const int all_steps = steps_per_head * ratio;
+  const int share = (all_steps + (int)gridDim.y - 1) / (int)gridDim.y;
+  const int step0 = min((int)blockIdx.y * share, all_steps);
+  const int nsteps = min(share, all_steps - step0);
 
   // loaders: global -> LDS, one wave instruction = 64 consecutive 16-byte slots
   int ld_row[LD_PER_WAVE];
@@ -389,10 +425,10 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
   auto next_of = [&](int& head, int& tile) {
     if (++head == ratio) { head = 0; --tile; }
   };
-  const int t_last = qtiles - 1;
+  const int h_first = step0 % ratio, t_last = qtiles - 1 - step0 / ratio;
   char* xch = smem + XCH + grp * 8192;
 
-  if (nsteps > 0) load_tile(0, t_last, 0);
+  if (nsteps > 0) load_tile(h_first, t_last, 0);
   fa_wait_loads();
   __syncthreads();
 
@@ -408,7 +444,7 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) row_rd[ks] = l32 * ROWB + ((((ks << 1) | lh) ^ bwd_swz<D>(l32)) << 4);
 
-    int cur_head = 0, cur_tile = t_last, st = 0;           // tile of this iteration and its stage
+    int cur_head = h_first, cur_tile = t_last, st = 0;           // tile of this iteration and its stage
     for (int i = 0; i <= nsteps; ++i) {
       int nxt_head = cur_head, nxt_tile = cur_tile;
       next_of(nxt_head, nxt_tile);
@@ -498,7 +534,7 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dk[dt][r] = 0.f; dv[dt][r] = 0.f; }
 
-  int ld_head = 0, ld_tile = t_last, lst = 0;              // tile i (whose successor is loaded) and its stage
+  int ld_head = h_first, ld_tile = t_last, lst = 0;              // tile i (whose successor is loaded) and its stage
   int cur_tile = t_last, st = 0;                           // tile i - 1 and its stage (from i = 1 on)
   for (int i = 0; i <= nsteps; ++i) {
     int nxt_head = ld_head, nxt_tile = ld_tile;
@@ -545,15 +581,18 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
     __syncthreads();
   }
   if (key >= p.Sk) return;
+  const long kvn = (long)p.B * p.Hkv * p.Sk * D;
+  float* dk_out = p.dkv_part ? p.dkv_part + (long)blockIdx.y * 2 * kvn : p.dK;
+  float* dv_out = p.dkv_part ? dk_out + kvn : p.dV;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       const int d = dt * 32 + 8 * a + 4 * lh;
       const long o = (kvrow0 + key) * D + d;
-      *reinterpret_cast<float4*>(p.dK + o) = make_float4(dk[dt][4 * a] * p.scale, dk[dt][4 * a + 1] * p.scale,
+      *reinterpret_cast<float4*>(dk_out + o) = make_float4(dk[dt][4 * a] * p.scale, dk[dt][4 * a + 1] * p.scale,
                                                          dk[dt][4 * a + 2] * p.scale, dk[dt][4 * a + 3] * p.scale);
-      *reinterpret_cast<float4*>(p.dV + o) =
+      *reinterpret_cast<float4*>(dv_out + o) =
           make_float4(dv[dt][4 * a], dv[dt][4 * a + 1], dv[dt][4 * a + 2], dv[dt][4 * a + 3]);
     }
 }

@@ -39,3 +39,22 @@ def test_forward_divisions(lane, b, hq, hkv, sq, sk, d, causal, window, dtype):
     assert orc.max_rel_err(o, ro) <= 2e-3
     seen = np.isfinite(rl)
     assert np.array_equal(np.isfinite(lse), seen) and np.max(np.abs(lse[seen] - rl[seen])) <= 2e-3
+
+
+@pytest.mark.parametrize("b,hq,hkv,sq,sk,d,causal,dtype", [
+    (1, 8, 1, 512, 512, 128, True, "bf16"),      # 8 heads a group: dK / dV walks shared, heads and tiles split unevenly
+    (1, 8, 1, 640, 640, 64, False, "f16"),
+    (1, 6, 2, 513, 513, 64, True, "bf16"),       # 3 heads a group, one row past a tile
+    (2, 4, 4, 129, 1100, 128, True, "bf16"),     # few query rows, long keys: dQ walks shared
+    (1, 4, 1, 1100, 300, 64, True, "f16"),       # more queries than keys
+    (1, 2, 2, 1024, 1024, 128, False, "bf16"),
+])
+def test_backward_shared_walks(lane, b, hq, hkv, sq, sk, d, causal, dtype):
+    (q, k, v, do), (qf, kf, vf, dof) = _case(b, hq, hkv, sq, sk, d, dtype, seed=5)
+    got = ops.flash_attn_backward(do, q, k, v, causal=causal)
+    ref = orc.flash_attn_backward(dof, qf, kf, vf, causal=causal)
+    bound = 5e-3 if dtype == "bf16" else 2e-3
+    for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+        assert orc.max_rel_err(g, r) <= bound, name
+    again = ops.flash_attn_backward(do, q, k, v, causal=causal)
+    assert all(np.array_equal(x, y) for x, y in zip(got, again))   # sums in split order: the same bits every time
