@@ -351,29 +351,22 @@ inline BwdSplits plan_bwd_splits(int B, int Hq, int Hkv, int Sq, int Sk, int D, 
 
 template <class T, int D>
 int launch_bwd(const FlashBwdParams& p, const BwdSplits& sp, hipStream_t s) {
-  constexpr int kDqSmem = 4 * FB_BKV * D * 2;
-  constexpr int kDkvSmem = flash_bwd_dkdv_lds_bytes<D>();
-  auto dq_kern = flash_bwd_dq_kernel<T, D>;
-  auto dkv_kern = flash_bwd_dkdv_kernel<T, D>;
+  constexpr int kSmem = std::max(4 * FB_BKV * D * 2, flash_bwd_dkdv_lds_bytes<D>());
+  auto kern = flash_bwd_kernel<T, D>;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
-    attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(dq_kern),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, kDqSmem);
-    if (attr_err == hipSuccess)
-      attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(dkv_kern),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, kDkvSmem);
+    attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
   });
   if (attr_err != hipSuccess) return kDeviceFailed;
-  hipLaunchKernelGGL(dq_kern, dim3(ceil_div(p.Sq, FB_BQ) * p.B * p.Hq, sp.dq), dim3(FB_DQ_THREADS), kDqSmem, s, p);
-  if (int rc = launch_status(); rc != kOk) return rc;
-  hipLaunchKernelGGL(dkv_kern, dim3(ceil_div(p.Sk, FB_BK) * p.B * p.Hkv, sp.dkv), dim3(FB_DKV_THREADS), kDkvSmem, s,
-                     p);
+  const int dq_blocks = ceil_div(p.Sq, FB_BQ) * p.B * p.Hq, dkv_blocks = ceil_div(p.Sk, FB_BK) * p.B * p.Hkv;
+  const int blocks = ceil_div(dkv_blocks * sp.dkv, 8) * 8 + dq_blocks * sp.dq;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(FB_DKV_THREADS), kSmem, s, p, dkv_blocks, sp.dkv, dq_blocks, sp.dq);
   if (sp.dq > 1 || sp.dkv > 1) {
     if (int rc = launch_status(); rc != kOk) return rc;
     const long qn4 = (long)p.B * p.Hq * p.Sq * D / 4, kvn4 = (long)p.B * p.Hkv * p.Sk * D / 4;
-    const long blocks = (std::max(sp.dq > 1 ? qn4 : 0, sp.dkv > 1 ? kvn4 : 0) + 255) / 256;
-    hipLaunchKernelGGL(flash_bwd_sum_kernel, dim3((unsigned)std::min<long>(blocks, 4096), 3), dim3(256), 0, s, p, sp.dq,
+    const long sums = (std::max(sp.dq > 1 ? qn4 : 0, sp.dkv > 1 ? kvn4 : 0) + 255) / 256;
+    hipLaunchKernelGGL(flash_bwd_sum_kernel, dim3((unsigned)std::min<long>(sums, 4096), 3), dim3(256), 0, s, p, sp.dq,
                        sp.dkv, qn4, kvn4);
   }
   return launch_status();

@@ -2,12 +2,14 @@
 // from dO, Q, K, V and the forward's O and log-sum-exp; GQA, 16-bit storage, f32
 // accumulate, f32 gradients.
 //
-// Three kernels, no atomics, results independent of scheduling:
+// No atomics, results independent of scheduling:
 //   flash_bwd_delta_kernel   Delta[q] = sum_d dO[q][d] O[q][d]
-//   flash_bwd_dq_kernel      one workgroup per 256 query rows, walks the key tiles
-//   flash_bwd_dkdv_kernel    one workgroup per 128 keys of one KV head, walks the
+//   flash_bwd_kernel         one launch of the workgroups of both walks:
+//     flash_bwd_dkdv         one workgroup per 128 keys of one KV head, walks the
 //                            query tiles of every query head that shares the KV head;
 //                            producer waves (S, dP, softmax) feed consumer waves (dK, dV)
+//     flash_bwd_dq           one workgroup per 256 query rows, walks the key tiles
+//   flash_bwd_sum_kernel     adds the partial gradients of walks that several workgroups share
 // Both walkers recompute P = exp(scale S - LSE) and dS = P (dP - Delta) tile by tile.
 // As in the forward kernel the products are oriented so that the index a lane owns
 // (its query row in the dQ kernel, its key in the dK/dV kernel) is the one the
@@ -39,7 +41,7 @@ struct FlashBwdParams {
   int B, Hq, Hkv, Sq, Sk;
   float scale;
   int causal;
-  // Few workgroups: the walk of each one is shared by gridDim.y workgroups, which write f32 partial
+  // Few workgroups: the walk of each one is shared by several workgroups, which write f32 partial
   // gradients here instead: dq_part [split][B Hq Sq D], dkv_part [split][dK | dV][B Hkv Sk D]; null
   // without a split.  flash_bwd_sum_kernel adds them in split order.
   float* dq_part;
@@ -129,8 +131,9 @@ __global__ __launch_bounds__(256) void flash_bwd_sum_kernel(const FlashBwdParams
 // ---------------------------------------------------------------------------------
 constexpr int FB_BQ = 256, FB_BKV = 64, FB_DQ_THREADS = 512;
 
+// (block, split, nsplits: this workgroup's place among those of dQ)
 template <class T, int D>
-__global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const FlashBwdParams p) {
+__device__ __forceinline__ void flash_bwd_dq(const FlashBwdParams& p, int block, int split, int nsplits) {
   constexpr int KSTEPS = D / 16, DT = D / 32, ROWB = D * 2, CHUNKS = D / 8;
   constexpr int TILE = FB_BKV * ROWB;
   constexpr int LD_PER_THREAD = FB_BKV * CHUNKS / FB_DQ_THREADS;
@@ -142,8 +145,8 @@ __global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const Fl
   const int l32 = lane & 31, lh = lane >> 5, r16 = lane & 15;
 
   const int qblocks = (p.Sq + FB_BQ - 1) / FB_BQ;
-  int qb = qblocks - 1 - blockIdx.x / (p.B * p.Hq);            // heavy causal blocks first
-  int bh = blockIdx.x % (p.B * p.Hq);
+  int qb = qblocks - 1 - block / (p.B * p.Hq);            // heavy causal blocks first
+  int bh = block % (p.B * p.Hq);
   if ((p.B * p.Hkv) % 8 == 0) {
     // Workgroups go to the XCDs round robin.  Runs of 8 ratio workgroups take 8 KV heads,
     // one per XCD, with all the query heads of a group on their KV head's XCD; then
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const Fl
     // The workgroups that walk the same K / V tiles share one L2, and an XCD works on
     // one or two KV heads at a time.
     const int ratio = p.Hq / p.Hkv;
-    const int w = blockIdx.x % (8 * ratio), r = blockIdx.x / (8 * ratio);
+    const int w = block % (8 * ratio), r = block / (8 * ratio);
     qb = qblocks - 1 - r % qblocks;
     bh = ((r / qblocks) * 8 + (w & 7)) * ratio + (w >> 3);
   }
@@ -166,8 +169,8 @@ __global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const Fl
   int kv_end = p.Sk;
   if (p.causal) kv_end = min(p.Sk, min(q0 + FB_BQ, p.Sq) - 1 + off + 1);
   const int all_tiles = (kv_end + FB_BKV - 1) / FB_BKV;
-  const int share = (all_tiles + (int)gridDim.y - 1) / (int)gridDim.y;     // key tiles of a split
-  const int t0 = min((int)blockIdx.y * share, all_tiles), ntiles = min(t0 + share, all_tiles);
+  const int share = (all_tiles + nsplits - 1) / nsplits;     // key tiles of a split
+  const int t0 = min(split * share, all_tiles), ntiles = min(t0 + share, all_tiles);
   int nt_w = 0;
   if (qw < p.Sq) {
     int e = kv_end;
@@ -302,7 +305,7 @@ __global__ __launch_bounds__(FB_DQ_THREADS, 1) void flash_bwd_dq_kernel(const Fl
     __syncthreads();
   }
   if (qi >= p.Sq) return;
-  float* out = p.dq_part ? p.dq_part + (long)blockIdx.y * p.B * p.Hq * p.Sq * D : p.dQ;
+  float* out = p.dq_part ? p.dq_part + (long)split * p.B * p.Hq * p.Sq * D : p.dQ;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -340,7 +343,7 @@ constexpr int flash_bwd_dkdv_lds_bytes() {
 }
 
 template <class T, int D>
-__global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const FlashBwdParams p) {
+__device__ __forceinline__ void flash_bwd_dkdv(const FlashBwdParams& p, int block, int split, int nsplits) {
   constexpr int KSTEPS = D / 16, DT = D / 32, ROWB = D * 2, CHUNKS = D / 8;
   constexpr int TILE = FB_BQT * ROWB;                      // bytes of a Q (or dO) tile
   constexpr int STAGE = 2 * TILE + 2 * FB_BQT * 4;         // Q | dO | -LSE/scale [64] | -Delta [64]
@@ -359,8 +362,8 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
   // an XCD one KV head after the other, all of its key blocks together, cuts the Q / dO
   // bytes fetched by the L2 to a third and costs 5 % in time: the blocks of one head
   // differ too much in length.)
-  const int kb = blockIdx.x / (p.B * p.Hkv);
-  const int bh = blockIdx.x % (p.B * p.Hkv);
+  const int kb = block / (p.B * p.Hkv);
+  const int bh = block % (p.B * p.Hkv);
   const int b = bh / p.Hkv, hkv = bh % p.Hkv;
   const int ratio = p.Hq / p.Hkv;
   const int off = p.Sk > p.Sq ? p.Sk - p.Sq : 0;
@@ -378,8 +381,8 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
   // this split's share of the walk: steps [step0, step0 + nsteps), step j being head j % ratio of the
   // tile j / ratio from the last one down
   const int all_steps = steps_per_head * ratio;
-  const int share = (all_steps + (int)gridDim.y - 1) / (int)gridDim.y;
-  const int step0 = min((int)blockIdx.y * share, all_steps);
+  const int share = (all_steps + nsplits - 1) / nsplits;
+  const int step0 = min(split * share, all_steps);
   const int nsteps = min(share, all_steps - step0);
 
   // loaders: global -> LDS, one wave instruction = 64 consecutive 16-byte slots
@@ -420,7 +423,7 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
   };
   // Walk order: query tiles from the last one down, the group's query heads innermost.
   // Every key block of a KV head starts at the same tile and moves at the same pace, so
-  // the workgroups that share Q / dO tiles (same XCD: blockIdx % 8 is the head's) read
+  // the workgroups that share Q / dO tiles (same XCD: block % 8 is the head's) read
   // them at the same time and the XCD's L2 serves all but one of those reads.
   auto next_of = [&](int& head, int& tile) {
     if (++head == ratio) { head = 0; --tile; }
@@ -582,7 +585,7 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
   }
   if (key >= p.Sk) return;
   const long kvn = (long)p.B * p.Hkv * p.Sk * D;
-  float* dk_out = p.dkv_part ? p.dkv_part + (long)blockIdx.y * 2 * kvn : p.dK;
+  float* dk_out = p.dkv_part ? p.dkv_part + (long)split * 2 * kvn : p.dK;
   float* dv_out = p.dkv_part ? dk_out + kvn : p.dV;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -595,6 +598,22 @@ __global__ __launch_bounds__(FB_DKV_THREADS) void flash_bwd_dkdv_kernel(const Fl
       *reinterpret_cast<float4*>(dv_out + o) =
           make_float4(dv[dt][4 * a], dv[dt][4 * a + 1], dv[dt][4 * a + 2], dv[dt][4 * a + 3]);
     }
+}
+
+// Both walks in one launch: neither needs the other's result, so the few workgroups of a small batch run side by side
+// and the last workgroups of dK / dV leave no compute unit idle.  dK / dV first (the longer walks); dQ starts at a
+// multiple of 8 workgroups, which keeps the XCD of each.
+template <class T, int D>
+__global__ __launch_bounds__(FB_DKV_THREADS, 2) void flash_bwd_kernel(const FlashBwdParams p, int dkv_blocks, int dkv_splits,
+                                                                      int dq_blocks, int dq_splits) {
+  static_assert(FB_DQ_THREADS == FB_DKV_THREADS, "one launch serves both");
+  const int n = dkv_blocks * dkv_splits, id = blockIdx.x;
+  if (id < n) {
+    flash_bwd_dkdv<T, D>(p, id % dkv_blocks, id / dkv_blocks, dkv_splits);
+  } else if (id >= (n + 7) / 8 * 8) {
+    const int j = id - (n + 7) / 8 * 8;
+    flash_bwd_dq<T, D>(p, j % dq_blocks, j / dq_blocks, dq_splits);
+  }
 }
 
 // Any head dimension: thread per query row (dQ) and thread per key row (dK, dV),
