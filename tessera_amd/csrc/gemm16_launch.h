@@ -306,16 +306,19 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     // splits keep that under about 0.4 of the operand traffic
     splits = (int)std::min<long>(splits, std::max<long>(2, (long)K * (M + N) / (10L * M * N)));
     while (splits > 1 && K % (splits * G16_BK) != 0) --splits;
-    // 9 to 32 rows: the streaming kernel on 128-column strips instead where its workgroups come out at
-    // nearly one per compute unit and B is more than a launch's worth of streaming (M = 16: 8192 x 8192
-    // 31.4 -> 28.1 us, 14336 x 4096 28.5 -> 25.8, 4096 x 4096 13.3 -> 11.4; level at 17 MB; at 186
-    // workgroups, 11840 columns, 20.9 against 22.8; with K ranges under 512, 16 x 2048 x 7168, 11.5 against
-    // 12.2), and where K has no even split that would give the tiles
-    // enough workgroups (27 x 3520 x 5312: 32.7 -> 13.7).
+    // 9 to 32 rows: the streaming kernel on 128-column strips instead where it streams faster than the tiles: one
+    // workgroup on every compute unit (16 x 8192 x 8192 31.4 -> 28.1 us, 4096 x 4096 12.7 -> 11.3, 8192 x 2048 10.4 ->
+    // 9.4; two parts of a short K, 16320 x 2560, 18.2 against 17.3), or nearly so and a B that is read with the
+    // non-temporal hint (7168 x 8192 29.4 -> 25.7, 14336 x 4096 28.5 -> 25.6).  Else the tiles: 7168 x 4096 15.4 against
+    // 13.0, 8064 x 4096 (252 workgroups) 16.2 against 14.1, 6144 x 8192 23.0 against 21.2, 14656 x 2176 15.4 against 13.9; with K ranges
+    // under 512, 2048 x 7168, 11.5 against 12.2.  And where K has no even split that would give the tiles enough
+    // workgroups (27 x 3520 x 5312: 32.7 -> 13.7).
     if (M <= kSkinnyWideMaxM && N >= 128) {
       const int wide = skinny_wide_splits(N, K);
       const long wgs = (long)ceil_div(N, 128) * wide;
-      if ((2.0 * K * N >= 2.4e7 && wgs >= 216 && wgs <= 256 && K >= 2048 && K / wide >= 512) || (K >= 2048 && tiles * splits < 128 && wgs > 2 * tiles * splits))
+      const double bytes = 2.0 * K * N;
+      const bool streams = bytes >= 1.1e8 ? wgs >= 216 : bytes >= 2.4e7 && wgs >= 256 && wide > 2;
+      if ((streams && wgs <= 256 && K >= 2048 && K / wide >= 512) || (K >= 2048 && tiles * splits < 128 && wgs > 2 * tiles * splits))
         return {128, wide, true};
     }
   }
