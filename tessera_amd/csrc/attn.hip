@@ -110,7 +110,8 @@ inline FlashShape flash_shape(const FlashParams& p) {
     return (p.B * p.Hkv % 8 ? 1.35 : 1.1) * std::max(longest, (w4.total + n4 * n * ends) / 512 + 0.5 * shortest) + merge;
   };
   int best = 1;
-  const int most = (int)std::min<long>(std::min<long>(std::max<long>(512 / n4, 1), ceil_div(p.Sk, FA_BKV) / 8), 64);
+  // (from 192 blocks on never: a split takes the stream's workspace, which a captured call must find allocated)
+  const int most = n8 >= 192 ? 1 : (int)std::min<long>(std::min<long>(std::max<long>(512 / n4, 1), ceil_div(p.Sk, FA_BKV) / 8), 64);
   for (int n = 2; n <= most; ++n)
     if (t4(n) < t4(best)) best = n;
   // (splits of short walks that put two workgroups on a unit are no better than 8 waves and theirs: B 1 x Hq 8 x
