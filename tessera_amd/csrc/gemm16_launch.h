@@ -2,6 +2,7 @@
 #pragma once
 #include <algorithm>
 #include <mutex>
+#include "few_rows.h"
 #include "gemm16.h"
 #include "gemm16_skinny.h"
 #include "host_util.h"
@@ -491,7 +492,7 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
                    (!p.bias || aligned16(p.bias));
   if (!vec) {
     // few rows: the streaming kernel reads B where it lies
-    if (p.groups == 1 && p.M <= kLooseMaxM && p.N >= 8)
+    if (p.groups == 1 && p.M <= kLooseMaxM && p.N >= 8 && few_rows16_in_range(p.M, p.N, p.K, p.lda, p.ldb))
       return launch_gemm16_skinny<T, EPI>(p, skinny_loose_splits(p.N, p.K), true, s);
     // small products go one thread per output element; above about 2^24 multiply-adds the
     // copies into aligned buffers cost less than that kernel loses

@@ -77,3 +77,28 @@ def test_attention_operands_beyond_2_31_elements(lane):
         ro, rl = orc.flash_attn_dense(qq, kk, vv, causal=True)       # bottom-right aligned: row i sees keys <= r0 + i
         assert orc.max_rel_err(_f32(out[b, h, rows]), ro[0, 0]) <= 2e-3 + 2.0 ** -8, (b, h, r0)
         assert np.max(np.abs(lse[b, h, rows] - rl[0, 0])) <= 2e-3, (b, h, r0)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 8, 17_100_000), (2, (1 << 26) + 129, 33)])
+def test_few_rows_with_pitches_beyond_32_bit_offsets(lane, M, N, K):
+    """Few rows off the 16-byte grid with a pitch whose row offsets pass 2^31 bytes (A: 64 rows of 34.2 MB) or wrap
+    2^32 (a slice of B: 32 rows of 134 MB).  Values -1, 0 and 1: every sum is a whole number below 2^24, exact in f32."""
+    rng = np.random.default_rng(K)
+    values = np.array([0xBF80, 0, 0x3F80], np.uint16)               # -1, 0, 1 in bf16
+    block = values[rng.integers(0, 3, 1 << 22)]
+    a = np.resize(block, M * K).reshape(M, K)
+    b = np.resize(block[12345:], K * N).reshape(K, N)
+    da, db = lane.DeviceBuffer.from_host(a), lane.DeviceBuffer.from_host(b)
+    dd = lane.DeviceBuffer(M * N * 4)
+    try:
+        lane.check(lane.load().tessera_gfx950_gemm_bf16_dev(da.ptr, db.ptr, dd.ptr, M, N, K, None), "gemm")
+        lane.synchronize()
+        out = dd.download((M, N), np.float32)
+    finally:
+        for buf in (da, db, dd):
+            buf.close()
+    cols = np.arange(N) if N < 1000 else np.r_[0:200, N // 2:N // 2 + 200, N - 300:N]
+    for m in (0, M // 2, M - 1):
+        ref = sum(_f32(a[m, k0:k0 + (1 << 20)]).astype(np.float64) @ _f32(b[k0:k0 + (1 << 20), cols]).astype(np.float64)
+                  for k0 in range(0, K, 1 << 20))
+        assert np.abs(ref).max() < 2 ** 24 and np.array_equal(out[m, cols], ref), m
