@@ -95,18 +95,29 @@ int gemm8_repitched(const Gemm8Params& p, hipStream_t s) {
   return rc;
 }
 
+// Whether a product off the 16-byte grid is worth the copies into aligned, zero-padded buffers: small ones go one
+// thread per output element; above about 2^24 multiply-adds the copies cost less than that kernel loses.
+inline bool gemm8_worth_copies(int M, int N, int K) {
+  return (double)M * N * K >= (double)(1L << 24) && M >= 16 && N >= 16 && K + 16 < (1 << 22) && N + 16 < (1 << 22);
+}
+
 // The few-row streaming kernel with K in `splits` parts (more than one: then the sum).  loose: rows of B on any boundary; A is
-// then copied into rows padded with zeros to a multiple of 16 where its own cannot be read 16 bytes at a time.
+// then copied into rows padded with zeros to a multiple of 16 where its own cannot be read 16 bytes at a time, and
+// fp8 products that it takes over from the one-thread-per-element kernel keep that kernel's f32 sums (WIDEN).
 // (8 waves and about 256 workgroups measured best for up to 32 rows: 4-wave workgroups, two per
 // compute unit, and 384 or 512 workgroups were level or slower on M = 1 ... 32 against 4096 ...
 // 28672 columns.  33 to 64 rows double the accumulators: 4 waves, one per SIMD.)
 template <class T, int EPI>
 int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
+  constexpr bool FP8 = !std::is_same<T, I8>::value;
   const bool one = p.M <= 32;
   const int nw = one ? 8 : 4;
+  const int form = !loose ? 0 : FP8 && !gemm8_worth_copies(p.M, p.N, p.K) ? 2 : 1;
   using Kernel = void (*)(const Gemm8Params, int, int, void*, int);
-  static const Kernel kernels[2][2] = {{gemm8_skinny_kernel<T, 4, 2, EPI, false>, gemm8_skinny_kernel<T, 4, 2, EPI, true>},
-                                       {gemm8_skinny_kernel<T, 8, 1, EPI, false>, gemm8_skinny_kernel<T, 8, 1, EPI, true>}};
+  static const Kernel kernels[2][3] = {{gemm8_skinny_kernel<T, 4, 2, EPI, false, false>, gemm8_skinny_kernel<T, 4, 2, EPI, true, false>,
+                                        gemm8_skinny_kernel<T, 4, 2, EPI, true, FP8>},
+                                       {gemm8_skinny_kernel<T, 8, 1, EPI, false, false>, gemm8_skinny_kernel<T, 8, 1, EPI, true, false>,
+                                        gemm8_skinny_kernel<T, 8, 1, EPI, true, FP8>}};
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
@@ -141,7 +152,7 @@ int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
   }
   void* part = splits > 1 ? ws + a_bytes : nullptr;
   const int vec = p.N % 4 == 0 && aligned16(p.D) && (!p.acc_out || aligned16(p.acc_out)) && (!p.col_scale || aligned16(p.col_scale));
-  hipLaunchKernelGGL(kernels[one][loose], dim3(strips, splits), dim3(nw * 64), g8s_smem(nw, std::min(p.M, 32)), s, q, lda, kps, part,
+  hipLaunchKernelGGL(kernels[one][form], dim3(strips, splits), dim3(nw * 64), g8s_smem(nw, std::min(p.M, 32)), s, q, lda, kps, part,
                      vec);
   if (int rc = launch_status(); rc != kOk || !part) return rc;
   return launch_gemm8_split_sum<T, EPI>(part, splits, ldw, vec, p, s);
@@ -159,10 +170,7 @@ int gemm8_dev(Gemm8Params p, hipStream_t s) {
     // few rows: the streaming kernel reads B where it lies
     if (p.M <= kGemm8SkinnyMaxM && p.N >= 16 && p.N < (1 << 25) && p.K < (1 << 24))
       return gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(p.M, p.N, p.K), true, s);
-    // small products go one thread per output element; above about 2^24 multiply-adds the copies
-    // into aligned, zero-padded buffers cost less than that kernel loses
-    if ((double)p.M * p.N * p.K >= (double)(1L << 24) && p.M >= 16 && p.N >= 16 && p.K + 16 < (1 << 22) && p.N + 16 < (1 << 22))
-      return gemm8_repitched<T, EPI>(p, s);
+    if (gemm8_worth_copies(p.M, p.N, p.K)) return gemm8_repitched<T, EPI>(p, s);
     dim3 block(32, 8), grid(ceil_div(p.N, 32), ceil_div(p.M, 8), 1);
     hipLaunchKernelGGL((gemm8_generic_kernel<T, EPI>), grid, block, 0, s, p);
     return launch_status();

@@ -49,3 +49,34 @@ def test_few_rows_8bit(lane, M, N, K):
     codes_a, _, sa = orc.quantize_fp8_e4m3(rng.standard_normal((M, K)).astype(np.float32))
     codes_b, _, sb = orc.quantize_fp8_e4m3(rng.standard_normal((K, N)).astype(np.float32))
     assert orc.max_rel_err(ops.gemm_fp8(codes_a, codes_b, sa, sb, out="f32"), orc.gemm_e4m3(codes_a, codes_b, sa, sb)) <= 2e-3
+
+
+# fp8 off the 16-byte grid, below 2^24 multiply-adds or under 16 rows (one and two row blocks, split and unsplit K)
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("M,N,K", [(1, 17, 203), (5, 130, 201), (15, 1003, 2111), (33, 33, 203), (64, 1003, 259)])
+def test_few_rows_fp8_adds_small_products(lane, fmt, M, N, K):
+    """Products 14 binary places below their neighbours: every partial sum has at most 21 bits, so sums in f32 are exact
+    in any order, where the fp8 matrix instruction drops all of them (4e-4 of the result)."""
+    big, small = (0x58, 0x20) if fmt == "e4m3" else (0x4C, 0x30)          # 16 and 1/8
+    at = np.arange(K) % 8 == 3
+    a = np.where(at, big, small).astype(np.uint8) * np.ones((M, 1), np.uint8)
+    b = (np.where(at, big, small).astype(np.uint8) * np.ones((N, 1), np.uint8)).T
+    want = at.sum() * 256.0 + (~at).sum() / 64.0
+    assert want * 64 < 2 ** 24
+    got = ops.gemm_fp8(a, np.ascontiguousarray(b), 1.0, 1.0, out="f32", format=fmt)
+    assert np.all(got == want), np.unique(got)[:5]
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+def test_few_rows_fp8_every_code(lane, fmt):
+    """All 256 codes times one, in an off-grid product of 16 rows: the value itself; a column that
+    holds an infinity or a NaN is NaN throughout."""
+    one = 0x38 if fmt == "e4m3" else 0x3C
+    a = np.where(np.eye(16, dtype=bool), one, 0).astype(np.uint8)
+    b = np.zeros((16, 17), np.uint8)
+    b[:, :16] = np.arange(256, dtype=np.uint8).reshape(16, 16).T          # column n: codes 16 n .. 16 n + 15
+    table = (orc.e4m3_decode_table() if fmt == "e4m3" else orc.e5m2_decode_table()).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = table[a] @ table[b]
+    got = ops.gemm_fp8(a, b, 1.0, 1.0, out="f32", format=fmt)
+    assert np.array_equal(got, want.astype(np.float32), equal_nan=True)
