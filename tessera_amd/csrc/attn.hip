@@ -147,8 +147,9 @@ int launch_flash_for(const FlashParams& p, bool ext, hipStream_t s) {
 }
 
 // Few query rows per KV head (decode, short speculative steps): the rows of a whole GQA group
-// share one MFMA tile and the key range is split over workgroups (flash_decode.h).  Returns
-// false when the problem is not of that kind (the general kernel then serves it).
+// share one MFMA tile and the key range is split over workgroups (flash_decode.h).  kNoScratch: padded head
+// dimensions, whose key splits found no workspace (a capture on a stream that has none); the general
+// kernel then serves them, whose launches of 192 and more blocks need none.
 template <class T, int DP, int NQ, bool PAD, bool NT>
 int launch_decode_as(const FlashParams& p, hipStream_t s) {
   using G = DecodeGeom<DP>;
@@ -176,8 +177,9 @@ int launch_decode_as(const FlashParams& p, hipStream_t s) {
   nsplit = ceil_div(tiles, dp.tiles_per_split);
   if (nsplit > 1) {
     const size_t rows = (size_t)p.B * p.Hq * p.Sq;
-    float* ws = static_cast<float*>(stream_workspace(s, (size_t)nsplit * rows * (p.D + 1) * sizeof(float)));
-    if (!ws) return kDeviceFailed;
+    const size_t bytes = (size_t)nsplit * rows * (p.D + 1) * sizeof(float);
+    float* ws = static_cast<float*>(PAD ? stream_workspace_or_null(s, bytes) : stream_workspace(s, bytes));
+    if (!ws) return PAD ? kNoScratch : kDeviceFailed;
     dp.part_o = ws;
     dp.part_lse = ws + (size_t)nsplit * rows * p.D;
   }
@@ -261,10 +263,11 @@ int flash_dev(const void* Q, const void* K, const void* V, void* O, void* LSE, i
   const bool ext = p.softcap > 0.f || p.bias != nullptr || !(scale > 0.f);
   if (al && !ext && decode_shaped(p)) {
     const int rows = p.ratio * p.Sq;
-    if (p.D <= 64) return rows <= 32 ? launch_decode<T, 64, 1>(p, s) : rows <= 64 ? launch_decode<T, 64, 2>(p, s)
-                                                                                  : launch_decode<T, 64, 4>(p, s);
-    if (p.D <= 128) return rows <= 32 ? launch_decode<T, 128, 1>(p, s) : launch_decode<T, 128, 2>(p, s);
-    return launch_decode<T, 256, 1>(p, s);
+    const int rc = p.D <= 64 ? (rows <= 32 ? launch_decode<T, 64, 1>(p, s) : rows <= 64 ? launch_decode<T, 64, 2>(p, s)
+                                                                                        : launch_decode<T, 64, 4>(p, s))
+                   : p.D <= 128 ? (rows <= 32 ? launch_decode<T, 128, 1>(p, s) : launch_decode<T, 128, 2>(p, s))
+                                : launch_decode<T, 256, 1>(p, s);
+    if (rc != kNoScratch) return rc;
   }
   if (al) return launch_flash_for<T>(p, ext, s);
   const long rows = (long)B * Hq * Sq;

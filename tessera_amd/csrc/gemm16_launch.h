@@ -342,11 +342,12 @@ int launch_gemm16_skinny_as(const Gemm16Params& p, int kps, int splits, float* p
 }
 
 // The few-row streaming kernel with K in `splits` parts.  loose: see the kernel; A is then copied into
-// rows padded with zeros to a multiple of 8 where its own cannot be read 16 bytes at a time.
+// rows padded with zeros to a multiple of 8 where its own cannot be read 16 bytes at a time.  Without a
+// workspace (a capture on a stream that has none) K stays whole; a copy of A that has no room is kNoScratch.
 template <class T, int EPI>
 int launch_gemm16_skinny(Gemm16Params p, int splits, bool loose, hipStream_t s) {
   const int cols = p.M <= kSkinnyMaxM && !loose ? 64 : 128;
-  const int kps = ceil_div(ceil_div(p.K, splits), 32) * 32;
+  int kps = ceil_div(ceil_div(p.K, splits), 32) * 32;
   splits = ceil_div(p.K, kps);
   const long ldw = (long)ceil_div(p.N, cols) * cols;
   const int K8 = (p.K + 7) & ~7;
@@ -355,8 +356,9 @@ int launch_gemm16_skinny(Gemm16Params p, int splits, bool loose, hipStream_t s) 
   const size_t part_bytes = splits > 1 ? (size_t)splits * p.M * ldw * 4 : 0;
   char* ws = nullptr;
   if (a_bytes + part_bytes) {
-    ws = static_cast<char*>(stream_workspace(s, a_bytes + part_bytes));
-    if (!ws) return kDeviceFailed;
+    ws = static_cast<char*>(stream_workspace_or_null(s, a_bytes + part_bytes));
+    if (!ws && a_copy) return kNoScratch;
+    if (!ws) { splits = 1; kps = ceil_div(p.K, 32) * 32; }
   }
   float* part = splits > 1 ? reinterpret_cast<float*>(ws + a_bytes) : nullptr;
   constexpr int dsz = EPI == EPI_F32 ? 4 : 2;
@@ -492,8 +494,10 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
                    (!p.bias || aligned16(p.bias));
   if (!vec) {
     // few rows: the streaming kernel reads B where it lies
-    if (p.groups == 1 && p.M <= kLooseMaxM && p.N >= 8 && few_rows16_in_range(p.M, p.N, p.K, p.lda, p.ldb))
-      return launch_gemm16_skinny<T, EPI>(p, skinny_loose_splits(p.N, p.K), true, s);
+    if (p.groups == 1 && p.M <= kLooseMaxM && p.N >= 8 && few_rows16_in_range(p.M, p.N, p.K, p.lda, p.ldb)) {
+      const int rc = launch_gemm16_skinny<T, EPI>(p, skinny_loose_splits(p.N, p.K), true, s);
+      if (rc != kNoScratch) return rc;
+    }
     // small products go one thread per output element; above about 2^24 multiply-adds the
     // copies into aligned buffers cost less than that kernel loses
     if ((double)p.M * p.N * p.K * p.groups >= (double)(1L << 24) && p.M >= 16 && p.N >= 16 &&

@@ -104,6 +104,7 @@ inline bool gemm8_worth_copies(int M, int N, int K) {
 // The few-row streaming kernel with K in `splits` parts (more than one: then the sum).  loose: rows of B on any boundary; A is
 // then copied into rows padded with zeros to a multiple of 16 where its own cannot be read 16 bytes at a time, and
 // fp8 products that it takes over from the one-thread-per-element kernel keep that kernel's f32 sums (WIDEN).
+// Without a workspace (a capture on a stream that has none) K stays whole; a copy of A that has no room is kNoScratch.
 // (8 waves and about 256 workgroups measured best for up to 32 rows: 4-wave workgroups, two per
 // compute unit, and 384 or 512 workgroups were level or slower on M = 1 ... 32 against 4096 ...
 // 28672 columns.  33 to 64 rows double the accumulators: 4 waves, one per SIMD.)
@@ -129,7 +130,7 @@ int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
   });
   if (attr_err != hipSuccess) return kDeviceFailed;
   const int strips = ceil_div(p.N, G8S_COLS);
-  const int kps = ceil_div(ceil_div(p.K, splits), G8S_ROWS) * G8S_ROWS;
+  int kps = ceil_div(ceil_div(p.K, splits), G8S_ROWS) * G8S_ROWS;
   splits = ceil_div(p.K, kps);
   const long ldw = (long)strips * G8S_COLS;
   const int K16 = (p.K + 15) & ~15;
@@ -138,8 +139,9 @@ int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
   const size_t part_bytes = splits > 1 ? (size_t)splits * p.M * ldw * 4 : 0;
   char* ws = nullptr;
   if (a_bytes + part_bytes) {
-    ws = static_cast<char*>(stream_workspace(s, a_bytes + part_bytes));
-    if (!ws) return kDeviceFailed;
+    ws = static_cast<char*>(stream_workspace_or_null(s, a_bytes + part_bytes));
+    if (!ws && a_copy) return kNoScratch;
+    if (!ws) { splits = 1; kps = ceil_div(p.K, G8S_ROWS) * G8S_ROWS; }
   }
   Gemm8Params q = p;
   int lda = p.K;
@@ -168,8 +170,10 @@ int gemm8_dev(Gemm8Params p, hipStream_t s) {
                    (!p.acc_out || aligned16(p.acc_out)) && (!p.col_scale || aligned16(p.col_scale));
   if (!vec) {
     // few rows: the streaming kernel reads B where it lies
-    if (p.M <= kGemm8SkinnyMaxM && p.N >= 16 && p.N < (1 << 25) && p.K < (1 << 24))
-      return gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(p.M, p.N, p.K), true, s);
+    if (p.M <= kGemm8SkinnyMaxM && p.N >= 16 && p.N < (1 << 25) && p.K < (1 << 24)) {
+      const int rc = gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(p.M, p.N, p.K), true, s);
+      if (rc != kNoScratch) return rc;
+    }
     if (gemm8_worth_copies(p.M, p.N, p.K)) return gemm8_repitched<T, EPI>(p, s);
     dim3 block(32, 8), grid(ceil_div(p.N, 32), ceil_div(p.M, 8), 1);
     hipLaunchKernelGGL((gemm8_generic_kernel<T, EPI>), grid, block, 0, s, p);

@@ -109,6 +109,11 @@ int bench_loop(Launch&& launch, int iters, double* avg_ms) {
 // buffer must already have its final size (run the call once outside the capture).
 // Returns null on failure.
 void* stream_workspace(hipStream_t s, size_t bytes);
+// The same for a path that has another one to fall back on: null, without an attempt to allocate, when
+// the stream is being captured and its workspace is not that large yet.
+void* stream_workspace_or_null(hipStream_t s, size_t bytes);
+// Status inside the library: the path needs scratch it could not have, nothing was launched, another path serves.
+constexpr int kNoScratch = -1;
 // Synchronises `s` and frees its workspace; a later call on the stream allocates afresh.
 int stream_workspace_release(hipStream_t s);
 // Looks up the device address of the allocation-free routing entry's scratch array for the

@@ -67,6 +67,19 @@ void* stream_workspace(hipStream_t s, size_t bytes) {
   return p;
 }
 
+void* stream_workspace_or_null(hipStream_t s, size_t bytes) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+  {
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    auto it = g_ws_slots.find({dev, s});
+    if (it != g_ws_slots.end() && it->second.ptr && it->second.bytes >= bytes) return it->second.ptr;
+  }
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) (void)hipGetLastError();
+  return status == hipStreamCaptureStatusNone ? stream_workspace(s, bytes) : nullptr;
+}
+
 // Waits for the stream, then frees its workspace (the buffer in use and the outgrown ones).
 int stream_workspace_release(hipStream_t s) {
   int dev = 0;
