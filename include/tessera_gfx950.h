@@ -102,7 +102,8 @@ int tessera_gfx950_free(void* dptr);
  * handed out again at once, and its next user must be on the default stream or ordered behind it.  shared != 0:
  * it may be in use in other streams; it is handed out again only after the device has been synchronised
  * (tessera_gfx950_synchronize, or by the pool itself once 16 blocks of a size, or 256 MB of them, wait).  The pool
- * caches at most 4 GiB and keeps blocks per device; pool_trim gives everything cached back.  Safe from any thread.
+ * caches at most 4 GiB and keeps blocks per device; pool_trim gives everything cached back, and so does any allocation
+ * of the library that finds the device out of memory.  Safe from any thread.
  * No counterpart in the reference, which allocates per call. */
 int tessera_gfx950_pool_malloc(void** dptr, size_t bytes);
 int tessera_gfx950_pool_free(void* dptr, int shared);

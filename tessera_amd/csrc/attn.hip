@@ -415,10 +415,7 @@ int flash_bwd_padded_dev(const void* dO, const void* Q, const void* K, const voi
   const size_t b16q = rows * DP * 2, b16k = kvrows * DP * 2, f32q = rows * DP * 4, f32k = kvrows * DP * 4;
   const size_t extra = recompute ? rows * D * 4 + rows * 4 : 0;
   char* ws = nullptr;
-  if (hipMallocAsync(reinterpret_cast<void**>(&ws), 2 * b16q + 2 * b16k + 2 * f32q + 2 * f32k + extra, s) != hipSuccess) {
-    (void)hipGetLastError();
-    return kDeviceFailed;
-  }
+  if (!device_malloc_async(reinterpret_cast<void**>(&ws), 2 * b16q + 2 * b16k + 2 * f32q + 2 * f32k + extra, s)) return kDeviceFailed;
   char* Qp = ws; char* dOp = Qp + b16q; char* Kp = dOp + b16q; char* Vp = Kp + b16k;
   char* Op = Vp + b16k; char* dQp = Op + f32q; char* dKp = dQp + f32q; char* dVp = dKp + f32k;
   int rc = kOk;
@@ -543,10 +540,7 @@ int flash_bwd_dense_dev(const void* dO, const void* Q, const void* K, const void
   const size_t budget = (size_t)2 << 30;                                      // aim for 2 GiB of scratch per chunk
   const int gpc = (int)std::max<size_t>(1, std::min<size_t>(groups, budget / per_group));
   char* ws = nullptr;
-  if (hipMallocAsync(reinterpret_cast<void**>(&ws), per_group * gpc + 256, s) != hipSuccess) {
-    (void)hipGetLastError();
-    return kDeviceFailed;
-  }
+  if (!device_malloc_async(reinterpret_cast<void**>(&ws), per_group * gpc + 256, s)) return kDeviceFailed;
   const size_t e = (size_t)rows * Sk;
   float* Sb = reinterpret_cast<float*>(ws);
   float* dPb = Sb + e * gpc;
@@ -614,10 +608,7 @@ int flash_bwd_dev(const void* dO, const void* Q, const void* K, const void* V, c
   const size_t head_floats = (2 * rows + (recompute ? rows * D + rows : 0) + 3) / 4 * 4;
   const size_t dq_part = splits.dq > 1 ? splits.dq * rows * D : 0;
   const size_t ws_floats = head_floats + dq_part + (splits.dkv > 1 ? splits.dkv * 2 * kvrows_all * D : 0);
-  if (hipMallocAsync(reinterpret_cast<void**>(&ws), ws_floats * sizeof(float), s) != hipSuccess) {
-    (void)hipGetLastError();
-    return kDeviceFailed;
-  }
+  if (!device_malloc_async(reinterpret_cast<void**>(&ws), ws_floats * sizeof(float), s)) return kDeviceFailed;
   int rc = kOk;
   float* delta = ws;
   if (recompute) {

@@ -407,10 +407,7 @@ int launch_gemm16_repitched(const Gemm16Params& p, hipStream_t s) {
   const size_t a_bytes = a_ok ? 0 : (size_t)G * p.M * K8 * 2, b_bytes = b_ok ? 0 : (size_t)G * K8 * N8 * 2;
   const size_t d_bytes = d_ok ? 0 : (size_t)G * p.M * N8 * dsz, bias_bytes = bias_ok ? 0 : (size_t)N8 * 4;
   char* ws = nullptr;
-  if (hipMallocAsync(reinterpret_cast<void**>(&ws), a_bytes + b_bytes + d_bytes + bias_bytes + 16, s) != hipSuccess) {
-    (void)hipGetLastError();
-    return kDeviceFailed;
-  }
+  if (!device_malloc_async(reinterpret_cast<void**>(&ws), a_bytes + b_bytes + d_bytes + bias_bytes + 16, s)) return kDeviceFailed;
   Gemm16Params q = p;
   q.K = K8;
   q.N = N8;
@@ -593,10 +590,7 @@ int launch_gemm16_gated(Gemm16Params p, hipStream_t s) {
       (long)p.M * p.N >= 128L * 128L) {
     const size_t mn = (size_t)p.M * p.N;
     float* tmp = nullptr;
-    if (hipMallocAsync(reinterpret_cast<void**>(&tmp), 2 * mn * sizeof(float), s) != hipSuccess) {
-      (void)hipGetLastError();
-      return kDeviceFailed;
-    }
+    if (!device_malloc_async(reinterpret_cast<void**>(&tmp), 2 * mn * sizeof(float), s)) return kDeviceFailed;
     Gemm16Params q = p;
     q.B2 = nullptr;
     q.act = ACT_NONE;

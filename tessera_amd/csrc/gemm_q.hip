@@ -46,10 +46,7 @@ int gemm8_repitched(const Gemm8Params& p, hipStream_t s) {
   const size_t d_bytes = d_ok ? 0 : (size_t)p.M * N16 * dsz, acc_bytes = acc_ok ? 0 : (size_t)p.M * N16 * 4;
   const size_t cs_bytes = cs_ok ? 0 : (size_t)N16 * 4;
   char* ws = nullptr;
-  if (hipMallocAsync(reinterpret_cast<void**>(&ws), a_bytes + b_bytes + d_bytes + acc_bytes + cs_bytes + 16, s) != hipSuccess) {
-    (void)hipGetLastError();
-    return kDeviceFailed;
-  }
+  if (!device_malloc_async(reinterpret_cast<void**>(&ws), a_bytes + b_bytes + d_bytes + acc_bytes + cs_bytes + 16, s)) return kDeviceFailed;
   Gemm8Params q = p;
   q.K = K16;
   q.N = N16;

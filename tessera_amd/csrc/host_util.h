@@ -16,6 +16,11 @@ int probe_device();
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// hipMalloc and hipMallocAsync for the whole library: where the device is out of memory, the blocks cached by the
+// pool of resident results (up to 4 GiB) are given back and the call is tried once more.
+bool device_malloc(void** p, size_t bytes);
+bool device_malloc_async(void** p, size_t bytes, hipStream_t s);
+
 // Serialises the host-pointer entry points.  Each of them uploads, runs its device-pointer
 // twin on the null stream, synchronises and downloads; the twin takes its scratch (split-K
 // partials, routing lists, quantiser maxima) from the null stream's workspace at offset 0.
@@ -38,7 +43,7 @@ class DeviceScope {
   // Allocates `bytes` (at least 16) and, when `src` is given, copies it in.
   void* alloc(size_t bytes, const void* src = nullptr) {
     void* d = nullptr;
-    if (hipMalloc(&d, bytes < 16 ? 16 : bytes) != hipSuccess) { failed_ = true; return nullptr; }
+    if (!device_malloc(&d, bytes < 16 ? 16 : bytes)) { failed_ = true; return nullptr; }
     ptrs_.push_back(d);
     if (src && bytes && hipMemcpy(d, src, bytes, hipMemcpyHostToDevice) != hipSuccess) failed_ = true;
     return d;

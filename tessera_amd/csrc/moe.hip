@@ -971,7 +971,7 @@ int swiglu_dev(const void* x, const void* wg, const void* wu, const void* wd, co
   if (probe_device() != kOk) return kNoDevice;
   if (S == 0) return kOk;
   void* h = hidden;
-  if (!h && hipMallocAsync(&h, (size_t)S * F * 2, s) != hipSuccess) return kDeviceFailed;
+  if (!h && !device_malloc_async(&h, (size_t)S * F * 2, s)) return kDeviceFailed;
   Gemm16Params p{};
   p.A = static_cast<const uint16_t*>(x);
   p.B = static_cast<const uint16_t*>(wg);

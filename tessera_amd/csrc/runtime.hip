@@ -1,5 +1,4 @@
 // Device management half of the C ABI: probe, raw buffers, event timers.
-#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstring>
@@ -8,6 +7,7 @@
 #include <utility>
 #include <vector>
 #include "../../include/tessera_gfx950.h"
+#include "device_pool.h"
 #include "host_util.h"
 
 namespace tsr950 {
@@ -39,6 +39,32 @@ int probe_device() {
 }
 
 namespace {
+PoolAlloc pool_alloc_of(hipError_t e) {
+  if (e == hipSuccess) return PoolAlloc::kOk;
+  (void)hipGetLastError();
+  return e == hipErrorOutOfMemory ? PoolAlloc::kNoMemory : PoolAlloc::kFailed;
+}
+struct HipPoolApi {
+  static bool ok(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  }
+  static bool device(int* dev) { return ok(hipGetDevice(dev)); }
+  static PoolAlloc malloc(void** p, size_t bytes) { return pool_alloc_of(hipMalloc(p, bytes)); }
+  static bool free(void* p) { return ok(hipFree(p)); }
+  static bool synchronize() { return hipDeviceSynchronize() == hipSuccess; }
+};
+DevicePool<HipPoolApi> g_pool;
+}  // namespace
+
+bool device_malloc(void** p, size_t bytes) {
+  return g_pool.allocate([&] { return pool_alloc_of(hipMalloc(p, bytes)); });
+}
+bool device_malloc_async(void** p, size_t bytes, hipStream_t s) {
+  return g_pool.allocate([&] { return pool_alloc_of(hipMallocAsync(p, bytes, s)); });
+}
+
+namespace {
 struct WorkspaceSlot {
   void* ptr = nullptr;
   size_t bytes = 0;
@@ -60,7 +86,7 @@ void* stream_workspace(hipStream_t s, size_t bytes) {
   size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
   if (want < 2 * slot.bytes) want = 2 * slot.bytes;
   void* p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+  if (!device_malloc(&p, want)) return nullptr;
   if (slot.ptr) slot.retired.push_back(slot.ptr);
   slot.ptr = p;
   slot.bytes = want;
@@ -99,128 +125,6 @@ int stream_workspace_release(hipStream_t s) {
     if (hipFree(p) != hipSuccess) rc = kDeviceFailed;
   if (rc != kOk) (void)hipGetLastError();
   return rc;
-}
-
-// Device memory for results that a chain of default-stream calls allocates and drops (hipMalloc and hipFree
-// cost about 65 us a pair and the free waits for the device: three of them were half the time of an attention
-// block over 1000 tokens).  Blocks are kept by size class and device and handed out again
-//   - at once, when only the library's own default-stream calls saw them: work on that stream runs in
-//     order, so the block's next writer comes after its last reader;
-//   - after the next synchronisation of the device, when the caller saw the address (`shared`) and may have work
-//     on it in other streams: what hipFree itself would have waited for.  Where none comes, an allocation that
-//     finds kPoolWaitBlocks blocks of its class (or kPoolWaitBytes of them) waiting makes one.
-// At most kPoolBytes are cached in a process; one block more, or an allocation that fails, gives all of them back.
-namespace {
-constexpr size_t kPoolBytes = size_t(4) << 30;
-constexpr size_t kPoolWaitBlocks = 16, kPoolWaitBytes = size_t(256) << 20;
-struct PoolBlock { size_t bytes; int device; unsigned long id; };
-struct PoolWaiting { void* p; unsigned long id; };
-using PoolClass = std::pair<int, size_t>;                            // device, bytes
-std::mutex g_pool_mu;
-unsigned long g_pool_next_id = 0;
-size_t g_pool_cached = 0;
-std::map<void*, PoolBlock> g_pool_live;                              // handed out
-std::map<void*, PoolBlock> g_pool_kept;                              // ready or waiting
-std::map<PoolClass, std::vector<void*>> g_pool_ready;
-std::map<PoolClass, std::vector<PoolWaiting>> g_pool_waiting;
-
-// Eight classes per power of two: at most an eighth of a block is unused.
-size_t pool_class(size_t bytes) {
-  size_t step = 512;
-  while (step * 16 <= bytes) step *= 2;
-  return (bytes + step - 1) / step * step;
-}
-// (the callers of the two functions below hold the lock)
-void pool_forget_all() {
-  g_pool_kept.clear();
-  g_pool_ready.clear();
-  g_pool_waiting.clear();
-  g_pool_cached = 0;
-}
-int pool_give_back_all() {
-  int rc = kOk;
-  for (auto& b : g_pool_kept)
-    if (hipFree(b.first) != hipSuccess) { (void)hipGetLastError(); rc = kDeviceFailed; }
-  pool_forget_all();
-  return rc;
-}
-}  // namespace
-
-// Synchronises the current device; blocks that waited for that when it began are ready afterwards.
-int pool_synchronize() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return kDeviceFailed; }
-  std::vector<PoolWaiting> before;
-  {
-    std::lock_guard<std::mutex> lock(g_pool_mu);
-    for (auto& c : g_pool_waiting)
-      if (c.first.first == dev) before.insert(before.end(), c.second.begin(), c.second.end());
-  }
-  if (hipDeviceSynchronize() != hipSuccess) return kDeviceFailed;
-  if (before.empty()) return kOk;
-  std::lock_guard<std::mutex> lock(g_pool_mu);
-  for (const PoolWaiting& w : before) {
-    auto it = g_pool_kept.find(w.p);
-    if (it == g_pool_kept.end() || it->second.id != w.id) continue;   // given back, or settled by another thread
-    auto& waiting = g_pool_waiting[{dev, it->second.bytes}];
-    auto at = std::find_if(waiting.begin(), waiting.end(), [&](const PoolWaiting& x) { return x.id == w.id; });
-    if (at == waiting.end()) continue;
-    waiting.erase(at);
-    g_pool_ready[{dev, it->second.bytes}].push_back(w.p);
-  }
-  return kOk;
-}
-
-int pool_malloc(void** out, size_t bytes) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return kDeviceFailed; }
-  const size_t size = pool_class(bytes < 512 ? 512 : bytes);
-  const PoolClass cls{dev, size};
-  std::unique_lock<std::mutex> lock(g_pool_mu);
-  if (g_pool_ready[cls].empty()) {
-    const size_t n = g_pool_waiting[cls].size();
-    if (n >= kPoolWaitBlocks || n * size >= kPoolWaitBytes) {
-      lock.unlock();
-      if (int rc = pool_synchronize(); rc != kOk) return rc;
-      lock.lock();
-    }
-  }
-  auto& ready = g_pool_ready[cls];
-  void* p = nullptr;
-  if (!ready.empty()) {
-    p = ready.back();
-    ready.pop_back();
-    g_pool_kept.erase(p);
-    g_pool_cached -= size;
-  } else if (hipMalloc(&p, size) != hipSuccess) {
-    (void)hipGetLastError();
-    (void)pool_give_back_all();
-    if (hipMalloc(&p, size) != hipSuccess) { (void)hipGetLastError(); return kDeviceFailed; }
-  }
-  g_pool_live[p] = PoolBlock{size, dev, ++g_pool_next_id};
-  *out = p;
-  return kOk;
-}
-
-int pool_free(void* p, bool shared) {
-  std::lock_guard<std::mutex> lock(g_pool_mu);
-  auto it = g_pool_live.find(p);
-  if (it == g_pool_live.end()) return kBadShape;
-  const PoolBlock b = it->second;
-  g_pool_live.erase(it);
-  if (b.bytes > kPoolBytes / 2) return finish(hipFree(p));
-  int rc = kOk;
-  if (g_pool_cached + b.bytes > kPoolBytes) rc = pool_give_back_all();
-  g_pool_kept[p] = b;
-  g_pool_cached += b.bytes;
-  if (shared) g_pool_waiting[{b.device, b.bytes}].push_back({p, b.id});
-  else g_pool_ready[{b.device, b.bytes}].push_back(p);
-  return rc;
-}
-
-int pool_trim() {
-  std::lock_guard<std::mutex> lock(g_pool_mu);
-  return pool_give_back_all();
 }
 
 struct Timer {
@@ -272,7 +176,7 @@ int tessera_gfx950_device_cus(int* cus) {
 int tessera_gfx950_malloc(void** dptr, size_t bytes) {
   if (!dptr) return kBadShape;
   if (probe_device() != kOk) return kNoDevice;
-  return finish(hipMalloc(dptr, bytes < 16 ? 16 : bytes));
+  return device_malloc(dptr, bytes < 16 ? 16 : bytes) ? kOk : kDeviceFailed;
 }
 
 int tessera_gfx950_free(void* dptr) {
@@ -284,18 +188,19 @@ int tessera_gfx950_free(void* dptr) {
 int tessera_gfx950_pool_malloc(void** dptr, size_t bytes) {
   if (!dptr) return kBadShape;
   if (probe_device() != kOk) return kNoDevice;
-  return pool_malloc(dptr, bytes);
+  return g_pool.malloc(dptr, bytes) ? kOk : kDeviceFailed;
 }
 
 int tessera_gfx950_pool_free(void* dptr, int shared) {
   if (!dptr) return kOk;
   if (probe_device() != kOk) return kNoDevice;
-  return pool_free(dptr, shared != 0);
+  const PoolStatus r = g_pool.free(dptr, shared != 0);
+  return r == PoolStatus::kOk ? kOk : r == PoolStatus::kForeign ? kBadShape : kDeviceFailed;
 }
 
 int tessera_gfx950_pool_trim(void) {
   if (probe_device() != kOk) return kNoDevice;
-  return pool_trim();
+  return g_pool.trim() ? kOk : kDeviceFailed;
 }
 
 int tessera_gfx950_memcpy_h2d(void* dst, const void* src, size_t bytes) {
@@ -331,7 +236,7 @@ int tessera_gfx950_memcpy_d2d_dev(void* dst, const void* src, size_t bytes, void
 
 int tessera_gfx950_synchronize(void) {
   if (probe_device() != kOk) return kNoDevice;
-  return pool_synchronize();
+  return g_pool.synchronize() ? kOk : kDeviceFailed;
 }
 
 int tessera_gfx950_timer_create(void** timer) {

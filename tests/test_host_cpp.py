@@ -50,3 +50,61 @@ def _few_row_cases():
     cases += [(m, n, k) for m in (1, 2, 9, 32, 33, 64) for n in (8, 9, 1003, 1 << 24, 69_273_000, 69_274_000, 1 << 28)
               for k in (1, 33, 4097, 1 << 24, 17_043_000, 17_044_000, 34_600_000, 1 << 30, 2 ** 31 - 1)]
     return [(m, n, k, k, n) for m, n, k in cases] + [(3, 100, 64, 1 << 29, 104), (3, 100, 64, 64, 1 << 27)]
+
+
+# A device of 100 units, counted, in the place of HIP: `used` units are out, `syncs` synchronisations happened.
+_FAKE_DEVICE = r"""
+#include "device_pool.h"
+#include <cstdio>
+#include <cstdlib>
+using namespace tsr950;
+static const size_t kUnit = size_t(64) << 20;
+static size_t used = 0, syncs = 0;
+static std::map<void*, size_t> out;
+static char* next_address = reinterpret_cast<char*>(4096);
+struct Fake {
+  static bool device(int* d) { *d = 0; return true; }
+  static PoolAlloc malloc(void** p, size_t bytes) {
+    if (used + bytes > 100 * kUnit) return PoolAlloc::kNoMemory;
+    *p = next_address; next_address += bytes; used += bytes; out[*p] = bytes;
+    return PoolAlloc::kOk;
+  }
+  static bool free(void* p) { used -= out.at(p); out.erase(p); return true; }
+  static bool synchronize() { ++syncs; return true; }
+};
+static DevicePool<Fake> pool;
+static void check(bool ok, int line) { if (!ok) { std::printf("line %d\n", line); std::exit(1); } }
+#define CHECK(x) check(x, __LINE__)
+"""
+
+
+def test_pool_gives_its_blocks_to_other_allocations(tmp_path):
+    """A full device: an allocation outside the pool (a stream's workspace, a raw buffer, a stream-ordered temporary)
+    takes what the pool has cached, and fails only where the memory is really out."""
+    out = _run(tmp_path, _FAKE_DEVICE + r"""
+int main() {
+  void *a, *b, *p = nullptr;
+  CHECK(pool.malloc(&a, 20 * kUnit) && pool.malloc(&b, 20 * kUnit));
+  CHECK(pool.free(a, false) == PoolStatus::kOk && pool.free(b, true) == PoolStatus::kOk && used == 40 * kUnit);
+  CHECK(pool.free(a, false) == PoolStatus::kForeign);
+  auto take = [&](size_t units) { return pool.allocate([&] { return Fake::malloc(&p, units * kUnit); }); };
+  CHECK(take(60) && used == 100 * kUnit);                // fits beside the cached blocks: they stay
+  CHECK(take(30) && used == 90 * kUnit);                 // 40 were idle in the pool
+  CHECK(!take(30) && used == 90 * kUnit);                // nothing cached any more
+  CHECK(take(10));
+  CHECK(!pool.malloc(&a, kUnit));
+  int calls = 0;                                         // another error is not answered by a second attempt
+  CHECK(!pool.allocate([&] { ++calls; return PoolAlloc::kFailed; }) && calls == 1);
+  std::printf("ok\n");
+}
+""")
+    assert out == "ok\n"
+
+
+def test_every_device_allocation_can_take_the_pools_blocks():
+    """hipMalloc and hipMallocAsync are called in one place, behind the retry."""
+    for f in sorted(CSRC.glob("*.h")) + sorted(CSRC.glob("*.hip")):
+        for i, line in enumerate(f.read_text().splitlines(), 1):
+            code = line.split("//")[0]
+            if "hipMalloc(" in code or "hipMallocAsync(" in code:
+                assert f.name == "runtime.hip" and "pool_alloc_of(hipMalloc" in code, (f.name, i, line)
