@@ -99,7 +99,8 @@ int tessera_gfx950_free(void* dptr);
 /* Device memory from the library's pool, for results that a chain of default-stream calls allocates and
  * drops; hipMalloc and hipFree cost about 65 us a pair, and hipFree waits for the device.  pool_free takes an
  * address of pool_malloc (else rc 1).  shared == 0: the block was used by work on the default stream only; it may be
- * handed out again at once, and its next user must be on the default stream or ordered behind it.  shared != 0:
+ * handed out again at once, and its next user must be on the default stream or ordered behind it: pool_settle waits
+ * for that (the device, and only where it has not been synchronised since the block was dropped).  shared != 0:
  * it may be in use in other streams; it is handed out again only after the device has been synchronised
  * (tessera_gfx950_synchronize, or by the pool itself once 16 blocks of a size, or 256 MB of them, wait).  The pool
  * caches at most 4 GiB and keeps blocks per device; pool_trim gives everything cached back, and so does any allocation
@@ -107,6 +108,7 @@ int tessera_gfx950_free(void* dptr);
  * No counterpart in the reference, which allocates per call. */
 int tessera_gfx950_pool_malloc(void** dptr, size_t bytes);
 int tessera_gfx950_pool_free(void* dptr, int shared);
+int tessera_gfx950_pool_settle(void* dptr);
 int tessera_gfx950_pool_trim(void);
 int tessera_gfx950_memcpy_h2d(void* dst, const void* src, size_t bytes);
 int tessera_gfx950_memcpy_d2h(void* dst, const void* src, size_t bytes);

@@ -16,7 +16,8 @@ enum class PoolStatus { kOk, kForeign, kFailed };
 // cost about 65 us a pair and the free waits for the device: three of them were half the time of an attention
 // block over 1000 tokens).  Blocks are kept by size class and device and handed out again
 //   - at once, when only the library's own default-stream calls saw them: work on that stream runs in
-//     order, so the block's next writer comes after its last reader;
+//     order, so the block's next writer comes after its last reader.  An owner that wants such a block for other
+//     streams calls `settle` first, which waits for the device where nothing has since the block was dropped;
 //   - after the next synchronisation of the device, when the caller saw the address (`shared`) and may have work
 //     on it in other streams: what hipFree itself would have waited for.  Where none comes, an allocation that
 //     finds kWaitBlocks blocks of its class (or kWaitBytes of them) waiting makes one.
@@ -24,7 +25,7 @@ enum class PoolStatus { kOk, kForeign, kFailed };
 // memory (`allocate`), gives all of them back.
 //
 // Api, static: bool device(int*), the current device; PoolAlloc malloc(void**, size_t); bool free(void*), which waits
-// for the work that uses the block; bool synchronize(), the current device.
+// for the work that uses the block; bool synchronize(int dev).
 template <class Api>
 class DevicePool {
  public:
@@ -47,9 +48,11 @@ class DevicePool {
     }
     auto& ready = ready_[cls];
     void* p = nullptr;
+    unsigned long dropped = 0;
     if (!ready.empty()) {
       p = ready.back();
       ready.pop_back();
+      dropped = kept_[p].dropped;
       kept_.erase(p);
       cached_ -= size;
     } else {
@@ -60,7 +63,7 @@ class DevicePool {
       }
       if (r != PoolAlloc::kOk) return false;
     }
-    live_[p] = Block{size, dev, ++next_id_};
+    live_[p] = Block{size, dev, ++clock_, dropped};
     *out = p;
     return true;
   }
@@ -69,11 +72,12 @@ class DevicePool {
     std::lock_guard<std::mutex> lock(mu_);
     auto it = live_.find(p);
     if (it == live_.end()) return PoolStatus::kForeign;
-    const Block b = it->second;
+    Block b = it->second;
     live_.erase(it);
     if (b.bytes > kBytes / 2) return Api::free(p) ? PoolStatus::kOk : PoolStatus::kFailed;
     bool ok = true;
     if (cached_ + b.bytes > kBytes) ok = give_back_all();
+    b.dropped = ++clock_;
     kept_[p] = b;
     cached_ += b.bytes;
     if (shared) waiting_[{b.device, b.bytes}].push_back({p, b.id});
@@ -81,29 +85,24 @@ class DevicePool {
     return ok ? PoolStatus::kOk : PoolStatus::kFailed;
   }
 
+  // Makes a handed-out block safe for any stream: waits for its device where the block's last owner dropped it
+  // after the latest synchronisation, so that work of that owner may still be queued on it.
+  PoolStatus settle(void* p) {
+    int dev = 0;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      auto it = live_.find(p);
+      if (it == live_.end()) return PoolStatus::kForeign;
+      dev = it->second.device;
+      if (it->second.dropped <= synced_[dev]) return PoolStatus::kOk;
+    }
+    return synchronize(dev) ? PoolStatus::kOk : PoolStatus::kFailed;
+  }
+
   // Synchronises the current device; blocks that waited for that when it began are ready afterwards.
   bool synchronize() {
     int dev = 0;
-    if (!Api::device(&dev)) return false;
-    std::vector<Waiting> before;
-    {
-      std::lock_guard<std::mutex> lock(mu_);
-      for (auto& c : waiting_)
-        if (c.first.first == dev) before.insert(before.end(), c.second.begin(), c.second.end());
-    }
-    if (!Api::synchronize()) return false;
-    if (before.empty()) return true;
-    std::lock_guard<std::mutex> lock(mu_);
-    for (const Waiting& w : before) {
-      auto it = kept_.find(w.p);
-      if (it == kept_.end() || it->second.id != w.id) continue;      // given back, or settled by another thread
-      auto& waiting = waiting_[{dev, it->second.bytes}];
-      auto at = std::find_if(waiting.begin(), waiting.end(), [&](const Waiting& x) { return x.id == w.id; });
-      if (at == waiting.end()) continue;
-      waiting.erase(at);
-      ready_[{dev, it->second.bytes}].push_back(w.p);
-    }
-    return true;
+    return Api::device(&dev) && synchronize(dev);
   }
 
   bool trim() {
@@ -127,9 +126,33 @@ class DevicePool {
   }
 
  private:
-  struct Block { size_t bytes; int device; unsigned long id; };
+  struct Block { size_t bytes; int device; unsigned long id, dropped; };   // dropped: when its last owner did, 0 = none
   struct Waiting { void* p; unsigned long id; };
   using Class = std::pair<int, size_t>;                              // device, bytes
+
+  bool synchronize(int dev) {
+    std::vector<Waiting> before;
+    unsigned long began = 0;
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      began = clock_;
+      for (auto& c : waiting_)
+        if (c.first.first == dev) before.insert(before.end(), c.second.begin(), c.second.end());
+    }
+    if (!Api::synchronize(dev)) return false;
+    std::lock_guard<std::mutex> lock(mu_);
+    synced_[dev] = std::max(synced_[dev], began);
+    for (const Waiting& w : before) {
+      auto it = kept_.find(w.p);
+      if (it == kept_.end() || it->second.id != w.id) continue;      // given back, or settled by another thread
+      auto& waiting = waiting_[{dev, it->second.bytes}];
+      auto at = std::find_if(waiting.begin(), waiting.end(), [&](const Waiting& x) { return x.id == w.id; });
+      if (at == waiting.end()) continue;
+      waiting.erase(at);
+      ready_[{dev, it->second.bytes}].push_back(w.p);
+    }
+    return true;
+  }
 
   // Eight classes per power of two: at most an eighth of a block is unused.
   static size_t size_class(size_t bytes) {
@@ -148,7 +171,8 @@ class DevicePool {
   }
 
   std::mutex mu_;
-  unsigned long next_id_ = 0;
+  unsigned long clock_ = 0;                                          // one tick per hand-out and per drop
+  std::map<int, unsigned long> synced_;                              // device: the tick up to which its work is done
   size_t cached_ = 0;
   std::map<void*, Block> live_;                                      // handed out
   std::map<void*, Block> kept_;                                      // ready or waiting

@@ -52,7 +52,12 @@ struct HipPoolApi {
   static bool device(int* dev) { return ok(hipGetDevice(dev)); }
   static PoolAlloc malloc(void** p, size_t bytes) { return pool_alloc_of(hipMalloc(p, bytes)); }
   static bool free(void* p) { return ok(hipFree(p)); }
-  static bool synchronize() { return hipDeviceSynchronize() == hipSuccess; }
+  static bool synchronize(int dev) {
+    int now = 0;
+    if (!ok(hipGetDevice(&now)) || (now != dev && !ok(hipSetDevice(dev)))) return false;
+    const bool done = hipDeviceSynchronize() == hipSuccess;
+    return (now == dev || ok(hipSetDevice(now))) && done;
+  }
 };
 DevicePool<HipPoolApi> g_pool;
 }  // namespace
@@ -195,6 +200,13 @@ int tessera_gfx950_pool_free(void* dptr, int shared) {
   if (!dptr) return kOk;
   if (probe_device() != kOk) return kNoDevice;
   const PoolStatus r = g_pool.free(dptr, shared != 0);
+  return r == PoolStatus::kOk ? kOk : r == PoolStatus::kForeign ? kBadShape : kDeviceFailed;
+}
+
+int tessera_gfx950_pool_settle(void* dptr) {
+  if (!dptr) return kBadShape;
+  if (probe_device() != kOk) return kNoDevice;
+  const PoolStatus r = g_pool.settle(dptr);
   return r == PoolStatus::kOk ? kOk : r == PoolStatus::kForeign ? kBadShape : kDeviceFailed;
 }
 

@@ -69,6 +69,7 @@ _SIGNATURES = {
     "tessera_gfx950_free": [_c_vp],
     "tessera_gfx950_pool_malloc": [_P(_c_vp), _c_sz],
     "tessera_gfx950_pool_free": [_c_vp, _c_int],
+    "tessera_gfx950_pool_settle": [_c_vp],
     "tessera_gfx950_pool_trim": [],
     "tessera_gfx950_memcpy_h2d": [_c_vp, _c_vp, _c_sz],
     "tessera_gfx950_memcpy_d2h": [_c_vp, _c_vp, _c_sz],
@@ -327,7 +328,9 @@ class PooledBuffer:
     """A device allocation from the library's pool, for results of calls on the default stream.
 
     ``address`` is for such calls.  Reading ``ptr`` marks the buffer as shared: its memory may then be in use in
-    other streams, and is not handed out again before the device has been synchronised."""
+    other streams, and is not handed out again before the device has been synchronised.  The memory may be an earlier
+    result's whose last default-stream work is still queued: other streams use it behind the call that
+    fills it, or after :meth:`settle`."""
 
     __slots__ = ("nbytes", "address", "_shared", "_free", "__weakref__")
 
@@ -345,6 +348,11 @@ class PooledBuffer:
     def ptr(self) -> Optional[int]:
         self._shared = 1
         return self.address
+
+    def settle(self) -> "PooledBuffer":
+        """Waits, where need be, until no earlier owner's work can touch the memory: it may then be used on any stream."""
+        check(load().tessera_gfx950_pool_settle(self.address), "pool_settle")
+        return self
 
     def upload(self, a: np.ndarray) -> None:
         a = np.ascontiguousarray(a)

@@ -47,12 +47,14 @@ class DeviceArray:
         self.shape = tuple(int(d) for d in shape)
         self.dtype = dtype
         self.nbytes = math.prod(self.shape) * _ITEMSIZE[dtype]
-        self.buf = buf if buf is not None else _lane.PooledBuffer(max(self.nbytes, 16))
+        # (an uninitialised array may be filled on any stream: no earlier owner's work may be queued on its memory)
+        self.buf = buf if buf is not None else _lane.PooledBuffer(max(self.nbytes, 16)).settle()
 
     @property
     def ptr(self) -> int:
         """The device address, for other libraries and calls on other streams (a pooled buffer whose address was
-        taken is not reused before the device has been synchronised)."""
+        taken is not reused before the device has been synchronised).  A result of this module is written on the default
+        stream: work on other streams, reads and writes, is ordered behind that."""
         return self.buf.ptr
 
     @property
@@ -92,6 +94,12 @@ class DeviceArray:
         return out
 
 
+def _result(shape, dtype: str) -> DeviceArray:
+    """An array that a call on the default stream is about to fill: memory of a dropped result serves at once."""
+    nbytes = math.prod(shape) * _ITEMSIZE[dtype]
+    return DeviceArray(shape, dtype, _lane.PooledBuffer(max(nbytes, 16)))
+
+
 def synchronize() -> None:
     _lane.synchronize()
 
@@ -118,7 +126,7 @@ def gemm(A: DeviceArray, B: DeviceArray, *, out: str = "storage") -> DeviceArray
     batch = math.prod(lead)
     if B.ndim > 2 and B.shape[:-2] != lead:
         raise ValueError(f"batched gemm: leading dims differ — A {A.shape} @ B {B.shape}")
-    D = DeviceArray(lead + (M, N), "f32" if out == "f32" else st)
+    D = _result(lead + (M, N), "f32" if out == "f32" else st)
     lib = _lane.load()
     if batch == 1:
         name = f"tessera_gfx950_gemm_{st}" + ("" if out == "f32" else f"_{st}") + "_dev"
@@ -172,8 +180,8 @@ def flash_attn(Q: DeviceArray, K: DeviceArray, V: DeviceArray, *, scale: Optiona
     if Hq % Hkv:
         raise ValueError("the number of query heads must be a multiple of the KV heads")
     sc = float(scale) if scale is not None else 1.0 / math.sqrt(D)
-    O = DeviceArray(Q.shape, "f32" if out == "f32" else st)
-    L = DeviceArray((B, Hq, Sq), "f32") if return_lse else None
+    O = _result(Q.shape, "f32" if out == "f32" else st)
+    L = _result((B, Hq, Sq), "f32") if return_lse else None
     _attention_call(st, Q.address, K.address, V.address, O, L, B, Hq, Hkv, Sq, Sk, D, qst + kst + kst + qst, sc, causal, window,
                     logit_softcap, out)
     return (O, L) if return_lse else O
@@ -191,8 +199,8 @@ def flash_attn_fused_qkv(QKV: DeviceArray, num_q_heads: int, num_kv_heads: int, 
     B, S, W = QKV.shape
     D = W // (num_q_heads + 2 * num_kv_heads)
     sc = float(scale) if scale is not None else 1.0 / math.sqrt(D)
-    O = DeviceArray((B, S, num_q_heads, D), "f32" if out == "f32" else st)
-    L = DeviceArray((B, num_q_heads, S), "f32") if return_lse else None
+    O = _result((B, S, num_q_heads, D), "f32" if out == "f32" else st)
+    L = _result((B, num_q_heads, S), "f32") if return_lse else None
     inb, outb = (S * W, D, W), (S * num_q_heads * D, D, num_q_heads * D)
     k_ptr = QKV.address + num_q_heads * D * 2
     v_ptr = k_ptr + num_kv_heads * D * 2
@@ -219,10 +227,10 @@ class ResidentPlan:
     num_slots: DeviceArray
 
     @classmethod
-    def empty(cls, T: int, k: int, E: int) -> "ResidentPlan":
+    def empty(cls, T: int, k: int, E: int, new=DeviceArray) -> "ResidentPlan":
         S = T * k
-        return cls(T, k, E, DeviceArray((S,), "i32"), DeviceArray((S,), "i32"), DeviceArray((S,), "f32"),
-                   DeviceArray((E,), "i32"), DeviceArray((E + 1,), "i32"), DeviceArray((1,), "i32"))
+        return cls(T, k, E, new((S,), "i32"), new((S,), "i32"), new((S,), "f32"),
+                   new((E,), "i32"), new((E + 1,), "i32"), new((1,), "i32"))
 
 
 def route_tokens(scores: DeviceArray, num_experts: int, top_k: int, *, normalize_weights: bool = True,
@@ -231,7 +239,7 @@ def route_tokens(scores: DeviceArray, num_experts: int, top_k: int, *, normalize
     if scores.dtype != "f32" or scores.ndim != 2 or scores.shape[1] != num_experts:
         raise ValueError(f"scores must be f32 (T, {num_experts}); got {scores.dtype} {scores.shape}")
     T = scores.shape[0]
-    plan = ResidentPlan.empty(T, top_k, num_experts)
+    plan = ResidentPlan.empty(T, top_k, num_experts, _result)
     rc = _lane.load().tessera_gfx950_moe_route_f32_dev(
         scores.address, T, num_experts, top_k, 1 if normalize_weights else 0, int(capacity or 0),
         plan.token_of_slot.address, plan.expert_of_slot.address, plan.combine_weights.address, plan.group_sizes.address,
@@ -266,8 +274,8 @@ def moe_layer(x: DeviceArray, W_router: Optional[DeviceArray], W_gate: DeviceArr
     need = ctypes.c_size_t(0)
     _lane.check(lib.tessera_gfx950_moe_layer_workspace_bytes(T, H, F, N, E, top_k, ctypes.byref(need)), "moe_layer")
     ws = _lane.PooledBuffer(need.value)
-    out = DeviceArray((T, N), "f32")
-    plan = ResidentPlan.empty(T, top_k, E)
+    out = _result((T, N), "f32")
+    plan = ResidentPlan.empty(T, top_k, E, _result)
     rc = lib.tessera_gfx950_moe_layer_bf16_dev(
         x.address, W_router.address if W_router is not None else None,
         router_logits.address if router_logits is not None else None, W_gate.address, W_up.address, W_down.address, out.address,

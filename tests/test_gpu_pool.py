@@ -1,4 +1,5 @@
 """The library's memory pool under the resident handles."""
+import ctypes
 import threading
 
 import numpy as np
@@ -39,6 +40,36 @@ def test_shared_blocks_wait_for_a_synchronisation(lane):
         seen.add(x.ptr)
         x.close()
     assert len(seen) <= 17
+
+
+def test_uninitialised_arrays_are_free_of_earlier_work(lane):
+    """A new DeviceArray may be written on a stream that nothing orders behind the default one: the products that its memory's
+    last owner has queued must not read or overwrite what is written there."""
+    hip = ctypes.CDLL("libamdhip64.so", mode=ctypes.RTLD_LOCAL)
+    p = ctypes.c_void_p
+    hip.hipStreamCreateWithFlags.argtypes = [ctypes.POINTER(p), ctypes.c_uint]
+    hip.hipStreamSynchronize.argtypes = hip.hipStreamDestroy.argtypes = [p]
+    copy = lane.load().tessera_gfx950_memcpy_d2d_dev
+    rng = np.random.default_rng(5)
+    n = 4096
+    x, w = (rs.DeviceArray.from_host(b16.from_float32((rng.standard_normal((n, n)) / 8).astype(np.float32))) for _ in range(2))
+    mine = rs.DeviceArray.from_host(b16.from_float32(np.full((n, n), 3.0, np.float32)))
+    want = np.asarray(rs.gemm(rs.gemm(x, w), w).to_host()).view(np.uint16).copy()
+    s = p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0          # non-blocking: no order with the default stream
+    try:
+        for _ in range(10):
+            h = rs.gemm(x, w)
+            y = rs.gemm(h, w)
+            del h
+            z = rs.DeviceArray((n, n), "bf16")
+            lane.check(copy(z.ptr, mine.ptr, z.nbytes, s), "copy")
+            assert hip.hipStreamSynchronize(s) == 0
+            assert np.array_equal(np.asarray(y.to_host()).view(np.uint16), want)
+            assert np.all(z.to_host().to_float32() == 3.0)
+            del y, z
+    finally:
+        hip.hipStreamDestroy(s)
 
 
 def test_pool_free_rejects_foreign_addresses(lane):

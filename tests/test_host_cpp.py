@@ -70,7 +70,7 @@ struct Fake {
     return PoolAlloc::kOk;
   }
   static bool free(void* p) { used -= out.at(p); out.erase(p); return true; }
-  static bool synchronize() { ++syncs; return true; }
+  static bool synchronize(int dev) { ++syncs; return dev == 0; }
 };
 static DevicePool<Fake> pool;
 static void check(bool ok, int line) { if (!ok) { std::printf("line %d\n", line); std::exit(1); } }
@@ -95,6 +95,27 @@ int main() {
   CHECK(!pool.malloc(&a, kUnit));
   int calls = 0;                                         // another error is not answered by a second attempt
   CHECK(!pool.allocate([&] { ++calls; return PoolAlloc::kFailed; }) && calls == 1);
+  std::printf("ok\n");
+}
+""")
+    assert out == "ok\n"
+
+
+def test_pool_blocks_settle_behind_their_last_owner(tmp_path):
+    """A block handed out again at once has its last owner's work queued on it: `settle` waits for the device then, and
+    only then."""
+    out = _run(tmp_path, _FAKE_DEVICE + r"""
+int main() {
+  void *a, *b, *c;
+  CHECK(pool.malloc(&a, kUnit) && pool.settle(a) == PoolStatus::kOk && syncs == 0);          // fresh memory
+  CHECK(pool.free(a, false) == PoolStatus::kOk && pool.settle(a) == PoolStatus::kForeign);
+  CHECK(pool.malloc(&b, kUnit) && b == a && syncs == 0);                                     // reused at once
+  CHECK(pool.settle(b) == PoolStatus::kOk && syncs == 1);
+  CHECK(pool.settle(b) == PoolStatus::kOk && syncs == 1);                                    // nothing queued since
+  CHECK(pool.free(b, false) == PoolStatus::kOk && pool.synchronize() && syncs == 2);
+  CHECK(pool.malloc(&a, kUnit) && a == b && pool.settle(a) == PoolStatus::kOk && syncs == 2); // dropped before the wait
+  CHECK(pool.free(a, true) == PoolStatus::kOk && pool.malloc(&c, kUnit) && c != a && pool.synchronize());
+  CHECK(pool.malloc(&b, kUnit) && b == a && pool.settle(b) == PoolStatus::kOk && syncs == 3); // shared: settled by that
   std::printf("ok\n");
 }
 """)
