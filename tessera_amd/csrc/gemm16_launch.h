@@ -373,8 +373,11 @@ int launch_gemm16_skinny(Gemm16Params p, int splits, bool loose, hipStream_t s) 
   }
   const bool nt = 2.0 * p.K * p.N >= kStreamOnceBytes;
   int rc;
+  // (loose: off the 128-byte grid a row's piece lies in two cache lines and neighbouring strips want the same line, and
+  // eight waves with a workgroup's whole K range in flight read at half the rate.  16 rows, eight / four waves / copies
+  // into aligned buffers: N 8191 x K 4097 64 / 35 / 67 us, 14335 x 2049 56 / 30 / 49, 12001 x 12003 149 / 99 / 253)
   if (loose)
-    rc = p.M <= 32 ? launch_gemm16_skinny_as<T, 1, 8, 4, EPI, false, true>(q, kps, splits, part, d_vec, s)
+    rc = p.M <= 32 ? launch_gemm16_skinny_as<T, 1, 4, 4, EPI, false, true>(q, kps, splits, part, d_vec, s)
                    : launch_gemm16_skinny_as<T, 2, 4, 4, EPI, false, true>(q, kps, splits, part, d_vec, s);
   else if (cols == 64)
     rc = nt ? launch_gemm16_skinny_as<T, 1, 8, 2, EPI, true, false>(q, kps, splits, part, d_vec, s)

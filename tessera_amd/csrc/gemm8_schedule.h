@@ -60,13 +60,19 @@ inline double est_gemm8_fit_us(int kind, int M, int N, int K, int splits) {
   return f.launch + std::max(compute, stream) + sum;
 }
 
+// Waves in a workgroup of the streaming kernel: 8 up to 32 rows, 4 above (twice the accumulators).  loose: four up to 32
+// rows, too.  Off the 128-byte grid a row's piece lies in two cache lines and neighbouring strips want the same line, and eight
+// waves with a workgroup's whole K range in flight read at half the rate (16 rows, N 8191 x K 4097: 65 us with
+// eight, 28 with four, 47 by copies into aligned buffers; 14335 x 2049 79, 35 and 41).  Up to one slice for each of
+// eight waves (K 512), eight: 16 x 1003 x 259 9.8 against 11.3.
+inline int gemm8_skinny_waves(int M, int K, bool loose) { return M <= 32 && (!loose || K <= 512) ? 8 : 4; }
+
 // K splits of the streaming kernel: never over one workgroup per compute unit (the second round would be
-// nearly empty), at least one 64-row slice for each of its waves (8 waves up to 32 rows, 4 above: twice the
-// accumulators), and within that the fewest microseconds by an estimate: a workgroup streams a 128-byte row
-// in 3.75 ns, the chip 5.6 TB/s; a split adds a launch and a sum, 3.6 us.
-inline int gemm8_skinny_splits(int M, int N, int K) {
+// nearly empty), at least one 64-row slice for each of its waves, and within that the fewest microseconds by an
+// estimate: a workgroup streams a 128-byte row in 3.75 ns, the chip 5.6 TB/s; a split adds a launch and a sum, 3.6 us.
+inline int gemm8_skinny_splits(int waves, int N, int K) {
   const int strips = (N + 127) / 128;
-  const int most = std::max(1, std::min(256 / strips, K / ((M <= 32 ? 8 : 4) * 64)));
+  const int most = std::max(1, std::min(256 / strips, K / (waves * 64)));
   int best = 1;
   double best_us = 1e30;
   for (int splits = 1; splits <= most; ++splits) {
@@ -84,7 +90,7 @@ inline Gemm8Schedule select_gemm8_rule(int M, int N, int K) {
   // At most 64 rows (quantised decode): the streaming kernel.  (Below 1024 rows of B the tiles are as good:
   // 48 x 4096 x 512 10.2 us against 12.3.)
   if (M <= kGemm8SkinnyMaxM && K % 16 == 0 && K >= 1024) {
-    const int kps = (int)cdiv(cdiv(K, gemm8_skinny_splits(M, N, K)), 64) * 64;
+    const int kps = (int)cdiv(cdiv(K, gemm8_skinny_splits(gemm8_skinny_waves(M, K, false), N, K)), 64) * 64;
     return {M <= 32 ? 32 : 64, 128, 64, (int)cdiv(K, kps), true};
   }
   // Tile rows (256 or 128) and K slices by estimated time.  Few tiles and a long K (few rows against a

@@ -108,22 +108,24 @@ inline bool gemm8_worth_copies(int M, int N, int K) {
 template <class T, int EPI>
 int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
   constexpr bool FP8 = !std::is_same<T, I8>::value;
-  const bool one = p.M <= 32;
-  const int nw = one ? 8 : 4;
+  const int nw = gemm8_skinny_waves(p.M, p.K, loose);
+  const int blocks = p.M <= 32 ? (nw == 8 ? 0 : 1) : 2;                 // 8 waves, 4 waves, 4 waves with two row blocks
   const int form = !loose ? 0 : FP8 && !gemm8_worth_copies(p.M, p.N, p.K) ? 2 : 1;
   using Kernel = void (*)(const Gemm8Params, int, int, void*, int);
-  static const Kernel kernels[2][3] = {{gemm8_skinny_kernel<T, 4, 2, EPI, false, false>, gemm8_skinny_kernel<T, 4, 2, EPI, true, false>,
-                                        gemm8_skinny_kernel<T, 4, 2, EPI, true, FP8>},
-                                       {gemm8_skinny_kernel<T, 8, 1, EPI, false, false>, gemm8_skinny_kernel<T, 8, 1, EPI, true, false>,
-                                        gemm8_skinny_kernel<T, 8, 1, EPI, true, FP8>}};
+  static const Kernel kernels[3][3] = {{gemm8_skinny_kernel<T, 8, 1, EPI, false, false>, gemm8_skinny_kernel<T, 8, 1, EPI, true, false>,
+                                        gemm8_skinny_kernel<T, 8, 1, EPI, true, FP8>},
+                                       {nullptr, gemm8_skinny_kernel<T, 4, 1, EPI, true, false>,
+                                        gemm8_skinny_kernel<T, 4, 1, EPI, true, FP8>},
+                                       {gemm8_skinny_kernel<T, 4, 2, EPI, false, false>, gemm8_skinny_kernel<T, 4, 2, EPI, true, false>,
+                                        gemm8_skinny_kernel<T, 4, 2, EPI, true, FP8>}};
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
-    for (int o = 0; o < 2; ++o)
+    for (int o = 0; o < 3; ++o)
       for (Kernel k : kernels[o])
-        if (attr_err == hipSuccess)
+        if (k && attr_err == hipSuccess)
           attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         g8s_smem(o ? 8 : 4, 32));
+                                         g8s_smem(o ? 4 : 8, 32));
   });
   if (attr_err != hipSuccess) return kDeviceFailed;
   const int strips = ceil_div(p.N, G8S_COLS);
@@ -151,7 +153,7 @@ int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
   }
   void* part = splits > 1 ? ws + a_bytes : nullptr;
   const int vec = p.N % 4 == 0 && aligned16(p.D) && (!p.acc_out || aligned16(p.acc_out)) && (!p.col_scale || aligned16(p.col_scale));
-  hipLaunchKernelGGL(kernels[one][form], dim3(strips, splits), dim3(nw * 64), g8s_smem(nw, std::min(p.M, 32)), s, q, lda, kps, part,
+  hipLaunchKernelGGL(kernels[blocks][form], dim3(strips, splits), dim3(nw * 64), g8s_smem(nw, std::min(p.M, 32)), s, q, lda, kps, part,
                      vec);
   if (int rc = launch_status(); rc != kOk || !part) return rc;
   return launch_gemm8_split_sum<T, EPI>(part, splits, ldw, vec, p, s);
@@ -168,7 +170,7 @@ int gemm8_dev(Gemm8Params p, hipStream_t s) {
   if (!vec) {
     // few rows: the streaming kernel reads B where it lies
     if (p.M <= kGemm8SkinnyMaxM && p.N >= 16 && p.N < (1 << 25) && p.K < (1 << 24)) {
-      const int rc = gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(p.M, p.N, p.K), true, s);
+      const int rc = gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(gemm8_skinny_waves(p.M, p.K, true), p.N, p.K), true, s);
       if (rc != kNoScratch) return rc;
     }
     if (gemm8_worth_copies(p.M, p.N, p.K)) return gemm8_repitched<T, EPI>(p, s);

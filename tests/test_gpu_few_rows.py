@@ -51,6 +51,18 @@ def test_few_rows_8bit(lane, M, N, K):
     assert orc.max_rel_err(ops.gemm_fp8(codes_a, codes_b, sa, sb, out="f32"), orc.gemm_e4m3(codes_a, codes_b, sa, sb)) <= 2e-3
 
 
+# up to 32 rows off the 16-byte grid: one slice of K for each of eight waves (8-bit: K 512) and beyond, whole, last and
+# missing slices of four waves, unsplit and split K
+@pytest.mark.parametrize("M,N,K", [(16, 1003, 512), (16, 1003, 513), (32, 2055, 577), (9, 141, 1025), (31, 4099, 1301), (24, 131, 4100)])
+def test_few_rows_off_the_grid_in_four_waves(lane, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.integers(-127, 128, (M, K)).astype(np.int8), rng.integers(-127, 128, (K, N)).astype(np.int8)
+    assert np.array_equal(ops.gemm_i8(a, b), orc.gemm_i8_i32(a, b))
+    A, B = rng.standard_normal((M, K)).astype(np.float32), (rng.standard_normal((K, N)) / np.sqrt(K)).astype(np.float32)
+    got = ops.gemm(b16.from_float32(A), b16.from_float32(B), out="f32")
+    assert orc.max_rel_err(got, orc.gemm_f64(A, B, "bf16")) <= 1e-5      # f32 sums of up to 4100 products
+
+
 # fp8 off the 16-byte grid, below 2^24 multiply-adds or under 16 rows (one and two row blocks, split and unsplit K)
 @pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
 @pytest.mark.parametrize("M,N,K", [(1, 17, 203), (5, 130, 201), (15, 1003, 2111), (33, 33, 203), (64, 1003, 259)])
