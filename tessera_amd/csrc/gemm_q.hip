@@ -170,7 +170,7 @@ int gemm8_dev(Gemm8Params p, hipStream_t s) {
   if (!vec) {
     // few rows: the streaming kernel reads B where it lies
     if (p.M <= kGemm8SkinnyMaxM && p.N >= 16 && p.N < (1 << 25) && p.K < (1 << 24)) {
-      const int rc = gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(gemm8_skinny_waves(p.M, p.K, true), p.N, p.K), true, s);
+      const int rc = gemm8_skinny<T, EPI>(p, gemm8_skinny_splits(gemm8_skinny_waves(p.M, p.K, true), p.M, p.N, p.K), true, s);
       if (rc != kNoScratch) return rc;
     }
     if (gemm8_worth_copies(p.M, p.N, p.K)) return gemm8_repitched<T, EPI>(p, s);

@@ -52,6 +52,35 @@ def _few_row_cases():
     return [(m, n, k, k, n) for m, n, k in cases] + [(3, 100, 64, 1 << 29, 104), (3, 100, 64, 64, 1 << 27)]
 
 
+def test_8bit_streaming_splits_count_their_partials(tmp_path):
+    """K splits of the 8-bit streaming kernel at shapes whose forced splits were timed (11.8 us in 16 parts against 14.2 in
+    32, and so on): within a few per cent of the best, never past one workgroup per compute unit or one slice a wave."""
+    timed = {(64, 1024, 8192): (12, 16), (48, 512, 14336): (16, 32), (32, 2048, 8192): (8, 12), (64, 2048, 4096): (6, 8),
+             (48, 1280, 5120): (8, 16), (16, 8192, 8192): (4, 4), (32, 4096, 14336): (8, 8), (16, 3072, 8192): (8, 10),
+             (64, 8192, 8192): (4, 4), (16, 14336, 4096): (1, 2), (32, 8192, 2048): (1, 3)}
+    tiled = [(16, 128256, 2048), (32, 128256, 2048)]         # timed 7 to 11 % below the streaming kernel
+    timed |= {(64, 28672, 4096): (1, 1), (48, 4096, 4096): (4, 8)}
+    many = [(m, n, k) for m in (1, 32, 33, 64) for n in (16, 129, 4096, 33000, 1 << 24) for k in (16, 63, 1024, 8193, 1 << 23)]
+    out = _run(tmp_path, r"""
+#include "gemm8_schedule.h"
+#include <cstdio>
+#include <cstdlib>
+int main(int argc, char** argv) {
+  for (int i = 1; i + 2 < argc; i += 3) {
+    const int M = atoi(argv[i]), N = atoi(argv[i + 1]), K = atoi(argv[i + 2]), w = tsr950::gemm8_skinny_waves(M, K, false);
+    std::printf("%d %d %d\n", tsr950::gemm8_skinny_splits(w, M, N, K), w, tsr950::select_gemm8_schedule(M, N, K).skinny);
+  }
+}
+""", *[x for c in [*timed, *tiled, *many] for x in c])
+    got = [tuple(map(int, line.split())) for line in out.splitlines()]
+    for (shape, (low, high)), (splits, _, skinny) in zip(timed.items(), got):
+        assert low <= splits <= high and skinny, (shape, splits)
+    assert not any(skinny for _, _, skinny in got[len(timed):len(timed) + len(tiled)])
+    for (m, n, k), (splits, waves, _) in zip(many, got[len(timed) + len(tiled):]):
+        strips = -(-n // 128)
+        assert waves == (8 if m <= 32 else 4) and 1 <= splits and (splits == 1 or (splits * strips <= 256 and splits * waves * 64 <= k))
+
+
 # A device of 100 units, counted, in the place of HIP: `used` units are out, `syncs` synchronisations happened.
 _FAKE_DEVICE = r"""
 #include "device_pool.h"
