@@ -643,10 +643,11 @@ int launch_gemm16_grouped(Gemm16Params p, hipStream_t s) {
   // groups that average at most a tile of rows (a chunk of a thousand tokens over 64 experts): the
   // instantiation whose last row tile also comes in a 128-row form
   const bool mid = (long)p.M <= 256L * p.groups;
-  // Weights that outgrow the memory-side cache are streamed past it: each panel is read by one row tile, or by
-  // a few running side by side on one XCD, whose L2 still serves them (64 experts of 4096 x 1408, the
-  // whole layer: 8 tokens 285 -> 256 us, 64 408 -> 378, 512 447 -> 423, 1024 539 -> 524, 1900 660 -> 654).
-  const bool nt = (long)p.M <= 256L * p.groups &&
+  // Weights that outgrow the memory-side cache are streamed past it while their panels are read by one row tile: groups
+  // that average at most 240 rows.  Closer to the tile's 256 half of the groups have a second tile, whose reads then miss (the
+  // whole layer with the hint / without: 64 experts of 4096 x 1408, 64 tokens 357 / 393 us, 1024 500 / 520, 1840, 230 rows a
+  // group, 576 / 613, 2048, 256 rows, 793 / 756; 8 experts of 4096 x 4096, 920 tokens 236 / 239, 1024 318 / 295).
+  const bool nt = (long)p.M <= 240L * p.groups &&
                   (EPI == EPI_SWIGLU16 ? 4.0 : 2.0) * p.K * p.N * p.groups >= kStreamOnceBytes;
   if constexpr (EPI == EPI_SWIGLU16) {
     if (mid && nt) return launch_gemm16_tile<T, 256, 256, 2, 2, EPI, true, kGroupedTileMfma, true, true>(p, s);
