@@ -57,7 +57,7 @@
  * combine and quantiser calls.  Two kinds use it where it is there and take a path without it
  * inside a capture on a stream that has none: single products of up to 64 rows whose N, K or pointers are off the
  * 16-byte grid, and attention of few query rows at head dimensions other than 64, 128 and 256 with 192 and
- * more (batch, head) pairs.  Any entry point (tessera_gfx950_probe is the cheapest) must have
+ * more (batch, head) pairs or under 1024 keys.  Any entry point (tessera_gfx950_probe is the cheapest) must have
  * been called once before the first capture: the first call initialises the device.
  */
 #ifndef TESSERA_GFX950_H

@@ -2,6 +2,7 @@
 #include <cmath>
 #include <mutex>
 #include "../../include/tessera_gfx950.h"
+#include "attn_rules.h"
 #include "flash_attn.h"
 #include "flash_decode.h"
 #include "flash_bwd.h"
@@ -149,7 +150,7 @@ int launch_flash_for(const FlashParams& p, bool ext, hipStream_t s) {
 // Few query rows per KV head (decode, short speculative steps): the rows of a whole GQA group
 // share one MFMA tile and the key range is split over workgroups (flash_decode.h).  kNoScratch: padded head
 // dimensions, whose key splits found no workspace (a capture on a stream that has none); the general
-// kernel then serves them, whose launches of 192 and more blocks need none.
+// kernel then serves them, which needs none from 192 blocks on and under 1024 keys.
 template <class T, int DP, int NQ, bool PAD, bool NT>
 int launch_decode_as(const FlashParams& p, hipStream_t s) {
   using G = DecodeGeom<DP>;
@@ -170,9 +171,9 @@ int launch_decode_as(const FlashParams& p, hipStream_t s) {
   dp.tile_lo = lo0 / G::BK;
   dp.tile_end = hi1 / G::BK + 1;
   const int tiles = dp.tile_end - dp.tile_lo;
-  // about two workgroups per compute unit, and at least two tiles for every wave of a split
+  // about two workgroups per compute unit, and at least two tiles for every wave of a split; see pad_splits
   const int kvheads = p.B * p.Hkv;
-  int nsplit = std::max(1, std::min(ceil_div(512, kvheads), tiles / (2 * G::WAVES)));
+  int nsplit = PAD ? pad_splits(DP, kvheads, tiles, G::WAVES) : std::max(1, std::min(ceil_div(512, kvheads), tiles / (2 * G::WAVES)));
   dp.tiles_per_split = ceil_div(ceil_div(tiles, nsplit), G::WAVES) * G::WAVES;
   nsplit = ceil_div(tiles, dp.tiles_per_split);
   if (nsplit > 1) {
@@ -206,6 +207,7 @@ inline bool decode_shaped(const FlashParams& p) {
   // beyond one query tile the gain is the shared read of K and V by the group's heads (measured: up to
   // 6x with 8 heads a group, a tie or a loss with one)
   if (rows > 32 && p.ratio == 1) return false;
+  if (p.ratio == 1 && pad_general(p.B * p.Hkv, p.Sk, p.D)) return false;
   int lo0, hi0, lo1, hi1;
   key_bounds(0, p.Sq, p.Sk, p.causal, p.window, lo0, hi0);
   key_bounds(p.Sq - 1, p.Sq, p.Sk, p.causal, p.window, lo1, hi1);

@@ -64,6 +64,7 @@ CASES = {
     "int8_on_the_grid": lambda lane, rng: _gemm8(lane, rng, 16, 512, 1024, False),
     "fp8_split": lambda lane, rng: _gemm8(lane, rng, 5, 131, 1024, True),
     "decode_padded": lambda lane, rng: _attention(lane, rng, 24, 8, 8, 1, 1500, 80),
+    "decode_padded_split": lambda lane, rng: _attention(lane, rng, 4, 8, 8, 1, 900, 80),
 }
 
 

@@ -28,6 +28,17 @@ def test_decode_padded_head_dims(lane, D, B, Hq, Hkv, Sq, Sk, causal):
     assert orc.max_rel_err(o, ro) <= TOL and np.max(np.abs(lse - rl)) <= TOL
 
 
+# padded head dimensions with as many KV heads as compute units and more: unsplit, two and more rounds, the general kernel
+@pytest.mark.parametrize("B,Hq,Hkv,Sk,D", [(32, 8, 8, 513, 80), (37, 8, 8, 300, 96), (33, 8, 8, 1030, 80), (33, 16, 8, 300, 112),
+                                           (20, 8, 8, 700, 48), (96, 8, 8, 70, 80)])
+def test_decode_padded_many_heads(lane, B, Hq, Hkv, Sk, D):
+    rng = np.random.default_rng(B + D)
+    q, k, v = _bf(rng, (B, Hq, 1, D)), _bf(rng, (B, Hkv, Sk, D)), _bf(rng, (B, Hkv, Sk, D))
+    o, lse = ops.gqa_attention(q, k, v, return_lse=True, out="f32")
+    ro, rl = orc.flash_attn_dense(q.to_float32(), k.to_float32(), v.to_float32())
+    assert orc.max_rel_err(o, ro) <= TOL and np.max(np.abs(lse - rl)) <= TOL
+
+
 def test_decode_large_cache(lane):
     B, H, Sk, D = 13, 8, 2051, 128                            # 109 MB of K and V
     rng = np.random.default_rng(1)

@@ -81,6 +81,28 @@ int main(int argc, char** argv) {
         assert waves == (8 if m <= 32 else 4) and 1 <= splits and (splits == 1 or (splits * strips <= 256 and splits * waves * 64 <= k))
 
 
+def test_padded_decode_fills_whole_rounds(tmp_path):
+    """Key splits and route of decode at padded head dimensions, at shapes timed both ways: one workgroup per compute unit
+    at DP 128 and 256, two at 64."""
+    splits = {(128, 256, 500): 1, (128, 192, 1000): 1, (128, 64, 2048): 4, (128, 128, 2048): 2, (64, 256, 500): 1, (64, 256, 4096): 2,
+              (128, 512, 4096): 1, (256, 256, 250): 1, (256, 64, 300): 2, (128, 8, 64): 1}
+    general = {(256, 500, 80): 0, (257, 500, 80): 1, (512, 64, 96): 1, (512, 1024, 80): 0, (768, 500, 80): 0, (1024, 250, 112): 1,
+               (512, 500, 48): 0, (512, 500, 64): 0, (512, 500, 128): 0, (512, 500, 160): 0}
+    out = _run(tmp_path, r"""
+#include "attn_rules.h"
+#include <cstdio>
+#include <cstdlib>
+int main(int argc, char** argv) {
+  for (int i = 2; i + 2 < argc; i += 3) {
+    const int a = atoi(argv[i]), b = atoi(argv[i + 1]), c = atoi(argv[i + 2]);
+    std::printf("%d\n", i < 2 + 3 * atoi(argv[1]) ? tsr950::pad_splits(a, b, (c + 31) / 32, a == 256 ? 2 : 4) : (int)tsr950::pad_general(a, b, c));
+  }
+}
+""", len(splits), *[x for c in [*splits, *general] for x in c])
+    got = dict(zip([*splits, *general], map(int, out.split())))
+    assert got == {**splits, **general}
+
+
 # A device of 100 units, counted, in the place of HIP: `used` units are out, `syncs` synchronisations happened.
 _FAKE_DEVICE = r"""
 #include "device_pool.h"
