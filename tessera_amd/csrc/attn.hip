@@ -34,7 +34,7 @@ int launch_flash_as(const FlashParams& p, int nsplit, hipStream_t s) {
   // heads and query blocks of the grid (the kernel's "Work order")
   auto grid_of = [&](int blocks) {
     const int groups = p.B * p.Hkv / 8;
-    return !xcd_grouped ? dim3(p.B * p.Hq, blocks, 1) : W == 4 ? dim3(8 * p.ratio, groups, blocks) : dim3(8 * p.ratio, blocks, groups);
+    return !xcd_grouped ? dim3(p.B * p.Hq, blocks, 1) : p.blocks_last ? dim3(8 * p.ratio, groups, blocks) : dim3(8 * p.ratio, blocks, groups);
   };
   const int tiles = ceil_div(p.Sk, FA_BKV);
   // Key splits: the key tiles are shared by nsplit workgroups, each of which writes a normalised partial O and
@@ -60,75 +60,24 @@ int launch_flash_as(const FlashParams& p, int nsplit, hipStream_t s) {
   return launch_status();
 }
 
-// Key splits of 8-wave workgroups of `rows` query rows: few workgroups against a long key range (a chunk of queries
-// against a long context) get about two workgroups per compute unit, at least 8 tiles (512 keys) a split.
-inline int split8(const FlashParams& p, int rows) {
-  const long wgs = (long)p.B * p.Hq * ceil_div(p.Sq, rows);
-  if (wgs >= 192 || p.bias) return 1;
-  return (int)std::max<long>(1, std::min<long>(std::min<long>(ceil_div(512, (int)wgs), ceil_div(p.Sk, FA_BKV) / 8), 64));
-}
-
-// Workgroup size and key splits of the plain kernel at DP <= 128.
-struct FlashShape { int waves, nsplit; };
-
-// Estimated in steps of a 256-row workgroup (a tile of 64 keys; 4 more for its start and end):
-//   8 waves (256 rows): one workgroup per compute unit, the longest walk or the work over 256 units;
-//   4 waves (128 rows): a step is 1.1 with a second workgroup on the unit (K and V tiles are loaded twice),
-//   0.7 without; a key split shares each walk and costs a merge launch, 6 steps.
-// What it weighs: 128 rows waste less on ragged lengths and spread short or few sequences over more units, 256
-// rows read K and V half as often.  Measured, 8 waves against 4 (bf16, D 128, Hq 32, Hkv 8, causal): B 2 x S 500
-// 23.0 -> 19.1 us, B 1 x S 1000 37.3 (two splits) -> 28.0 (none), B 1 x S 2048 61.6 -> 54.9, B 9 x S 384 45.5 -> 37.1,
-// 512 rows on 4096 keys 60.4 (8 splits) -> 50.8 (4); but B 1 x S 4096 149 -> 162, and the same at more rows, which
-// stay on 8 waves.
-inline FlashShape flash_shape(const FlashParams& p) {
-  const long heads = (long)p.B * p.Hq;
-  if (p.Sq > 8192 || heads * p.Sq > (1L << 22)) return {8, split8(p, 256)};
-  struct Walks { double longest, shortest, total; };
-  auto walks = [&](int rows) {
-    Walks w{0, 1e30, 0};
-    for (int q0 = 0; q0 < p.Sq; q0 += rows) {
-      int lo0, hi0, lo1, hi1;
-      key_bounds(q0, p.Sq, p.Sk, p.causal, p.window, lo0, hi0);
-      key_bounds(std::min(q0 + rows, p.Sq) - 1, p.Sq, p.Sk, p.causal, p.window, lo1, hi1);
-      const double n = std::max((hi1 + FA_BKV) / FA_BKV - lo0 / FA_BKV, 0);
-      w.longest = std::max(w.longest, n);
-      w.shortest = std::min(w.shortest, n);
-      w.total += n * heads;
-    }
-    return w;
-  };
-  const double ends = 4.0;
-  const long n8 = heads * ceil_div(p.Sq, 256), n4 = heads * ceil_div(p.Sq, 128);
-  const Walks w8 = walks(256), w4 = walks(128);
-  // (one block of at most 128 rows keeps half of eight waves busy; heads that no XCD owns share no L2, and the
-  // second read of K and V then costs more: B 13 x Hq 32 x Hkv 4 x S 591 101 -> 106 us)
-  const double t8 = n8 <= 256 ? (p.Sq <= 128 ? 0.68 : 1.0) * (w8.longest + ends)
-                              : std::max(w8.longest + ends, (w8.total + n8 * ends) / 256 + 0.5 * (w8.shortest + ends));
-  auto t4 = [&](int n) {
-    const double longest = w4.longest / n + ends, shortest = w4.shortest / n + ends, merge = n > 1 ? 6.0 : 0.0;
-    if (n4 * n <= 256) return 0.7 * longest + merge;
-    if (n4 * n <= 512) return 1.1 * shortest + 0.7 * (longest - shortest) + merge;
-    return (p.B * p.Hkv % 8 ? 1.35 : 1.1) * std::max(longest, (w4.total + n4 * n * ends) / 512 + 0.5 * shortest) + merge;
-  };
-  int best = 1;
-  // (from 192 blocks on never: a split takes the stream's workspace, which a captured call must find allocated)
-  const int most = n8 >= 192 ? 1 : (int)std::min<long>(std::min<long>(std::max<long>(512 / n4, 1), ceil_div(p.Sk, FA_BKV) / 8), 64);
-  for (int n = 2; n <= most; ++n)
-    if (t4(n) < t4(best)) best = n;
-  // (splits of short walks that put two workgroups on a unit are no better than 8 waves and theirs: B 1 x Hq 8 x
-  // Hkv 8 x S 2048 36.8 us against 35.4)
-  if (best > 1 && n4 * best > 256 && w4.longest < 48) return {8, split8(p, 256)};
-  return 1.03 * t4(best) < t8 ? FlashShape{4, best} : FlashShape{8, split8(p, 256)};
-}
-
 template <class T, int DP, bool EXT, bool PAD>
 int launch_flash(const FlashParams& p, hipStream_t s) {
+  const FlashProblem problem{p.B, p.Hq, p.Hkv, p.Sq, p.Sk, p.D, p.bias != nullptr};
   if constexpr (DP <= 128 && !EXT) {
-    const FlashShape f = flash_shape(p);
-    return f.waves == 4 ? launch_flash_as<T, DP, EXT, PAD, 4>(p, f.nsplit, s)
-                        : launch_flash_as<T, DP, EXT, PAD, 8>(p, f.nsplit, s);
+    const FlashShape f = flash_shape(problem, [&](int q0, int rows) {
+      int lo0, hi0, lo1, hi1;
+      key_bounds(q0, p.Sq, p.Sk, p.causal, p.window, lo0, hi0);
+      key_bounds(q0 + rows - 1, p.Sq, p.Sk, p.causal, p.window, lo1, hi1);
+      return std::max((hi1 + FA_BKV) / FA_BKV - lo0 / FA_BKV, 0);
+    });
+    if (f.waves == 4) {
+      FlashParams q = p;
+      q.blocks_last = flash_blocks_last(problem) && (p.B * p.Hkv) % 8 == 0;
+      return launch_flash_as<T, DP, EXT, PAD, 4>(q, f.nsplit, s);
+    }
+    return launch_flash_as<T, DP, EXT, PAD, 8>(p, f.nsplit, s);
   } else {
-    return launch_flash_as<T, DP, EXT, PAD, 8>(p, split8(p, FlashGeom<DP>::BQ), s);
+    return launch_flash_as<T, DP, EXT, PAD, 8>(p, split8(problem, FlashGeom<DP>::BQ), s);
   }
 }
 

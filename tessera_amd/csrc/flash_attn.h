@@ -65,13 +65,14 @@ struct FlashParams {
   float softcap;       // > 0: scaled scores pass through cap * tanh(s / cap); 0: none
   int ratio;           // Hq / Hkv
   const float* bias;   // additive bias [B, Hq, Sq, Sk] f32 added to the (capped) scaled scores, or null
-  // Key splits (few workgroups against a long key range): gridDim.y = query blocks x nsplit;
-  // split s of a workgroup covers the 64-key tiles [s tiles_per_split, (s + 1) tiles_per_split)
+  // Key splits (few workgroups against a long key range): query blocks x nsplit in gridDim.y (gridDim.z with
+  // blocks_last); split s of a workgroup covers the 64-key tiles [s tiles_per_split, (s + 1) tiles_per_split)
   // of its key range and writes a normalised partial O (f32, contiguous [B, Hq, Sq, D]) and its
   // log-sum-exp at O + s split_o_elems and LSE + s B Hq Sq; flash_decode_merge_kernel merges them.
   int nsplit;          // 0 or 1: none
   int tiles_per_split;
   long split_o_elems;  // B Hq Sq D
+  int blocks_last;     // order of the grid, see the kernel's "work order"; B Hkv a multiple of 8 only
 };
 
 // Visible keys [lo, hi] of query row i — the reference's attention_bounds
@@ -212,12 +213,12 @@ __global__ __launch_bounds__((FlashGeom<DP, W>::THREADS), 2) void flash_fwd_kern
   // the grid is (B * Hq, query blocks, 1), heaviest blocks first.  No index needs a
   // division either way.
   // qlin / kvlin: linear (batch, head) index of the query head / of its KV head.
-  // Workgroups of 4 waves serve short sequences, whose K and V stay in the L2 in any order, two to a compute
-  // unit: their query blocks come last in the grid, so that the heavy blocks of all heads are dealt out first
+  // blocks_last (workgroups of 4 waves, two to a compute unit, while K and V of all heads are found again in the caches):
+  // the grid is (8 * ratio, B * Hkv / 8, query blocks), so that the heavy blocks of all heads are dealt out first
   // and share a unit with light ones (with the order above B 2 x S 1024 put two heavy ones on one unit).
   const int nsplit = p.nsplit > 1 ? p.nsplit : 1;
   const bool grouped = gridDim.z > 1 || (int)gridDim.x == 8 * p.ratio;
-  const bool blocks_last = W == 4 && grouped;
+  const bool blocks_last = W == 4 && p.blocks_last;
   const int yblocks = blocks_last ? gridDim.z : gridDim.y, yblock = blocks_last ? blockIdx.z : blockIdx.y;
   const int split = p.nsplit > 1 ? yblock % nsplit : 0;
   const int qb = yblocks / nsplit - 1 - yblock / nsplit;

@@ -41,6 +41,18 @@ def test_forward_divisions(lane, b, hq, hkv, sq, sk, d, causal, window, dtype):
     assert np.array_equal(np.isfinite(lse), seen) and np.max(np.abs(lse[seen] - rl[seen])) <= 2e-3
 
 
+@pytest.mark.parametrize("d,causal,sq,sk", [(128, True, 350, 350), (112, False, 290, 400)])
+def test_forward_many_heads_past_the_caches(lane, d, causal, sq, sk):
+    """K and V of 90 MB in heads that share none: 4-wave workgroups head after head.  Every head and row block must be served by
+    its own K and V: reference for the first, the last and a few heads between."""
+    b, h = 64, 8
+    (q, k, v, _), (qf, kf, vf, _) = _case(b, h, h, sq, sk, d, "bf16")
+    o, lse = ops.gqa_attention(q, k, v, causal=causal, return_lse=True, out="f32")
+    for i, j in ((0, 0), (0, 7), (1, 0), (31, 3), (40, 5), (63, 7)):
+        ro, rl = orc.flash_attn_dense(*(x[i:i + 1, j:j + 1] for x in (qf, kf, vf)), causal=causal)
+        assert orc.max_rel_err(o[i, j], ro[0, 0]) <= 2e-3 and np.max(np.abs(lse[i, j] - rl[0, 0])) <= 2e-3, (i, j)
+
+
 @pytest.mark.parametrize("b,hq,hkv,sq,sk,d,causal,dtype", [
     (1, 8, 1, 512, 512, 128, True, "bf16"),      # 8 heads a group: dK / dV walks shared, heads and tiles split unevenly
     (1, 8, 1, 640, 640, 64, False, "f16"),

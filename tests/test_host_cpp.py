@@ -103,6 +103,49 @@ int main(int argc, char** argv) {
     assert got == {**splits, **general}
 
 
+def test_attention_shapes_follow_their_timings(tmp_path):
+    """Waves and key splits of the plain attention forward at shapes timed both ways (causal, D 128 where not said)."""
+    wide, four = 8, 4
+    timed = {  # (B, Hq, Hkv, Sq, Sk, D, causal): waves
+        (2, 32, 8, 500, 500, 128, 1): four, (1, 32, 8, 1000, 1000, 128, 1): four, (1, 32, 8, 2048, 2048, 128, 1): four,
+        (9, 32, 8, 384, 384, 128, 1): four, (1, 32, 8, 4096, 4096, 128, 1): wide, (4, 32, 8, 4096, 4096, 128, 1): wide,
+        # few rows on long contexts, the 8-wave form with its own splits: 282 us against 298, 517 / 540, 548 / 587, 287 / 318
+        (1, 32, 8, 512, 32768, 128, 1): wide, (1, 32, 8, 1024, 32768, 128, 1): wide, (1, 32, 8, 256, 131072, 128, 1): wide,
+        (1, 8, 8, 1024, 65536, 128, 1): wide, (1, 32, 8, 512, 4096, 128, 1): four, (1, 32, 8, 256, 16384, 128, 1): four,
+        (2, 16, 16, 233, 1133, 80, 1): four, (1, 32, 8, 227, 1127, 80, 1): four, (7, 8, 1, 108, 1008, 64, 1): wide,
+        # one round of 8 waves, a half-empty second block: 17.5 / 18.5; a small third one 17.2 / 16.3
+        (4, 32, 4, 350, 350, 128, 1): wide, (8, 16, 16, 384, 384, 128, 1): wide, (4, 32, 4, 300, 300, 128, 1): four,
+        # heads that share no K and V, past the caches: 39.3 / 46.0, 59.6 / 66.9; within them 35.4 / 34.0; half as wide 23.2 / 21.6
+        (16, 32, 32, 256, 256, 128, 1): wide, (24, 32, 32, 256, 256, 128, 1): wide, (10, 32, 32, 256, 256, 128, 1): four,
+        (16, 32, 32, 256, 256, 64, 1): four, (20, 32, 32, 500, 500, 128, 1): wide, (24, 32, 32, 640, 640, 128, 1): four,
+        (18, 8, 8, 1559, 1559, 80, 1): four, (1, 8, 8, 256, 65536, 128, 1): four,
+        (16, 8, 8, 1572, 1572, 128, 1): four, (34, 32, 32, 107, 307, 80, 1): four, (26, 32, 32, 99, 999, 128, 1): four,
+        (1, 8, 2, 3065, 3065, 80, 1): four, (1, 32, 4, 342, 342, 80, 1): wide, (41, 8, 8, 881, 881, 80, 1): four,
+        (1, 8, 1, 180, 1080, 128, 1): wide, (1, 16, 16, 133, 1033, 128, 1): wide, (8, 16, 16, 160, 160, 128, 1): four,
+        (1, 8, 1, 3333, 4233, 80, 1): wide, (10, 8, 2, 640, 640, 80, 1): wide, (10, 8, 2, 512, 512, 80, 1): four, (8, 16, 16, 300, 300, 80, 1): wide}
+    out = _run(tmp_path, r"""
+#include "attn_rules.h"
+#include <cstdio>
+#include <cstdlib>
+int main(int argc, char** argv) {
+  for (int i = 1; i + 6 < argc; i += 7) {
+    int v[7];
+    for (int j = 0; j < 7; ++j) v[j] = atoi(argv[i + j]);
+    const tsr950::FlashProblem p{v[0], v[1], v[2], v[3], v[4], v[5], false};
+    const int off = p.Sk > p.Sq ? p.Sk - p.Sq : 0;
+    const auto f = tsr950::flash_shape(p, [&](int q0, int rows) { return ((v[6] ? std::min(p.Sk, q0 + rows + off) : p.Sk) + 63) / 64; });
+    std::printf("%d %d %d\n", f.waves, f.nsplit, tsr950::flash_blocks_last(p));
+  }
+}
+""", *[x for c in timed for x in c])
+    for (shape, waves), line in zip(timed.items(), out.splitlines()):
+        got, nsplit, last = map(int, line.split())
+        b, hq, hkv, sq, sk, d, _ = shape
+        assert got == waves, (shape, line)
+        assert nsplit == 1 or (b * hq * -(-sq // 256) < 192 and nsplit <= -(-sk // 64) // 8)
+        assert last == (hq != hkv or d <= 96 or b * hkv < 300 or 4 * d * b * hkv * sk < 9e7)
+
+
 # A device of 100 units, counted, in the place of HIP: `used` units are out, `syncs` synchronisations happened.
 _FAKE_DEVICE = r"""
 #include "device_pool.h"
