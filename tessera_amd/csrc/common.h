@@ -123,7 +123,13 @@ __device__ __forceinline__ uint4 buffer_load_b128(const void* base, uint32_t byt
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// A weight matrix of at least this many bytes is streamed with the non-temporal hint (above).
+// A matrix (the weights of all experts, a layer's K and V) of at least this many bytes is streamed with the non-temporal hint.
+// What counts is whether it is still in the 256 MB cache at its next use.  In a model other layers' weights or caches come
+// between, some hundred megabytes of them, and the line is where the hint gains then: several matrices in turn, 16 x 8192 x
+// 8192 (134 MB) 31.0 -> 28.4 us, 8 x 14336 x 4096 (117 MB) 25.7 -> 24.6, decode on 134 to 600 MB of K and V 5 to 11 %, but 67 MB
+// 5 to 10 % slower.  One matrix of 100 to 256 MB alone in a loop stays in the cache without the hint and pays for it:
+// 8 x 8192 x 8192 24.8 -> 27.0 us, 8 x 12288 x 4096 18.7 -> 22.9, decode 4 to 9 %.  The forms without the hint: 8-bit and
+// off-grid few-row products, decode at padded head dimensions and with more than 32 rows a KV head; not measured with it.
 constexpr double kStreamOnceBytes = 1.0e8;
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }

@@ -313,7 +313,9 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     // non-temporal hint (7168 x 8192 29.4 -> 25.7, 14336 x 4096 28.5 -> 25.6).  Else the tiles: 7168 x 4096 15.4 against
     // 13.0, 8064 x 4096 (252 workgroups) 16.2 against 14.1, 6144 x 8192 23.0 against 21.2, 14656 x 2176 15.4 against 13.9; with K ranges
     // under 512, 2048 x 7168, 11.5 against 12.2.  And where K has no even split that would give the tiles enough
-    // workgroups (27 x 3520 x 5312: 32.7 -> 13.7).
+    // workgroups (27 x 3520 x 5312: 32.7 -> 13.7).  (The lines lie between those points, all but the last at 16 rows; 1.1e8 stands
+    // above kStreamOnceBytes because 6144 x 8192, 1.007e8, gains nothing.  Over 16 weight shapes under 9 to 32 rows, several
+    // matrices in turn, no choice is slower than the tiles by more than 1 %; a matrix alone in a loop: see kStreamOnceBytes.)
     if (M <= kSkinnyWideMaxM && N >= 128) {
       const int wide = skinny_wide_splits(N, K);
       const long wgs = (long)ceil_div(N, 128) * wide;

@@ -8,8 +8,8 @@
 //   topk_kernel    one wavefront per token: f32 max-subtracted softmax over the
 //                  experts, k rounds of (max value, lowest index) selection,
 //                  optional renormalisation of the k weights.
-//   plan_kernel    up to 16384 slots: the three passes below by one workgroup, and up to
-//                  128 tokens the selection as well (a launch costs more than the work it holds).
+//   plan_kernel    up to kPlanMaxSlots slots: the three passes below by one workgroup, and up to
+//                  kPlanTopkMaxTokens tokens the selection as well (a launch costs more than the work it holds).
 //   count_kernel   per-chunk histogram of the selected experts.
 //   scan_kernel    per-expert exclusive scan over chunks (= each chunk's first
 //                  rank inside every expert, in token-major order), capacity
