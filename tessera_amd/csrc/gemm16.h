@@ -58,29 +58,43 @@ enum Activation : int { ACT_NONE = 0, ACT_RELU = 1, ACT_GELU = 2, ACT_SILU = 3, 
 // All of them but relu are a logistic function of a linear or cubic argument:
 //   silu v sig(v); sigmoid sig(v); tanh 2 sig(2v) - 1;
 //   gelu (tanh form, argument clamped to +-30) 0.5 v (1 + tanh t) = v sig(2t).
+// 4 sig(x) = 1 / (1/4 + 2^t / 4) with t = -x log2(e): the hardware reciprocal and one Newton step instead of the
+// correctly rounded division (about 10 instructions, on a 256 x 256 tile as long as 8 K steps), with the same
+// measured error against 64 bits.  The factor 4 keeps the reciprocal of the largest finite denominator a
+// normal number (the instruction flushes smaller ones).  An infinite denominator gives 0: the Newton step's
+// inf * 0 is caught by the maximum, which drops a NaN; a NaN argument stays one through the factor v, or is passed on
+// where there is none.
+__device__ __forceinline__ float four_logistic(float t) {
+  const float d = fmaf(__builtin_amdgcn_exp2f(t), 0.25f, 0.25f);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaxf(fmaf(fmaf(-d, r, 1.0f), r, r), 0.0f);
+}
+constexpr float kNegLog2e = -1.44269504088896340736f;
 template <int ACT>
 __device__ __forceinline__ float activate_as(float v) {
   if constexpr (ACT == ACT_NONE) return v;
   if constexpr (ACT == ACT_RELU) return fmaxf(v, 0.f);
-  float x = v;
-  if constexpr (ACT == ACT_GELU) x = 2.f * fminf(fmaxf(0.7978845608028654f * (v + 0.044715f * v * v * v), -30.f), 30.f);
-  if constexpr (ACT == ACT_TANH) x = 2.f * v;
-  const float sg = 1.0f / (1.0f + __expf(-x));
-  if constexpr (ACT == ACT_SIGMOID) return sg;
-  if constexpr (ACT == ACT_TANH) return 2.f * sg - 1.f;
-  return v * sg;
+  if constexpr (ACT == ACT_GELU) {
+    constexpr float c = 2.0f * 0.7978845608028654f * kNegLog2e, most = -60.0f * kNegLog2e;
+    const float t = v * fmaf(v * v, 0.044715f * c, c);
+    return (0.25f * v) * four_logistic(fminf(fmaxf(t, -most), most));
+  }
+  if constexpr (ACT == ACT_SILU) return (0.25f * v) * four_logistic(v * kNegLog2e);
+  if constexpr (ACT == ACT_SIGMOID) return v != v ? v : 0.25f * four_logistic(v * kNegLog2e);
+  return v != v ? v : 0.5f * four_logistic(2.0f * kNegLog2e * v) - 1.0f;
 }
 __device__ __forceinline__ float activate(float v, int act) {
-  if (act == ACT_NONE) return v;
-  if (act == ACT_RELU) return fmaxf(v, 0.f);
-  float x = v;
-  if (act == ACT_GELU) x = 2.f * fminf(fmaxf(0.7978845608028654f * (v + 0.044715f * v * v * v), -30.f), 30.f);
-  if (act == ACT_TANH) x = 2.f * v;
-  const float sg = 1.0f / (1.0f + __expf(-x));
-  if (act == ACT_SIGMOID) return sg;
-  if (act == ACT_TANH) return 2.f * sg - 1.f;
-  return v * sg;
+  switch (act) {
+    case ACT_NONE: return v;
+    case ACT_RELU: return activate_as<ACT_RELU>(v);
+    case ACT_GELU: return activate_as<ACT_GELU>(v);
+    case ACT_TANH: return activate_as<ACT_TANH>(v);
+    case ACT_SIGMOID: return activate_as<ACT_SIGMOID>(v);
+    default: return activate_as<ACT_SILU>(v);
+  }
 }
+// silu on the storage grid times up: the SwiGLU of the expert layers.
+__device__ __forceinline__ float swiglu_of(float g, float u) { return activate_as<ACT_SILU>(g) * u; }
 
 // Four result columns n .. n + 3 of one row (row_at: element offset of the row) through the bias /
 // activation epilogue, stored as f32 or in the storage dtype.  vec: the row takes one vector store;
@@ -591,6 +605,13 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, c
   auto emit = [&](auto act_c, auto bias_c) __attribute__((always_inline)) {
     constexpr int ACT = decltype(act_c)::value;
     constexpr bool HAS_BIAS = decltype(bias_c)::value;
+    // Bias and activation are applied between the LDS read and the store: a lane's four columns are the same in
+    // every row it stores, so the bias is one load per lane, and the arithmetic runs while earlier rows drain to
+    // memory.  (On the accumulators, before staging: 4096^3 into f32 110 us plain, 116 with a bias, 129 with gelu.)
+    float4 bv = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (EPI == EPI_F32_FUSED && HAS_BIAS) {
+      if (st_n < p.N) bv = *reinterpret_cast<const float4*>(p.bias + st_n);
+    }
 #pragma unroll
     for (int b0 = 0; b0 < MB; b0 += IB) {
 #pragma unroll
@@ -600,18 +621,8 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, c
         for (int j = 0; j < NJ_OUT; ++j) {
 #pragma unroll
           for (int q = 0; q < QG; ++q) {
-            const int n = nw0 + j * MS + q * 8 + lk * 4;
             float v0 = acc[i][j][q * 4 + 0], v1 = acc[i][j][q * 4 + 1];
             float v2 = acc[i][j][q * 4 + 2], v3 = acc[i][j][q * 4 + 3];
-            if constexpr (EPI == EPI_F32_FUSED) {
-              if constexpr (HAS_BIAS) {
-                // (a column past N is never stored; its bias read stays in range)
-                const float4 bv = *reinterpret_cast<const float4*>(p.bias + (n < p.N ? n : 0));
-                v0 += bv.x; v1 += bv.y; v2 += bv.z; v3 += bv.w;
-              }
-              v0 = activate_as<ACT>(v0); v1 = activate_as<ACT>(v1);
-              v2 = activate_as<ACT>(v2); v3 = activate_as<ACT>(v3);
-            }
             if constexpr (EPI == EPI_GATED_F32) {
               const acc_t& u = acc[i][j + NJ / 2];
               v0 = activate_as<ACT>(v0) * u[q * 4 + 0]; v1 = activate_as<ACT>(v1) * u[q * 4 + 1];
@@ -630,7 +641,7 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, c
                   // every intermediate lives on the storage grid, as in the reference
                   const float gs = from_storage<T>(to_storage<T>(g[e]));
                   const float us = from_storage<T>(to_storage<T>(u[q * 4 + e]));
-                  o[e] = (gs / (1.0f + __expf(-gs))) * us;
+                  o[e] = swiglu_of(gs, us);
                 }
                 v0 = o[0]; v1 = o[1]; v2 = o[2]; v3 = o[3];
               }
@@ -646,7 +657,13 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, c
 #pragma unroll
       for (int it = 0; it < IB * 32 / RPI; ++it) {
         const int row = it * RPI + st_row;
-        const uint4 v = lds_read_b128(stg, row * PITCH + st_chunk * 16);
+        uint4 v = lds_read_b128(stg, row * PITCH + st_chunk * 16);
+        if constexpr (EPI == EPI_F32_FUSED) {
+          float4 f = __builtin_bit_cast(float4, v);
+          if constexpr (HAS_BIAS) { f.x += bv.x; f.y += bv.y; f.z += bv.z; f.w += bv.w; }
+          f = make_float4(activate_as<ACT>(f.x), activate_as<ACT>(f.y), activate_as<ACT>(f.z), activate_as<ACT>(f.w));
+          v = __builtin_bit_cast(uint4, f);
+        }
         const int m = m_begin + wm * TM + b0 * 32 + row;
         // N % 8 == 0 on this path: a 16-byte chunk is inside or outside as a whole
         if (m < m_end && st_n < p.N)

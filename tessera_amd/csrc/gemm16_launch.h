@@ -56,7 +56,7 @@ __global__ void gemm16_grouped_generic_kernel(const Gemm16Params p) {
     for (int k = 0; k < p.K; ++k) up += from_storage<T>(A[k]) * from_storage<T>(B2[(long)k * p.ldb]);
     const float gs = from_storage<T>(to_storage<T>(acc));
     const float us = from_storage<T>(to_storage<T>(up));
-    acc = (gs / (1.0f + __expf(-gs))) * us;
+    acc = swiglu_of(gs, us);
   }
   const long o = (long)m * p.ldd + n;
   if constexpr (EPI == EPI_F32) reinterpret_cast<float*>(p.D)[o] = acc;

@@ -1159,7 +1159,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
                                                        uint16_t* __restrict__ out, long n) {
   auto one = [](uint16_t ga, uint16_t ub) -> uint16_t {
     const float g = from_storage<T>(ga), u = from_storage<T>(ub);
-    return to_storage<T>((g / (1.0f + __expf(-g))) * u);
+    return to_storage<T>(swiglu_of(g, u));
   };
   const long tid = (long)blockIdx.x * 256 + threadIdx.x, nth = (long)gridDim.x * 256;
   const bool vec = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;

@@ -156,3 +156,31 @@ def test_gemm_epilogue_keyword(lane, act):
     assert np.array_equal(np.asarray(ops.gemm(a, b, epilogue={}), np.uint16), np.asarray(ops.gemm(a, b), np.uint16))
     with pytest.raises(NotImplementedError):
         ops.gemm(a, b, epilogue={"residual": np.zeros((3, 70, 136), np.float32)})
+
+
+# The activations themselves, through the epilogue of each product kernel: a zero product leaves the bias, here every binary
+# order of magnitude of either sign, zeros, infinities and a NaN.  Bound: the exponent -x log2(e) is off by at most its own
+# rounding (|x| 2^-24 log2(e), as a relative error of the exponential |x| 2^-24) and the exponential, the sum, the reciprocal
+# and the last two products by an ulp each; gelu's cubic argument by three more.  Below the smallest normal number of f32
+# the exponential is flushed: an absolute 1.2e-38 (times |x| where x is a factor).
+@pytest.mark.parametrize("M,N,K", [(2, 640, 64), (64, 640, 64), (128, 2048, 64), (2048, 4096, 64)])
+@pytest.mark.parametrize("act", ["silu", "gelu", "sigmoid", "tanh"])
+def test_activation_values(lane, M, N, K, act):
+    x = np.array([s * m * 2.0 ** e for s in (1, -1) for m in (1.0, 1.37, 1.83) for e in range(-40, 7)] + [0.0, 86.9, 87.6, 88.3, -86.9, -87.6, -88.3])
+    bias = np.zeros(N, np.float32)
+    bias[:x.size] = x
+    bias[-3:] = [np.inf, -np.inf, np.nan]
+    got = ops.fused_gemm(np.zeros((M, K), np.float16), np.zeros((K, N), np.float16), bias=bias, activation=act)
+    assert np.array_equal(got[0], got[-1], equal_nan=True)
+    v = bias[:-3].astype(np.float64)
+    with np.errstate(over="ignore"):
+        arg = 2 * 0.7978845608028654 * (v + 0.044715 * v ** 3) if act == "gelu" else 2 * v if act == "tanh" else v
+        arg = np.clip(arg, -60, 60) if act == "gelu" else arg
+        sig = 1 / (1 + np.exp(-arg))
+        ref = {"silu": v * sig, "gelu": v * sig, "sigmoid": sig, "tanh": np.tanh(v)}[act]
+    rel = (8 + np.abs(arg)) * 2.0 ** -24 * (2 if act == "gelu" else 1)
+    size = 2 * np.maximum(np.abs(ref), sig) if act == "tanh" else np.abs(ref)      # tanh = 2 sig - 1 cancels
+    assert np.all(np.abs(got[0, :-3] - ref) <= rel * size + 1.2e-38 * np.maximum(1, np.abs(v)))
+    inf, ninf, nan = got[0, -3:]
+    assert np.isnan(nan) and inf == (np.inf if act in ("silu", "gelu") else 1.0)
+    assert {"silu": np.isnan(ninf), "gelu": ninf == -np.inf, "sigmoid": ninf == 0, "tanh": ninf == -1}[act]
