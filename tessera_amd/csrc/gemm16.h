@@ -875,4 +875,43 @@ __global__ __launch_bounds__(256) void gemm16_rest_sum_kernel(const float* __res
   }
 }
 
+// A dense product on 256 x 256 tiles whose last, mostly empty round is cut finer: the first main_tiles tiles (in the order
+// of tile_of_block) are computed whole, each of the others by `pieces` workgroups, two 128 x 256 or four 128 x 128
+// pieces, so that more compute units share the last round and none of them needs another one's sums (which the K split
+// above pays for with a pass over the partial tiles, 3.7 TB/s to write and less to read).  The pieces of a tile run on
+// one XCD.  A tile's last rows run on a shorter body where 128 or 64 rows are enough.  f32 results, whole tiles / K
+// split of the last round / pieces: 1531 x 14336 x 4096 with gelu 206 / 206 / 177 us, 1100 x 16384 x 4096 181 / 158 /
+// 143, 2048 x 12288 x 4096 184 / 186 / 171, 6140 x 6136 x 2048 161 / 158 / 143; bound by the pieces' LDS traffic
+// (1125 of 1300 cycles a K step of a 128 x 256 piece).
+template <class T, int EPI>
+__global__ __launch_bounds__(256, 1) void gemm16_pieces_kernel(const Gemm16Params p, int main_tiles, int pieces) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  int tile = blockIdx.x, piece = 0;
+  if (tile >= main_tiles) {
+    const int r = tile - main_tiles;
+    piece = (r >> 3) % pieces;
+    tile = main_tiles + ((r >> 3) / pieces) * 8 + (r & 7);
+    if (tile >= p.tiles_m * p.tiles_n) return;
+  } else {
+    pieces = 1;
+  }
+  int tm, tn;
+  tile_of_block(tile, p.tiles_m, p.tiles_n, tm, tn);
+  const int m_begin = tm * 256 + (pieces == 2 ? piece : piece >> 1) * 128;
+  char* Db = reinterpret_cast<char*>(p.D);
+  if (m_begin >= p.M) return;
+  if (pieces == 4) {
+    tn = tn * 2 + (piece & 1);
+    if (tn * 128 < p.N)
+      gemm16_tile<T, 128, 128, 2, 2, EPI, false, 16>(p, smem, m_begin, p.M, tn, p.A, p.B, nullptr, Db);
+    return;
+  }
+  if (p.M - m_begin <= 64)
+    gemm16_tile<T, 64, 256, 1, 4, EPI, false, 16>(p, smem, m_begin, p.M, tn, p.A, p.B, nullptr, Db);
+  else if (pieces == 2 || p.M - m_begin <= 128)
+    gemm16_tile<T, 128, 256, 2, 2, EPI, false, 16>(p, smem, m_begin, p.M, tn, p.A, p.B, nullptr, Db);
+  else
+    gemm16_tile<T, 256, 256, 2, 2, EPI, false, 16>(p, smem, m_begin, p.M, tn, p.A, p.B, nullptr, Db);
+}
+
 }  // namespace tsr950

@@ -139,6 +139,7 @@ struct Gemm16Schedule {
   int split_k;   // number of K splits (1 = none)
   bool skinny;   // the few-row streaming kernel (32 x 64 workgroup tile up to 8 rows, 32 x 128 above; K slices of 32)
   int rest_split = 1;   // 256 tiles, split_k 1: K splits of the tiles beyond the last full round of 256
+  int pieces = 1;       // ... or 2 or 4: pieces of the output these tiles are cut into
   int tile_m = 0;       // 128 with tile 256: the 128 x 256 tile (tile rows x tile columns); 0: square
 };
 constexpr int kSkinnyMaxM = 8;           // 64-column strips up to here,
@@ -226,7 +227,7 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     // tiles enough for three quarters of the compute units without a K split, which would add a
     // pass over the partials and little parallelism.  The wider tile reads 512 contiguous bytes
     // of a row of B instead of 256 and streams faster once it, too, fills the chip.
-    if ((long)ceil_div(M, 128) * ceil_div(N, 256) >= 192) return {256, 1, false, 1, 128};
+    if ((long)ceil_div(M, 128) * ceil_div(N, 256) >= 192) return {256, 1, false, 1, 1, 128};
     if ((long)ceil_div(M, 128) * ceil_div(N, 128) >= 192) return {128, 1, false};
   }
   if (batch == 1 && M <= kSkinnyMaxM && K % 32 == 0 && K >= 512) {
@@ -247,7 +248,7 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
         const double us = est_few_rows_us(t, M, N, K, splits);
         if (us < best_us) {
           best_us = us;
-          best = t.tile_n == 256 ? Gemm16Schedule{256, splits, false, 1, 128} : Gemm16Schedule{t.tile_m, splits, false};
+          best = t.tile_n == 256 ? Gemm16Schedule{256, splits, false, 1, 1, 128} : Gemm16Schedule{t.tile_m, splits, false};
         }
       }
     return best;
@@ -268,7 +269,7 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
       // (its estimate is the least certain of the three — the per-step figure moved by 13 % between
       // shapes of equal tile count — so it has to win by a margin)
       const double us = 1.06 * est_tiles128x256_us((long)ceil_div(M, 128) * ceil_div(N, 256) * batch, ksteps);
-      if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, 1, 128}; }
+      if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, 1, 1, 128}; }
     }
     if (batch == 1) {
       for (int splits : {2, 3, 4, 8}) {
@@ -278,16 +279,27 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
         consider(128, splits, est_tiles128_us(tiles128 * splits, ksteps / splits) + sum_us);
       }
     }
-    // A tile count a little over a multiple of 256 leaves a last round with most compute units
-    // idle: those tiles can be split along K among them (one more launch and a sum over the
-    // partial tiles).
+    // A tile count that is not a multiple of 256 leaves compute units idle in the last round: its tiles can be cut into
+    // two or four pieces, or, where they are few and K is long, split along K among those units (one more launch and
+    // a sum over the partial tiles: 16 tiles left at K = 4096 137 against 139 us in pieces, at K = 14336 406 against 489;
+    // 80 left at K = 4096 185 against 177).  Pieces still have a whole round before them: under 12 K steps, where prologue and
+    // epilogue are most of it, they have to win against 128 x 128 tiles, two on a unit, by a fifth (5860 x 3424 x 520 with
+    // gelu 51 us on those, 58 in pieces).
     const long full = tiles256 / 256, rest = tiles256 % 256;
-    if (batch == 1 && full >= 1 && rest > 0 && rest <= 128) {
+    if (batch == 1 && full >= 1 && rest > 0 && rest <= 128 && tiles256 < (1L << 30)) {
       const double main_us = (double)full * (9.6 + ksteps * 1.43);
+      const double margin = best.tile == 128 && ksteps < 12 ? 1.2 : 1.0;
+      auto cut = [&](int pieces, double us) {
+        us *= margin;
+        if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, 1, pieces}; }
+      };
+      cut(2, main_us + est_tiles128x256_us(2 * rest, ksteps));
+      // (128 x 128 pieces, alone on their compute units: 0.52 us a K step up to 64 of them, 0.65 from 192 on)
+      if (rest <= 64) cut(4, main_us + 5.0 + ksteps * (0.52 + 0.13 * std::min(1.0, std::max(0.0, (4 * rest - 64) / 128.0))));
       for (int splits : {2, 3, 4, 6, 8, 12, 16}) {
         const int per = ceil_div(ksteps, splits);
         if (rest * splits > 256 || per < 2 || (long)per * (splits - 1) >= ksteps) continue;
-        const double us = main_us + 3.0 + est_tiles256_us(rest * splits, per) +
+        const double us = main_us + 8.0 + est_tiles256_us(rest * splits, per) +
                           est_split_sum_us(rest * 65536L, splits);
         if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, splits}; }
       }
@@ -484,6 +496,24 @@ int launch_gemm16_rest(Gemm16Params p, int first_tile, int rest, int splits, hip
   return launch_status();
 }
 
+// A dense product on 256 x 256 tiles with those beyond the last full round of 256 in `pieces` pieces each.
+template <class T, int EPI>
+int launch_gemm16_pieces(Gemm16Params p, int pieces, hipStream_t s) {
+  using S = Gemm16Smem<256, 256>;
+  auto kern = gemm16_pieces_kernel<T, EPI>;
+  static std::once_flag once;
+  static hipError_t attr_err = hipSuccess;
+  std::call_once(once, [&] {
+    attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, S::kBytes);
+  });
+  if (attr_err != hipSuccess) return kDeviceFailed;
+  p.tiles_m = ceil_div(p.M, 256);
+  p.tiles_n = ceil_div(p.N, 256);
+  const int tiles = p.tiles_m * p.tiles_n, main_tiles = tiles / 256 * 256, rest = tiles - main_tiles;
+  hipLaunchKernelGGL(kern, dim3(main_tiles + ceil_div(rest, 8) * 8 * pieces), dim3(256), S::kBytes, s, p, main_tiles, pieces);
+  return launch_status();
+}
+
 // Dense / batched.  p.groups = batch count (>= 1).
 template <class T, int EPI>
 int launch_gemm16(Gemm16Params p, hipStream_t s) {
@@ -527,9 +557,11 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
     int rc = kOk;
     if (EPI == EPI_F32 && fused) {
       if constexpr (EPI == EPI_F32)
-        rc = launch_gemm16_tile<T, 256, 256, 2, 2, EPI_F32_FUSED, false, kBigTileMfma>(p, s, main_wgs);
+        rc = sch.pieces > 1 ? launch_gemm16_pieces<T, EPI_F32_FUSED>(p, sch.pieces, s)
+                            : launch_gemm16_tile<T, 256, 256, 2, 2, EPI_F32_FUSED, false, kBigTileMfma>(p, s, main_wgs);
     } else {
-      rc = launch_gemm16_tile<T, 256, 256, 2, 2, EPI, false, kBigTileMfma>(p, s, main_wgs);
+      rc = sch.pieces > 1 ? launch_gemm16_pieces<T, EPI>(p, sch.pieces, s)
+                          : launch_gemm16_tile<T, 256, 256, 2, 2, EPI, false, kBigTileMfma>(p, s, main_wgs);
     }
     if (rc != kOk || sch.rest_split <= 1) return rc;
     return launch_gemm16_rest<T, EPI>(p, main_wgs, tiles - main_wgs, sch.rest_split, s);

@@ -45,7 +45,7 @@ class Gfx950ScheduleDescriptor:
     raster_order: str = "xcd_banded"
     raster_group: int = 4
     rest_tiles: int = 0               # tiles beyond the last full round of 256 workgroups that are ...
-    rest_split_k: int = 1             # ... split along K into this many parts (1: none are)
+    rest_split_k: int = 1             # ... divided into this many parts, along K or in the output (1: none are)
 
     @property
     def mt(self) -> int:

@@ -292,3 +292,23 @@ def test_bad_shapes_rejected(lane):
     d = np.zeros(16, np.float32)
     assert lib.tessera_gfx950_gemm_bf16(z.ctypes.data, z.ctypes.data, d.ctypes.data, 0, 4, 4) == 1
     assert lib.tessera_gfx950_gemm_bf16(z.ctypes.data, z.ctypes.data, d.ctypes.data, 4, -1, 4) == 1
+
+
+# The last, mostly empty round in pieces of the output (two 128 x 256 or four 128 x 128 to a tile): row and column edges
+# inside a piece, pieces that lie past an edge altogether, last row tiles of at most 64 and 128 rows among the whole
+# tiles, a number of rest tiles that is not a multiple of 8, a K that ends inside a step.  f32 sums: 1e-5.
+@pytest.mark.parametrize("M,N,K,parts", [(4100, 4104, 1096, 4), (1345, 12424, 1032, 4), (1430, 13960, 1032, 2),
+                                         (1100, 15400, 840, 4), (4096, 4352, 776, 4), (2303, 9480, 1600, 2)])
+def test_rest_round_in_pieces(lane, M, N, K, parts):
+    from tessera_amd.schedule import select_gfx950_gemm_schedule
+    sch = select_gfx950_gemm_schedule(M, N, K, dtype="bf16")
+    assert sch.workgroup_tile[:2] == (256, 256) and sch.split_k == 1 and sch.rest_split_k == parts
+    rng = np.random.default_rng(M + 2 * N + 3 * K)
+    a = b16.from_float32((rng.standard_normal((M, K)) / np.sqrt(K)).astype(np.float32))
+    b = b16.from_float32(rng.standard_normal((K, N)).astype(np.float32))
+    ref = a.to_float32().astype(np.float64) @ b.to_float32().astype(np.float64)
+    acc = ops.gemm(a, b, out="f32")
+    assert orc.max_rel_err(acc, ref) <= 1e-5
+    assert np.array_equal(np.asarray(ops.gemm(a, b)).view(np.uint16), np.asarray(b16.from_float32(acc)).view(np.uint16))
+    bias = rng.standard_normal(N).astype(np.float32)
+    assert orc.max_rel_err(ops.fused_gemm(a, b, bias=bias, activation="relu"), np.maximum(ref + bias, 0.0)) <= 1e-5
