@@ -695,9 +695,12 @@ __device__ __forceinline__ void gemm16_tile(const Gemm16Params& p, char* smem, c
   }
 }
 
-// MID (grouped 256-row tiles only): a last row tile of 65 to 128 rows runs on the 128-row tile
-// body.  A separate instantiation, for launches whose groups average at most a tile of rows: the
-// kernel that serves large groups keeps its two bodies.
+// Grouped kernels whose groups have several row tiles take a last one of at most 64 rows in tiles of two columns.
+template <int BM, int WAVES, bool GROUPED, bool MID>
+constexpr bool gemm16_paired_tail() { return GROUPED && BM == 256 && WAVES == 4 && !MID; }
+
+// MID (grouped 256-row tiles only): groups that average at most a tile of rows.  Their short last tiles come one column
+// at a time: there are few workgroups, and no full tiles to keep pace with.
 template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32, bool MID = false, bool NTB = false>
 __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Params p) {
   constexpr bool SWIGLU = (EPI == EPI_SWIGLU16 || EPI == EPI_GATED_F32);
@@ -706,6 +709,8 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Par
 
   // ---- which tile ---------------------------------------------------------
   int tm, tn, m_begin, m_end;
+  constexpr bool PAIRED = gemm16_paired_tail<BM, WM * WN, GROUPED, MID>();
+  bool paired = false;
   const uint16_t* Ab = p.A;
   const uint16_t* Bb = p.B;
   const uint16_t* B2b = p.B2;
@@ -721,10 +726,13 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Par
     // costs microseconds per workgroup, so each wave reads 64 groups per step with one
     // coalesced load, scans their tile counts across its lanes and finds the group of
     // its tile with a ballot.
+    // (PAIRED: a last row tile of at most 64 rows comes in tiles of two columns, see below)
     auto tiles_of = [&](int g, int& lo, int& hi) -> int {
       lo = g < p.groups ? p.offsets[g] : 0;
       hi = g < p.groups ? p.offsets[g + 1] : 0;
-      return ((hi - lo + BM - 1) / BM) * p.tiles_n;
+      const int full = (hi - lo) / BM, left = (hi - lo) % BM;
+      if (PAIRED && left > 0 && left <= 64) return full * p.tiles_n + (p.tiles_n + 1) / 2;
+      return (full + (left > 0)) * p.tiles_n;
     };
     auto wave_scan = [&](int v) -> int {             // inclusive prefix sum over the 64 lanes
 #pragma unroll
@@ -773,8 +781,21 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Par
     g_hi = __builtin_amdgcn_readfirstlane(g_hi);
     mt = __builtin_amdgcn_readfirstlane(mt);
     const int r = lin - acc;
-    tn = r / mt;
-    tm = r - tn * mt;
+    const int left = (g_hi - g_lo) % BM;
+    if (PAIRED && left > 0 && left <= 64) {
+      // two columns of full tiles, then the tile of the last rows across both of them: they run together and share the
+      // weight panels in their XCD's L2
+      const int full = mt - 1, run = 2 * full + 1;
+      const int pair = r / run, x = r - pair * run;
+      const bool odd = 2 * pair + 1 == p.tiles_n;           // a last column by itself
+      paired = x == (odd ? full : 2 * full);
+      const int second = !odd && full > 0 && x >= full;
+      tn = paired ? pair : 2 * pair + second;
+      tm = paired ? full : x - second * full;
+    } else {
+      tn = r / mt;
+      tm = r - tn * mt;
+    }
     m_begin = g_lo + tm * BM;
     m_end = g_hi;
     Bb += (long)e * p.strideB;
@@ -792,15 +813,25 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Par
     // A group's last row tile is often nearly empty (rows per expert are a little over a
     // multiple of BM about half of the time).  With at most 64 rows left the four waves
     // share the columns of a 64-row tile instead: a quarter of the matrix work of the
-    // full tile, whose other 192 rows would be computed and thrown away.
-    if (m_end - m_begin <= 64) {
+    // full tile, whose other 192 rows would be computed and thrown away.  Where groups have
+    // several row tiles it takes two columns at once, 64 x 512 (64 MFMAs a wave and K step and the LDS traffic of three
+    // quarters of a full tile: it keeps pace with the full tiles that share its weight panels by itself, where the
+    // narrow one was slowed down to them and sat on its compute unit as long for one column).  64 experts of 4096 x
+    // 1408, top-8, the whole layer: 8192 tokens 2150 -> 2046 us, 4096 1170 -> 1130; 8 experts of 3968 x 3392, 1026
+    // tokens top-4, 423 -> 357.
+    if constexpr (PAIRED) {
+      if (paired) {
+        gemm16_tile<T, 64, 2 * BN, 1, 4, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
+        return;
+      }
+    } else if (m_end - m_begin <= 64) {
       // (paced when full tiles of the same group and column run beside it; 16-wide step only)
       gemm16_tile<T, 64, BN, 1, 4, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db, MS == 16 && tm > 0);
       return;
     }
-    // (up to 128 rows left — a group of about a hundred rows, a chunk of a thousand tokens over
-    // 64 experts — the 128-row tile: half the matrix work)
-    if (MID && m_end - m_begin <= 128) {
+    // (up to 128 rows left: the 128-row tile, half the matrix work; 2542 tokens top-4 over 16 experts of 2368 x 3776
+    // 614 -> 585 us)
+    if (m_end - m_begin <= 128) {
       gemm16_tile<T, 128, BN, 2, 2, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
       return;
     }

@@ -74,13 +74,14 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // (the caller serves the remaining tiles itself).
 template <class T, int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int MS = 32, bool MID = false, bool NTB = false>
 int launch_gemm16_tile(Gemm16Params p, hipStream_t s, int wg_limit = 0) {
-  using S = Gemm16Smem<BM, BN>;
+  constexpr int kLds = gemm16_paired_tail<BM, WM * WN, GROUPED, MID>() ? std::max(Gemm16Smem<BM, BN>::kBytes, Gemm16Smem<64, 2 * BN>::kBytes)
+                                                                       : Gemm16Smem<BM, BN>::kBytes;
   auto kern = gemm16_kernel<T, BM, BN, WM, WN, EPI, GROUPED, MS, MID, NTB>;
   static std::once_flag once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(once, [&] {
     attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, S::kBytes);
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   });
   if (attr_err != hipSuccess) return kDeviceFailed;
   constexpr int BN_OUT = (EPI == EPI_SWIGLU16 || EPI == EPI_GATED_F32) ? BN / 2 : BN;
@@ -95,7 +96,7 @@ int launch_gemm16_tile(Gemm16Params p, hipStream_t s, int wg_limit = 0) {
     p.tiles_m = ceil_div(p.M, BM);
     grid = dim3(wg_limit > 0 ? wg_limit : p.tiles_m * p.tiles_n, 1, p.groups);
   }
-  hipLaunchKernelGGL(kern, grid, dim3(WM * WN * 64), S::kBytes, s, p);
+  hipLaunchKernelGGL(kern, grid, dim3(WM * WN * 64), kLds, s, p);
   return launch_status();
 }
 
@@ -674,8 +675,7 @@ int launch_gemm16_grouped(Gemm16Params p, hipStream_t s) {
     hipLaunchKernelGGL((gemm16_grouped_generic_kernel<T, EPI>), grid, block, 0, s, p);
     return launch_status();
   }
-  // groups that average at most a tile of rows (a chunk of a thousand tokens over 64 experts): the
-  // instantiation whose last row tile also comes in a 128-row form
+  // groups that average at most a tile of rows (a chunk of a thousand tokens over 64 experts): see MID at the kernel
   const bool mid = (long)p.M <= 256L * p.groups;
   // Weights that outgrow the memory-side cache are streamed past it while their panels are read by one row tile: groups
   // that average at most 240 rows.  Closer to the tile's 256 half of the groups have a second tile, whose reads then miss (the

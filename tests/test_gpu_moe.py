@@ -264,6 +264,24 @@ def test_moe_swiglu_block(lane, sizes, K, F, N):
     assert np.mean(got != ref) < 0.05
 
 
+# Groups of several row tiles (more than 256 rows on average): a last row tile of 1 to 64 rows is computed two column tiles
+# at a time, 65 and more whole.  One, two and three column tiles of 256 (the product; 128 in the block), the last of them
+# narrow; a group that is nothing but such a tile, an empty one, a K that ends inside a step.
+@pytest.mark.parametrize("K,F,N", [(136, 128, 256), (200, 256, 512), (72, 328, 760), (520, 384, 1288)])
+def test_last_rows_across_two_column_tiles(lane, K, F, N):
+    sizes = [320, 257, 64, 0, 833, 577, 1089, 512, 321]
+    x, wg, wu, wd = _swiglu_inputs(sizes, K, F, N, 7)
+    ref = orc.moe_swiglu_block(x, wg, wu, wd, sizes)
+    got = ops.moe_swiglu_block(*(b16.from_float32(a) for a in (x, wg, wu, wd)), sizes).to_float32()
+    assert orc.max_rel_err(got, ref) <= TOL + 2.0 ** -8       # (bounds as for the block above)
+    assert np.mean(got != ref) < 0.05
+    w = (np.random.default_rng(K).standard_normal((len(sizes), K, N)) / np.sqrt(K)).astype(np.float32)
+    acc = ops.grouped_gemm(b16.from_float32(x), b16.from_float32(w), sizes, out="f32")
+    assert orc.max_rel_err(acc, orc.grouped_gemm(x, w, sizes, store=False)) <= 1e-5          # f32 sums
+    stored = ops.grouped_gemm(b16.from_float32(x), b16.from_float32(w), sizes)
+    assert np.array_equal(stored.to_float32(), orc.round_to_storage(acc, "bf16"))
+
+
 @pytest.mark.parametrize("T,K,F,N,E,k", [(300, 256, 384, 128, 8, 2), (1024, 128, 1408, 256, 16, 4),
                                           (77, 64, 128, 64, 4, 1)])
 def test_swiglu_block_reading_through_the_dispatch_map(lane, T, K, F, N, E, k):
