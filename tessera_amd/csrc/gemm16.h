@@ -153,6 +153,7 @@ struct Gemm16Params {
                           // into the A load); null: row m
   int groups;             // E (grouped) or batch count
   int tiles_m, tiles_n;   // tile grid (grouped: tiles_m is an upper bound)
+  int k_total;            // K splits as batches: the whole K, of which batch z has [z K, min((z + 1) K, k_total)); else 0
 };
 
 
@@ -836,7 +837,13 @@ __global__ __launch_bounds__(WM * WN * 64, 1) void gemm16_kernel(const Gemm16Par
       return;
     }
   }
-  gemm16_tile<T, BM, BN, WM, WN, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
+  if constexpr (GROUPED) {
+    gemm16_tile<T, BM, BN, WM, WN, EPI, GROUPED, MS, NTB>(p, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
+  } else {
+    Gemm16Params part = p;
+    if (p.k_total) part.K = min(p.K, p.k_total - (int)blockIdx.z * p.K);
+    gemm16_tile<T, BM, BN, WM, WN, EPI, GROUPED, MS, NTB>(part, smem, m_begin, m_end, tn, Ab, Bb, B2b, Db);
+  }
 }
 
 // The tiles that are left when the tile count is not a multiple of the 256 compute units would

@@ -149,6 +149,12 @@ constexpr int kLooseMaxM = 64;           // and for rows of B on any boundary up
 constexpr long kSplitTargetWgs = 768;
 constexpr int kWeightStreamMaxM = 128;   // up to here a product is bound by reading B once
 
+// K steps in each part of a K split: as many in every part but the last, which may be shorter.  (A split used to need a
+// K that it divides into whole steps: 202 x 5120 x 9152 stayed whole, 93 us, and
+// takes 42 in three; 961 x 960 x 11344 84 -> 37, 64 x 896 x 14000 82 -> 14.)
+inline int split_steps(int K, int splits) { return ceil_div(ceil_div(K, G16_BK), splits); }
+inline bool can_split(int K, int splits) { return (long)(splits - 1) * split_steps(K, splits) < ceil_div(K, G16_BK); }
+
 // Time estimates (microseconds) behind the choice for products with more than kWeightStreamMaxM
 // rows, fitted to timings of forced (tile, split) pairs on this part over products from 1024^3
 // to 7168^3: a 256 x 256 tile spends 9.6 us outside its K loop and 1.09 us per 64-deep K step
@@ -192,13 +198,67 @@ constexpr FewRowTile kFewRowTiles[3] = {{64, 64, 0.26, 0.514, 0.256, 5.39},
                                         {128, 256, 3.97, 0.693, 1.582, 7.01}};
 inline double est_few_rows_us(const FewRowTile& t, int M, int N, int K, int splits) {
   const long wgs = (long)ceil_div(M, t.tile_m) * ceil_div(N, t.tile_n) * splits;
-  const double steps = (double)K / G16_BK / splits;
+  const double steps = split_steps(K, splits);
   const double busiest = (double)((wgs + 255) / 256);
   const double compute = steps * (t.step + t.shared * (busiest - 1.0));
   const double bytes = 2.0 * K * ceil_div(N, t.tile_n) * t.tile_n;
   const double stream = bytes / (t.tbs * 1e6 * std::min(1.0, wgs / 185.0));
   const double sum = splits > 1 ? 3.4 + (double)M * N * splits * 1.6e-6 : 0.0;
   return t.launch + std::max(compute, stream) + sum;
+}
+
+// Second opinion for single products of 129 to about 3000 rows on fewer than 260 tiles of 256 x 256, where the estimates
+// above (fitted to matrices found in the caches, and without the 64 x 64 tile) were on average 5.6 % behind the best of
+// the forced schedules and up to 47 %: fitted (4 to 12 % rms) to 2033 timings of forced (tile, split) pairs over 260
+// products, weights streamed from memory.  A launch, then the larger of the K steps and of streaming B; 64- and 128-wide
+// tiles share a compute unit (the first at `step` a K step, each further one `more`), 256-wide ones come in rounds (a
+// step `step` on a quiet chip, `more` on a full one); a split adds its sum.
+// 100 products of 16 to 3000 rows with another schedule than before, by this or by uneven parts: 1.5 times as fast on average.
+struct MidTile { int tile_m, tile_n; double launch, step, more, tbs, sum, per_mega; };
+constexpr MidTile kMidTiles[4] = {{64, 64, 1.158, 0.4031, 0.1924, 14.09, 2.744, 1.677},
+                                  {128, 128, 2.436, 0.5124, 0.5325, 2.914, 3.348, 1.262},
+                                  {128, 256, 3.896, 0.749, 1.006, 5.977, 3.825, 0.9554},
+                                  {256, 256, 8.098, 1.089, 1.506, 6.356, 4.376, 0.8394}};
+inline double est_mid_us(const MidTile& t, int M, int N, int K, int splits) {
+  const long wgs = (long)ceil_div(M, t.tile_m) * ceil_div(N, t.tile_n) * splits;
+  const double per = split_steps(K, splits);
+  const double bytes = 2.0 * K * ceil_div(N, t.tile_n) * t.tile_n;
+  const double stream = t.launch + bytes / (t.tbs * 1e6 * std::min(1.0, wgs / 185.0));
+  double steps;
+  if (t.tile_n < 256) {
+    steps = t.launch + per * (t.step + t.more * (double)((wgs + 255) / 256 - 1));
+  } else {
+    const double rest = (double)(wgs % 256);
+    steps = (double)(wgs / 256) * (t.launch + per * t.more);
+    if (rest > 0) steps += t.launch + per * (t.step + (t.more - t.step) * std::min(1.0, std::max(0.0, (rest - 96.0) / 128.0)));
+  }
+  return std::max(steps, stream) + (splits > 1 ? t.sum + (double)M * N * splits * t.per_mega * 1e-6 : 0.0);
+}
+// The schedule `first` or, where this estimate sees a tenth less time, its own choice.  (Over the 260 products 2.5 %
+// behind the best, and no product more than 5 % behind what it had before.)
+inline Gemm16Schedule second_opinion_mid(const Gemm16Schedule& first, int M, int N, int K) {
+  auto is = [&](const MidTile& t) { return t.tile_n == first.tile && t.tile_m == (first.tile_m ? first.tile_m : first.tile); };
+  double first_us = 0.0, best_us = 1e30, whole_us = 1e30;
+  Gemm16Schedule best = first, whole = first;           // whole: the best without a K split
+  for (const MidTile& t : kMidTiles) {
+    if (is(t)) first_us = est_mid_us(t, M, N, K, first.split_k);
+    if (t.tile_n == 64 && M > 512) continue;           // (not measured)
+    for (int splits : {1, 2, 3, 4, 6, 8}) {
+      if (splits > 1 && (!can_split(K, splits) || K / splits < 256)) continue;
+      const double us = est_mid_us(t, M, N, K, splits);
+      const Gemm16Schedule sch = t.tile_m < t.tile_n ? Gemm16Schedule{256, splits, false, 1, 1, 128} : Gemm16Schedule{t.tile_n, splits, false};
+      if (us < best_us) { best_us = us; best = sch; }
+      if (splits == 1 && us < whole_us) { whole_us = us; whole = sch; }
+    }
+  }
+  // (from a 256-wide tile to 128 x 128 ones, whose third and fourth on a unit cost more than the estimate has them, by a
+  // fifth; to more parts by 2 us at least: 1052 x 704 x 1472 in four parts 14.9 us, whole 12.5)
+  const bool narrower = first.tile == 256 && best.tile < 256;
+  if (best_us < (narrower ? 0.8 : 0.9) * first_us && (best.split_k <= first.split_k || best_us + 2.0 < first_us)) return best;
+  // (a split into unequal parts that it sees nothing in is not taken: 1240 x 704 x 1368 whole / in two parts 13.1 / 14.8
+  // us, 2104 x 2560 x 4288 56 / 64)
+  if (first.split_k > 1 && K % (first.split_k * G16_BK) != 0 && whole_us < 1.05 * first_us) return whole;
+  return first;
 }
 
 // Workgroups of the few-row kernel on 128-column strips with K in as many parts as keep it within one workgroup
@@ -245,8 +305,10 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     double best_us = 1e30;
     for (const FewRowTile& t : kFewRowTiles)
       for (int splits : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        if (K % (splits * G16_BK) != 0 || K / splits < 512) continue;
-        const double us = est_few_rows_us(t, M, N, K, splits);
+        if (!can_split(K, splits) || K / splits < 512) continue;
+        // (the estimate was fitted to equal parts; others have to be worth a twelfth: 84 x 4864 x 1600 whole / in three
+        // parts 11.3 / 12.6 us)
+        const double us = est_few_rows_us(t, M, N, K, splits) * (K % (splits * G16_BK) != 0 && splits > 1 ? 1.08 : 1.0);
         if (us < best_us) {
           best_us = us;
           best = t.tile_n == 256 ? Gemm16Schedule{256, splits, false, 1, 1, 128} : Gemm16Schedule{t.tile_m, splits, false};
@@ -274,10 +336,10 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     }
     if (batch == 1) {
       for (int splits : {2, 3, 4, 8}) {
-        if (K % (splits * G16_BK) != 0 || K / splits < 512) continue;
+        if (!can_split(K, splits) || K / splits < 512) continue;
         const double sum_us = est_split_sum_us((long)M * N, splits);
-        consider(256, splits, est_tiles256_us(tiles256 * splits, ksteps / splits) + sum_us);
-        consider(128, splits, est_tiles128_us(tiles128 * splits, ksteps / splits) + sum_us);
+        consider(256, splits, est_tiles256_us(tiles256 * splits, split_steps(K, splits)) + sum_us);
+        consider(128, splits, est_tiles128_us(tiles128 * splits, split_steps(K, splits)) + sum_us);
       }
     }
     // A tile count that is not a multiple of 256 leaves compute units idle in the last round: its tiles can be cut into
@@ -305,6 +367,8 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
         if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, splits}; }
       }
     }
+    if (batch == 1 && M <= 3000 && tiles256 < 260 && best.rest_split == 1 && best.pieces == 1)
+      best = second_opinion_mid(best, M, N, K);
     return best;
   }
   // Few rows: the weight matrix streams from HBM once and the tiles are small; for a single
@@ -319,7 +383,11 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     // 2 K (M + N) bytes of operands: B dominates under few rows, A over few columns): beyond two
     // splits keep that under about 0.4 of the operand traffic
     splits = (int)std::min<long>(splits, std::max<long>(2, (long)K * (M + N) / (10L * M * N)));
-    while (splits > 1 && K % (splits * G16_BK) != 0) --splits;
+    while (splits > 1 && !can_split(K, splits)) --splits;
+    // (equal parts where they are at least two thirds as many: 21 x 10272 x 2816 in 5 / 4 parts 20.0 / 18.5 us)
+    int equal = splits;
+    while (equal > 1 && K % (equal * G16_BK) != 0) --equal;
+    if (3 * equal >= 2 * splits) splits = equal;
     // 9 to 32 rows: the streaming kernel on 128-column strips instead where it streams faster than the tiles: one
     // workgroup on every compute unit (16 x 8192 x 8192 31.4 -> 28.1 us, 4096 x 4096 12.7 -> 11.3, 8192 x 2048 10.4 ->
     // 9.4; two parts of a short K, 16320 x 2560, 18.2 against 17.3), or nearly so and a B that is read with the
@@ -473,9 +541,9 @@ int launch_gemm16_repitched(const Gemm16Params& p, hipStream_t s) {
 }
 
 // The tiles first_tile .. first_tile + rest - 1 of a dense product on 256 x 256 tiles, each split
-// along K over `splits` workgroups, then summed (with the bias / activation of the product).
+// along K over `splits` workgroups into ws, then summed (with the bias / activation of the product).
 template <class T, int EPI>
-int launch_gemm16_rest(Gemm16Params p, int first_tile, int rest, int splits, hipStream_t s) {
+int launch_gemm16_rest(Gemm16Params p, int first_tile, int rest, int splits, float* ws, hipStream_t s) {
   using S = Gemm16Smem<256, 256>;
   auto kern = gemm16_rest_splitk_kernel<T, kBigTileMfma>;
   static std::once_flag once;
@@ -485,8 +553,6 @@ int launch_gemm16_rest(Gemm16Params p, int first_tile, int rest, int splits, hip
                                    hipFuncAttributeMaxDynamicSharedMemorySize, S::kBytes);
   });
   if (attr_err != hipSuccess) return kDeviceFailed;
-  float* ws = static_cast<float*>(stream_workspace(s, (size_t)rest * splits * 256 * 256 * sizeof(float)));
-  if (!ws) return kDeviceFailed;
   p.tiles_m = ceil_div(p.M, 256);
   p.tiles_n = ceil_div(p.N, 256);
   const int ksplit = ceil_div(ceil_div(p.K, G16_BK), splits) * G16_BK;
@@ -540,7 +606,16 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
     hipLaunchKernelGGL((gemm16_generic_kernel<T, EPI>), grid, block, 0, s, p);
     return launch_status();
   }
-  const Gemm16Schedule sch = select_gemm16_schedule(p.M, p.N, p.K, p.groups);
+  Gemm16Schedule sch = select_gemm16_schedule(p.M, p.N, p.K, p.groups);
+  // The f32 partials of a K split lie in the stream's workspace; without one (a capture on a stream that has none, a full
+  // device) K stays whole on the same tiles.
+  float* ws = nullptr;
+  if (!sch.skinny && (sch.split_k > 1 || sch.rest_split > 1)) {
+    const size_t rest = (size_t)ceil_div(p.M, 256) * ceil_div(p.N, 256) % 256;
+    const size_t floats = sch.split_k > 1 ? (size_t)p.M * p.N * sch.split_k : rest * sch.rest_split * 256 * 256;
+    ws = static_cast<float*>(stream_workspace_or_null(s, floats * sizeof(float)));
+    if (!ws) sch.split_k = sch.rest_split = 1;
+  }
   // bias / activation: the tile kernels have a separate instantiation for it (f32 out)
   const bool fused = p.bias != nullptr || p.act != ACT_NONE;
   if constexpr (EPI != EPI_F32) {
@@ -565,7 +640,7 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
                           : launch_gemm16_tile<T, 256, 256, 2, 2, EPI, false, kBigTileMfma>(p, s, main_wgs);
     }
     if (rc != kOk || sch.rest_split <= 1) return rc;
-    return launch_gemm16_rest<T, EPI>(p, main_wgs, tiles - main_wgs, sch.rest_split, s);
+    return launch_gemm16_rest<T, EPI>(p, main_wgs, tiles - main_wgs, sch.rest_split, ws, s);
   }
   const bool t128 = sch.tile == 128;
   if (sch.skinny) return launch_gemm16_skinny<T, EPI>(p, sch.split_k, false, s);
@@ -575,10 +650,9 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
     const int splits = sch.split_k;
     if (splits > 1) {
       const size_t mn = (size_t)p.M * p.N;
-      float* ws = static_cast<float*>(stream_workspace(s, mn * splits * sizeof(float)));
-      if (!ws) return kDeviceFailed;
       Gemm16Params q = p;
-      q.K = p.K / splits;
+      q.K = split_steps(p.K, splits) * G16_BK;
+      q.k_total = p.K;
       q.groups = splits;
       q.strideA = q.K;                       // split z reads A[:, z Ks ..) and B[z Ks .., :)
       q.strideB = (long)q.K * p.ldb;

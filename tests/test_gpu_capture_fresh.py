@@ -60,6 +60,7 @@ CASES = {
     "gemm_copy_of_a": lambda lane, rng: _gemm16(lane, rng, 5, 131, 777),       # K off 8: A would be copied
     "gemm_split": lambda lane, rng: _gemm16(lane, rng, 33, 1003, 1024),        # N off 8: only the K split needs scratch
     "gemm_strips": lambda lane, rng: _gemm16(lane, rng, 27, 3520, 5312),       # on the grid, 128-column strips
+    "gemm_tiles_split": lambda lane, rng: _gemm16(lane, rng, 150, 576, 5384),  # tiles, K in eight parts that are not equal
     "int8_copy_of_a": lambda lane, rng: _gemm8(lane, rng, 5, 131, 777, False),
     "int8_on_the_grid": lambda lane, rng: _gemm8(lane, rng, 16, 512, 1024, False),
     "fp8_split": lambda lane, rng: _gemm8(lane, rng, 5, 131, 1024, True),

@@ -312,3 +312,22 @@ def test_rest_round_in_pieces(lane, M, N, K, parts):
     assert np.array_equal(np.asarray(ops.gemm(a, b)).view(np.uint16), np.asarray(b16.from_float32(acc)).view(np.uint16))
     bias = rng.standard_normal(N).astype(np.float32)
     assert orc.max_rel_err(ops.fused_gemm(a, b, bias=bias, activation="relu"), np.maximum(ref + bias, 0.0)) <= 1e-5
+
+
+# K in parts that are not all of one length (K steps that the number of parts does not divide, a last step that is not
+# whole), on each tile, with the partial sums added in their order.  f32 sums: 1e-5.
+@pytest.mark.parametrize("M,N,K,tile", [(435, 1920, 12704, (128, 128)), (167, 1536, 11912, (128, 128)), (150, 576, 5384, (64, 64)),
+                                        (224, 10088, 5200, (128, 256)), (100, 1024, 6472, None), (20, 1000, 9032, None)])
+def test_uneven_k_splits(lane, M, N, K, tile):
+    from tessera_amd.schedule import select_gfx950_gemm_schedule
+    sch = select_gfx950_gemm_schedule(M, N, K, dtype="bf16")
+    assert sch.split_k > 1 and K % (64 * sch.split_k) and tile in (None, sch.workgroup_tile[:2])
+    rng = np.random.default_rng(M + 2 * N + 3 * K)
+    a = b16.from_float32((rng.standard_normal((M, K)) / np.sqrt(K)).astype(np.float32))
+    b = b16.from_float32(rng.standard_normal((K, N)).astype(np.float32))
+    ref = a.to_float32().astype(np.float64) @ b.to_float32().astype(np.float64)
+    acc = ops.gemm(a, b, out="f32")
+    assert orc.max_rel_err(acc, ref) <= 1e-5
+    assert np.array_equal(np.asarray(ops.gemm(a, b)).view(np.uint16), np.asarray(b16.from_float32(acc)).view(np.uint16))
+    bias = rng.standard_normal(N).astype(np.float32)
+    assert orc.max_rel_err(ops.fused_gemm(a, b, bias=bias, activation="relu"), np.maximum(ref + bias, 0.0)) <= 1e-5
