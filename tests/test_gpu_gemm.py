@@ -317,7 +317,8 @@ def test_rest_round_in_pieces(lane, M, N, K, parts):
 # K in parts that are not all of one length (K steps that the number of parts does not divide, a last step that is not
 # whole), on each tile, with the partial sums added in their order.  f32 sums: 1e-5.
 @pytest.mark.parametrize("M,N,K,tile", [(435, 1920, 12704, (128, 128)), (167, 1536, 11912, (128, 128)), (150, 576, 5384, (64, 64)),
-                                        (224, 10088, 5200, (128, 256)), (100, 1024, 6472, None), (20, 1000, 9032, None)])
+                                        (224, 10088, 5200, (128, 256)), (100, 1024, 6472, None), (20, 1000, 9032, None),
+                                        (104, 864, 2376, (64, 64)), (65, 2040, 1096, (64, 64))])
 def test_uneven_k_splits(lane, M, N, K, tile):
     from tessera_amd.schedule import select_gfx950_gemm_schedule
     sch = select_gfx950_gemm_schedule(M, N, K, dtype="bf16")
@@ -331,3 +332,17 @@ def test_uneven_k_splits(lane, M, N, K, tile):
     assert np.array_equal(np.asarray(ops.gemm(a, b)).view(np.uint16), np.asarray(b16.from_float32(acc)).view(np.uint16))
     bias = rng.standard_normal(N).astype(np.float32)
     assert orc.max_rel_err(ops.fused_gemm(a, b, bias=bias, activation="relu"), np.maximum(ref + bias, 0.0)) <= 1e-5
+
+
+# Stacks of products on 64 x 64 tiles where 128 x 128 ones would fill half of the compute units: either side of that line and
+# of the K where they stop, ragged edges.  f32 sums: 1e-5.
+@pytest.mark.parametrize("batch,M,N,K,tile", [(4, 128, 256, 64, 64), (3, 189, 200, 264, 64), (7, 130, 640, 640, 64), (7, 130, 640, 648, 128),
+                                              (16, 500, 264, 136, 128), (9, 300, 512, 72, 64)])
+def test_stacks_of_small_products(lane, batch, M, N, K, tile):
+    from tessera_amd.schedule import select_gfx950_gemm_schedule
+    assert select_gfx950_gemm_schedule(M, N, K, dtype="bf16", batch=batch).workgroup_tile[:2] == (tile, tile)
+    rng = np.random.default_rng(batch * M + N + K)
+    a = b16.from_float32((rng.standard_normal((batch, M, K)) / np.sqrt(K)).astype(np.float32))
+    b = b16.from_float32(rng.standard_normal((batch, K, N)).astype(np.float32))
+    ref = a.to_float32().astype(np.float64) @ b.to_float32().astype(np.float64)
+    assert orc.max_rel_err(ops.batched_gemm(a, b, out="f32"), ref) <= 1e-5
