@@ -468,8 +468,9 @@ int launch_gemm16_skinny(Gemm16Params p, int splits, bool loose, hipStream_t s) 
   const int d_vec = p.N % 4 == 0 && (p.ldd * dsz) % (4 * dsz) == 0 && aligned16(p.D) && (!p.bias || aligned16(p.bias));
   Gemm16Params q = p;
   if (a_copy) {
-    hipLaunchKernelGGL(pad_rows_kernel<uint16_t>, copy_grid(p.M, K8, 8, 1), copy_block(), 0, s, reinterpret_cast<uint16_t*>(ws),
-                       (long)K8, 0L, p.A, p.lda, 0L, p.M, p.K, p.M);
+    PadLaunch<uint16_t> pad(1);
+    pad.add({reinterpret_cast<uint16_t*>(ws), K8, 0, p.A, p.lda, 0, p.M, p.K, p.M});
+    pad.run(s);
     if (int rc = launch_status(); rc != kOk) return rc;
     q.A = reinterpret_cast<const uint16_t*>(ws);
     q.lda = K8;
@@ -517,19 +518,18 @@ int launch_gemm16_repitched(const Gemm16Params& p, hipStream_t s) {
   Gemm16Params q = p;
   q.K = K8;
   q.N = N8;
+  PadLaunch<uint16_t> pad(G);
   char* at = ws;
   if (!a_ok) {
     uint16_t* a2 = reinterpret_cast<uint16_t*>(at);
     at += a_bytes;
-    hipLaunchKernelGGL(pad_rows_kernel<uint16_t>, copy_grid(p.M, K8, 8, G), copy_block(), 0, s, a2, (long)K8,
-                       (long)p.M * K8, p.A, p.lda, p.strideA, p.M, p.K, p.M);
+    pad.add({a2, K8, (long)p.M * K8, p.A, p.lda, p.strideA, p.M, p.K, p.M});
     q.A = a2; q.lda = K8; q.strideA = (long)p.M * K8;
   }
   if (!b_ok) {
     uint16_t* b2 = reinterpret_cast<uint16_t*>(at);
     at += b_bytes;
-    hipLaunchKernelGGL(pad_rows_kernel<uint16_t>, copy_grid(K8, N8, 8, G), copy_block(), 0, s, b2, (long)N8,
-                       (long)K8 * N8, p.B, p.ldb, p.strideB, p.K, p.N, K8);
+    pad.add({b2, N8, (long)K8 * N8, p.B, p.ldb, p.strideB, p.K, p.N, K8});
     q.B = b2; q.ldb = N8; q.strideB = (long)K8 * N8;
   }
   void* d2 = nullptr;
@@ -540,10 +540,10 @@ int launch_gemm16_repitched(const Gemm16Params& p, hipStream_t s) {
   }
   if (!bias_ok) {
     float* bias2 = reinterpret_cast<float*>(at);
-    hipLaunchKernelGGL(pad_rows_kernel<float>, copy_grid(1, N8, 4, 1), copy_block(), 0, s, bias2, (long)N8, (long)N8,
-                       p.bias, (long)p.N, (long)p.N, 1, p.N, 1);
+    pad.add_vector(bias2, N8, p.bias, p.N);
     q.bias = bias2;
   }
+  pad.run(s);
   int rc = launch_status();
   if (rc == kOk) rc = launch_gemm16<T, EPI>(q, s);
   if (rc == kOk && !d_ok) {

@@ -50,16 +50,15 @@ int gemm8_repitched(const Gemm8Params& p, hipStream_t s) {
   Gemm8Params q = p;
   q.K = K16;
   q.N = N16;
+  PadLaunch<uint8_t> pad(1);
   char* at = ws;
   if (!a_ok) {
-    hipLaunchKernelGGL(pad_rows_kernel<uint8_t>, copy_grid(p.M, K16, 16, 1), copy_block(), 0, s, reinterpret_cast<uint8_t*>(at),
-                       (long)K16, 0L, p.A, (long)p.K, 0L, p.M, p.K, p.M);
+    pad.add({reinterpret_cast<uint8_t*>(at), K16, 0, p.A, p.K, 0, p.M, p.K, p.M});
     q.A = reinterpret_cast<const uint8_t*>(at);
     at += a_bytes;
   }
   if (!b_ok) {
-    hipLaunchKernelGGL(pad_rows_kernel<uint8_t>, copy_grid(K16, N16, 16, 1), copy_block(), 0, s, reinterpret_cast<uint8_t*>(at),
-                       (long)N16, 0L, p.B, (long)p.N, 0L, p.K, p.N, K16);
+    pad.add({reinterpret_cast<uint8_t*>(at), N16, 0, p.B, p.N, 0, p.K, p.N, K16});
     q.B = reinterpret_cast<const uint8_t*>(at);
     at += b_bytes;
   }
@@ -68,10 +67,10 @@ int gemm8_repitched(const Gemm8Params& p, hipStream_t s) {
   int32_t* acc2 = nullptr;
   if (!acc_ok) { acc2 = reinterpret_cast<int32_t*>(at); q.acc_out = acc2; at += acc_bytes; }
   if (!cs_ok) {
-    hipLaunchKernelGGL(pad_rows_kernel<float>, copy_grid(1, N16, 4, 1), copy_block(), 0, s, reinterpret_cast<float*>(at),
-                       (long)N16, 0L, p.col_scale, (long)p.N, 0L, 1, p.N, 1);
+    pad.add_vector(reinterpret_cast<float*>(at), N16, p.col_scale, p.N);
     q.col_scale = reinterpret_cast<const float*>(at);
   }
+  pad.run(s);
   int rc = launch_status();
   if (rc == kOk) rc = gemm8_dev<T, EPI>(q, s);
   if (rc == kOk && !d_ok) {
@@ -145,8 +144,9 @@ int gemm8_skinny(const Gemm8Params& p, int splits, bool loose, hipStream_t s) {
   Gemm8Params q = p;
   int lda = p.K;
   if (a_copy) {
-    hipLaunchKernelGGL(pad_rows_kernel<uint8_t>, copy_grid(p.M, K16, 16, 1), copy_block(), 0, s, reinterpret_cast<uint8_t*>(ws),
-                       (long)K16, 0L, p.A, (long)p.K, 0L, p.M, p.K, p.M);
+    PadLaunch<uint8_t> pad(1);
+    pad.add({reinterpret_cast<uint8_t*>(ws), K16, 0, p.A, p.K, 0, p.M, p.K, p.M});
+    pad.run(s);
     if (int rc = launch_status(); rc != kOk) return rc;
     q.A = reinterpret_cast<const uint8_t*>(ws);
     lda = K16;

@@ -18,29 +18,45 @@ static_assert(alignof(LooseChunk<uint8_t>) == 1 && alignof(LooseChunk<uint16_t>)
 constexpr int kCopyRowsPerBlock = 4;
 
 // dst[b][r][c] (rows_dst x ld_dst, 16-byte aligned) = src[b][r][c] inside rows_src x cols_src, else 0.
+template <class E> struct PadJob {
+  E* dst;
+  long ld_dst, stride_dst;
+  const E* src;
+  long ld_src, stride_src;
+  int rows_src, cols_src, rows_dst;
+  unsigned bx = 0, by = 0, end = 0;    // filled in by PadLaunch: blocks along a row and over the rows, and the launch's blocks up to here
+};
+// Up to three matrices in one launch (the operands of a product and a vector that goes with them, as bytes of E): each launch
+// more costs a small product 3 to 5 us (int8 1017 x 734 x 2905 45.6 us in a launch each, 35.0 in one).  The jobs' blocks lie
+// one after the other along blockIdx.x: on a common grid of the widest and the tallest job most blocks were empty (int8 74 x
+// 557 x 11705 65 us, 34 so).
+template <class E> struct PadJobs { PadJob<E> job[3]; };
 template <class E>
-__global__ void __launch_bounds__(64 * kCopyRowsPerBlock)
-pad_rows_kernel(E* __restrict__ dst, long ld_dst, long stride_dst, const E* __restrict__ src, long ld_src,
-                long stride_src, int rows_src, int cols_src, int rows_dst) {
+__global__ void __launch_bounds__(64 * kCopyRowsPerBlock) pad_rows_kernel(const PadJobs<E> jobs) {
   constexpr int V = 16 / sizeof(E);
-  const int c0 = (blockIdx.x * 64 + threadIdx.x) * V;
-  if (c0 >= ld_dst) return;
-  const long b = blockIdx.z;
-  for (int r = blockIdx.y * kCopyRowsPerBlock + threadIdx.y; r < rows_dst; r += gridDim.y * kCopyRowsPerBlock) {
+  const unsigned id = blockIdx.x;
+  const int which = id < jobs.job[0].end ? 0 : id < jobs.job[1].end ? 1 : 2;
+  const PadJob<E>& j = jobs.job[which];
+  const unsigned at = id - (which ? jobs.job[which - 1].end : 0u), per = j.bx * j.by;
+  const long b = at / per;
+  const unsigned in = at - (unsigned)b * per;
+  const long c0 = ((long)(in % j.bx) * 64 + threadIdx.x) * V;
+  if (c0 >= j.ld_dst) return;
+  for (int r = (int)(in / j.bx) * kCopyRowsPerBlock + threadIdx.y; r < j.rows_dst; r += (int)j.by * kCopyRowsPerBlock) {
     uint4 out = make_uint4(0u, 0u, 0u, 0u);
-    if (r < rows_src && c0 < cols_src) {
-      const E* sp = src + b * stride_src + (long)r * ld_src + c0;
-      if (c0 + V <= cols_src) {
+    if (r < j.rows_src && c0 < j.cols_src) {
+      const E* sp = j.src + b * j.stride_src + (long)r * j.ld_src + c0;
+      if (c0 + V <= j.cols_src) {
         const u32x4 t = reinterpret_cast<const LooseChunk<E>*>(sp)->v;
         out = make_uint4(t[0], t[1], t[2], t[3]);
       } else {
         alignas(16) E v[V];
 #pragma unroll
-        for (int u = 0; u < V; ++u) v[u] = c0 + u < cols_src ? sp[u] : E(0);
+        for (int u = 0; u < V; ++u) v[u] = c0 + u < j.cols_src ? sp[u] : E(0);
         out = *reinterpret_cast<const uint4*>(v);
       }
     }
-    *reinterpret_cast<uint4*>(dst + b * stride_dst + (long)r * ld_dst + c0) = out;
+    *reinterpret_cast<uint4*>(j.dst + b * j.stride_dst + (long)r * j.ld_dst + c0) = out;
   }
 }
 // dst[b][r][c] = src[b][r][c] for r < rows, c < cols; src 16-byte aligned with pitch ld_src, dst any.
@@ -71,5 +87,33 @@ inline dim3 copy_grid(long rows, long ld, int vec, int batch) {
   return dim3((unsigned)bx, (unsigned)std::max<long>(1, std::min<long>(by, 16384)), (unsigned)batch);
 }
 inline dim3 copy_block() { return dim3(64, kCopyRowsPerBlock, 1); }
+
+// Collects the jobs of one launch.
+template <class E>
+class PadLaunch {
+ public:
+  explicit PadLaunch(int batch) : batch_(batch) {}
+  void add(PadJob<E> j) { push(j, batch_); }
+  // a vector of n 4-byte values, padded to n_dst (whose bytes are a multiple of 16)
+  void add_vector(float* dst, long n_dst, const float* src, int n) {
+    constexpr int per = 4 / sizeof(E);
+    push({reinterpret_cast<E*>(dst), n_dst * per, 0, reinterpret_cast<const E*>(src), (long)n * per, 0, 1, n * per, 1}, 1);
+  }
+  void run(hipStream_t s) const {
+    if (count_) hipLaunchKernelGGL(pad_rows_kernel<E>, dim3(jobs_.job[count_ - 1].end), copy_block(), 0, s, jobs_);
+  }
+
+ private:
+  void push(PadJob<E> j, int batch) {
+    // (at most 2^29 blocks a job: the sum stays inside a grid; the rows beyond are walked in strides)
+    const dim3 g = copy_grid(j.rows_dst, j.ld_dst, 16 / sizeof(E), batch);
+    j.bx = g.x;
+    j.by = std::max(1u, std::min(g.y, (unsigned)(1 << 29) / std::max(1u, g.x * (unsigned)batch)));
+    j.end = (count_ ? jobs_.job[count_ - 1].end : 0u) + j.bx * j.by * (unsigned)batch;
+    jobs_.job[count_++] = j;
+  }
+  PadJobs<E> jobs_{};
+  int batch_, count_ = 0;
+};
 
 }  // namespace tsr950

@@ -346,3 +346,17 @@ def test_stacks_of_small_products(lane, batch, M, N, K, tile):
     b = b16.from_float32(rng.standard_normal((batch, K, N)).astype(np.float32))
     ref = a.to_float32().astype(np.float64) @ b.to_float32().astype(np.float64)
     assert orc.max_rel_err(ops.batched_gemm(a, b, out="f32"), ref) <= 1e-5
+
+
+# Off the 16-byte grid in a stack: both operands of every product (and the bias's padded copy, where there is one) are
+# copied by one launch; wide over tall, tall over wide, a copy of one operand only.  f32 sums: 1e-5.
+@pytest.mark.parametrize("batch,M,N,K", [(3, 130, 203, 517), (5, 700, 17, 2051), (2, 33, 3001, 300), (2, 260, 1003, 512)])
+def test_off_grid_stacks(lane, batch, M, N, K):
+    rng = np.random.default_rng(batch + M + N + K)
+    a = b16.from_float32((rng.standard_normal((batch, M, K)) / np.sqrt(K)).astype(np.float32))
+    b = b16.from_float32(rng.standard_normal((batch, K, N)).astype(np.float32))
+    ref = a.to_float32().astype(np.float64) @ b.to_float32().astype(np.float64)
+    assert orc.max_rel_err(ops.batched_gemm(a, b, out="f32"), ref) <= 1e-5
+    bias = rng.standard_normal(N).astype(np.float32)
+    one = ops.fused_gemm(b16.from_bits(np.asarray(a)[0]), b16.from_bits(np.asarray(b)[0]), bias=bias, activation="relu")
+    assert orc.max_rel_err(one, np.maximum(ref[0] + bias, 0.0)) <= 1e-5
