@@ -54,9 +54,9 @@
  * weight, the router product is a GEMM like any other and may split K through the stream's
  * workspace).  Calls that use the workspace: products that split K (few rows, or few tiles under a long K),
  * attention that splits the keys (decode, and prefill with under 192 blocks of 256 query rows), routing,
- * combine and quantiser calls.  Two kinds use it where it is there and take a path without it
- * inside a capture on a stream that has none: single products of up to 64 rows whose N, K or pointers are off the
- * 16-byte grid, and attention of few query rows at head dimensions other than 64, 128 and 256 with 192 and
+ * combine and quantiser calls.  Three kinds use it where it is there and take a path without it
+ * inside a capture on a stream that has none: single 16-bit products (K then stays whole), single 8-bit products of up to
+ * 64 rows whose N, K or pointers are off the 16-byte grid, and attention of few query rows at head dimensions other than 64, 128 and 256 with 192 and
  * more (batch, head) pairs or under 1024 keys.  Any entry point (tessera_gfx950_probe is the cheapest) must have
  * been called once before the first capture: the first call initialises the device.
  */
