@@ -417,12 +417,15 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     // workgroups (27 x 3520 x 5312: 32.7 -> 13.7).  (The lines lie between those points, all but the last at 16 rows; 1.1e8 stands
     // above kStreamOnceBytes because 6144 x 8192, 1.007e8, gains nothing.  Over 16 weight shapes under 9 to 32 rows, several
     // matrices in turn, no choice is slower than the tiles by more than 1 %; a matrix alone in a loop: see kStreamOnceBytes.)
+    // (Under 16 rows against the tiles' equal parts only: in unequal ones they lose there, 7 x 1280 x 2584 on strips 7.1 us, on tiles in five
+    // parts 8.3, and win above, 19 x 896 x 9280 13.2 and 10.9.)
     if (M <= kSkinnyWideMaxM && N >= 128) {
+      const int parts = M < 16 ? equal : splits;
       const int wide = skinny_wide_splits(N, K);
       const long wgs = (long)ceil_div(N, 128) * wide;
       const double bytes = 2.0 * K * N;
       const bool streams = bytes >= 1.1e8 ? wgs >= 216 : bytes >= 2.4e7 && wgs >= 256 && wide > 2;
-      if ((streams && wgs <= 256 && K >= 2048 && K / wide >= 512) || (K >= 2048 && tiles * splits < 128 && wgs > 2 * tiles * splits))
+      if ((streams && wgs <= 256 && K >= 2048 && K / wide >= 512) || (K >= 2048 && tiles * parts < 128 && wgs > 2 * tiles * parts))
         return {128, wide, true};
     }
   }
