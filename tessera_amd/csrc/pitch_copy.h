@@ -3,19 +3,19 @@
 #pragma once
 #include <algorithm>
 #include "common.h"
+#include "pad_blocks.h"
 
 namespace tsr950 {
 
-// A thread moves one 16-byte chunk: blockIdx.x / threadIdx.x run along a row, blockIdx.y /
-// threadIdx.y over rows, blockIdx.z over the batch.  The side of any alignment is accessed with one
-// 16-byte instruction where the whole chunk is inside the row (global memory takes accesses off
+// A thread moves one 16-byte chunk: threadIdx.x runs along a row, threadIdx.y over rows; the copy back has its blocks along
+// a row, over rows and over the batch in blockIdx.x, y and z, the padding copy all of them along x (pad_blocks.h).  The side of
+// any alignment is accessed with one 16-byte instruction where the whole chunk is inside the row (global memory takes accesses off
 // their natural alignment), element by element at the row's end.
 // (the field is a plain vector type: a packed attribute is ignored on a field of class type, which would
 // leave the struct 16-byte aligned and the access free to assume it)
 template <class E> struct __attribute__((packed, aligned(sizeof(E)))) LooseChunk { u32x4 v; };
 static_assert(alignof(LooseChunk<uint8_t>) == 1 && alignof(LooseChunk<uint16_t>) == 2 && sizeof(LooseChunk<uint16_t>) == 16,
               "LooseChunk must carry its element's alignment");
-constexpr int kCopyRowsPerBlock = 4;
 
 // dst[b][r][c] (rows_dst x ld_dst, 16-byte aligned) = src[b][r][c] inside rows_src x cols_src, else 0.
 template <class E> struct PadJob {
@@ -24,39 +24,42 @@ template <class E> struct PadJob {
   const E* src;
   long ld_src, stride_src;
   int rows_src, cols_src, rows_dst;
-  unsigned bx = 0, by = 0, end = 0;    // filled in by PadLaunch: blocks along a row and over the rows, and the launch's blocks up to here
+  int batch = 0;                         // filled in by PadLaunch, as are its blocks and the launch's blocks up to here
+  PadBlocks blocks{};
+  unsigned end = 0;
 };
 // Up to three matrices in one launch (the operands of a product and a vector that goes with them, as bytes of E): each launch
 // more costs a small product 3 to 5 us (int8 1017 x 734 x 2905 45.6 us in a launch each, 35.0 in one).  The jobs' blocks lie
 // one after the other along blockIdx.x: on a common grid of the widest and the tallest job most blocks were empty (int8 74 x
 // 557 x 11705 65 us, 34 so).
-template <class E> struct PadJobs { PadJob<E> job[3]; };
+template <class E> struct PadJobs { PadJob<E> job[kPadJobs]; };
 template <class E>
 __global__ void __launch_bounds__(64 * kCopyRowsPerBlock) pad_rows_kernel(const PadJobs<E> jobs) {
   constexpr int V = 16 / sizeof(E);
   const unsigned id = blockIdx.x;
   const int which = id < jobs.job[0].end ? 0 : id < jobs.job[1].end ? 1 : 2;
   const PadJob<E>& j = jobs.job[which];
-  const unsigned at = id - (which ? jobs.job[which - 1].end : 0u), per = j.bx * j.by;
-  const long b = at / per;
-  const unsigned in = at - (unsigned)b * per;
-  const long c0 = ((long)(in % j.bx) * 64 + threadIdx.x) * V;
+  const unsigned at = id - (which ? jobs.job[which - 1].end : 0u), bx = j.blocks.bx, by = j.blocks.by, per = bx * by;
+  const unsigned b0 = at / per, in = at - b0 * per;
+  const long c0 = ((long)(in % bx) * 64 + threadIdx.x) * V;
   if (c0 >= j.ld_dst) return;
-  for (int r = (int)(in / j.bx) * kCopyRowsPerBlock + threadIdx.y; r < j.rows_dst; r += (int)j.by * kCopyRowsPerBlock) {
-    uint4 out = make_uint4(0u, 0u, 0u, 0u);
-    if (r < j.rows_src && c0 < j.cols_src) {
-      const E* sp = j.src + b * j.stride_src + (long)r * j.ld_src + c0;
-      if (c0 + V <= j.cols_src) {
-        const u32x4 t = reinterpret_cast<const LooseChunk<E>*>(sp)->v;
-        out = make_uint4(t[0], t[1], t[2], t[3]);
-      } else {
-        alignas(16) E v[V];
+  for (long b = b0; b < j.batch; b += j.blocks.bz) {
+    for (int r = (int)(in / bx) * kCopyRowsPerBlock + threadIdx.y; r < j.rows_dst; r += (int)by * kCopyRowsPerBlock) {
+      uint4 out = make_uint4(0u, 0u, 0u, 0u);
+      if (r < j.rows_src && c0 < j.cols_src) {
+        const E* sp = j.src + b * j.stride_src + (long)r * j.ld_src + c0;
+        if (c0 + V <= j.cols_src) {
+          const u32x4 t = reinterpret_cast<const LooseChunk<E>*>(sp)->v;
+          out = make_uint4(t[0], t[1], t[2], t[3]);
+        } else {
+          alignas(16) E v[V];
 #pragma unroll
-        for (int u = 0; u < V; ++u) v[u] = c0 + u < j.cols_src ? sp[u] : E(0);
-        out = *reinterpret_cast<const uint4*>(v);
+          for (int u = 0; u < V; ++u) v[u] = c0 + u < j.cols_src ? sp[u] : E(0);
+          out = *reinterpret_cast<const uint4*>(v);
+        }
       }
+      *reinterpret_cast<uint4*>(j.dst + b * j.stride_dst + (long)r * j.ld_dst + c0) = out;
     }
-    *reinterpret_cast<uint4*>(j.dst + b * j.stride_dst + (long)r * j.ld_dst + c0) = out;
   }
 }
 // dst[b][r][c] = src[b][r][c] for r < rows, c < cols; src 16-byte aligned with pitch ld_src, dst any.
@@ -105,11 +108,9 @@ class PadLaunch {
 
  private:
   void push(PadJob<E> j, int batch) {
-    // (at most 2^29 blocks a job: the sum stays inside a grid; the rows beyond are walked in strides)
-    const dim3 g = copy_grid(j.rows_dst, j.ld_dst, 16 / sizeof(E), batch);
-    j.bx = g.x;
-    j.by = std::max(1u, std::min(g.y, (unsigned)(1 << 29) / std::max(1u, g.x * (unsigned)batch)));
-    j.end = (count_ ? jobs_.job[count_ - 1].end : 0u) + j.bx * j.by * (unsigned)batch;
+    j.batch = batch;
+    j.blocks = pad_blocks(j.rows_dst, j.ld_dst, 16 / sizeof(E), batch);
+    j.end = (count_ ? jobs_.job[count_ - 1].end : 0u) + j.blocks.bx * j.blocks.by * j.blocks.bz;
     jobs_.job[count_++] = j;
   }
   PadJobs<E> jobs_{};

@@ -102,3 +102,42 @@ def test_few_rows_with_pitches_beyond_32_bit_offsets(lane, M, N, K):
         ref = sum(_f32(a[m, k0:k0 + (1 << 20)]).astype(np.float64) @ _f32(b[k0:k0 + (1 << 20), cols]).astype(np.float64)
                   for k0 in range(0, K, 1 << 20))
         assert np.abs(ref).max() < 2 ** 24 and np.array_equal(out[m, cols], ref), m
+
+
+# 4096 products of 65536 x 17 x 9, off the 16-byte grid: their padded copies have a row for each of 2^28 results, more than a launch
+# with a block for every four of them may have (2^26).  A repeats four products, B one: each result is one of four.
+# The first and last rows of the first, a middle and the last product; f32 sums: 1e-5.
+def test_off_grid_stack_of_more_rows_than_blocks(lane):
+    batch, M, N, K = 4096, 65536, 17, 9
+    rng = np.random.default_rng(33)
+    a, b = _bf16_bits(rng.standard_normal((4, M, K))), _bf16_bits(rng.standard_normal((K, N)))
+    lib, bufs = lane.load(), []
+
+    def repeated(block, bytes_):
+        buf = lane.DeviceBuffer(bytes_)
+        bufs.append(buf)
+        lane.check(lib.tessera_gfx950_memcpy_h2d(buf.ptr, block.ctypes.data, block.nbytes), "upload")
+        have = block.nbytes
+        while have < bytes_:
+            lane.check(lib.tessera_gfx950_memcpy_d2d_dev(buf.ptr + have, buf.ptr, min(have, bytes_ - have), None), "copy")
+            have *= 2
+        return buf
+
+    try:
+        # (B's block is 16 products, so that the copies move multiples of 16 bytes)
+        da, db = repeated(a, batch * M * K * 2), repeated(np.tile(b, (16, 1, 1)), batch * K * N * 2)
+        dd = lane.DeviceBuffer(batch * M * N * 4)
+        bufs.append(dd)
+        lane.check(lib.tessera_gfx950_batched_gemm_bf16_dev(da.ptr, db.ptr, dd.ptr, batch, M, N, K, None), "gemm")
+        lane.synchronize()
+        got = np.empty((2, 64, N), np.float32)
+        for p in (0, 2049, batch - 1):
+            for i, row in enumerate((0, M - 64)):
+                at = dd.ptr + ((p * M + row) * N) * 4
+                lane.check(lib.tessera_gfx950_memcpy_d2h(got[i].ctypes.data, at, got[i].nbytes), "download")
+            rows = np.concatenate([a[p % 4, :64], a[p % 4, -64:]])
+            ref = _f32(rows).astype(np.float64) @ _f32(b).astype(np.float64)
+            assert orc.max_rel_err(got.reshape(128, N), ref) <= 1e-5, p
+    finally:
+        for buf in bufs:
+            buf.close()

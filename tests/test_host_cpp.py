@@ -223,3 +223,29 @@ def test_every_device_allocation_can_take_the_pools_blocks():
             code = line.split("//")[0]
             if "hipMalloc(" in code or "hipMallocAsync(" in code:
                 assert f.name == "runtime.hip" and "pool_alloc_of(hipMalloc" in code, (f.name, i, line)
+
+
+def test_padding_copies_stay_inside_a_grid(tmp_path):
+    """The launch that pads a product's operands: under 2^26 blocks of 64 threads along x for any three matrices (HIP takes
+    fewer than 2^32 threads there; 65535 products of 4096 x 17 x 17 would be 67 million blocks with one for every four
+    rows), every row and product reached, and one block for each four rows where there is room."""
+    cases = [(4096, 24, 8, 65535), (24, 24, 8, 65535), (65536, 24, 8, 4096), (16384, 24, 8, 16384), (131, 784, 8, 1), (1, 16, 8, 1),
+             (2 ** 31 - 1, 2 ** 21, 8, 2 ** 31 - 1), (1, 2 ** 33, 16, 1), (5, 2 ** 31, 16, 3), (2048, 520, 8, 2 ** 26 + 1)]
+    out = _run(tmp_path, r"""
+#include "pad_blocks.h"
+#include <cstdio>
+#include <cstdlib>
+int main(int argc, char** argv) {
+  for (int i = 1; i + 3 < argc; i += 4) {
+    const tsr950::PadBlocks b = tsr950::pad_blocks(atol(argv[i]), atol(argv[i + 1]), atoi(argv[i + 2]), atol(argv[i + 3]));
+    std::printf("%u %u %u\n", b.bx, b.by, b.bz);
+  }
+}
+""", *[x for c in cases for x in c])
+    blocks = [tuple(map(int, line.split())) for line in out.splitlines()]
+    assert len(blocks) == len(cases)
+    for (rows, ld, vec, batch), (bx, by, bz) in zip(cases, blocks):
+        assert 3 * bx * by * bz < 2 ** 26
+        assert bx * 64 * vec >= ld and 1 <= by <= -(-rows // 4) and 1 <= bz <= batch      # (rows and products in strides)
+        if bx * -(-rows // 4) * batch <= 2 ** 24 and rows <= 65536:
+            assert by == -(-rows // 4) and bz == batch
