@@ -207,13 +207,13 @@ inline double est_few_rows_us(const FewRowTile& t, int M, int N, int K, int spli
   return t.launch + std::max(compute, stream) + sum;
 }
 
-// Second opinion for single products of 129 to about 3000 rows on fewer than 260 tiles of 256 x 256, where the estimates
-// above (fitted to matrices found in the caches, and without the 64 x 64 tile) were on average 5.6 % behind the best of
-// the forced schedules and up to 47 %: fitted (4 to 12 % rms) to 2033 timings of forced (tile, split) pairs over 260
-// products, weights streamed from memory.  A launch, then the larger of the K steps and of streaming B; 64- and 128-wide
-// tiles share a compute unit (the first at `step` a K step, each further one `more`), 256-wide ones come in rounds (a
-// step `step` on a quiet chip, `more` on a full one); a split adds its sum.
-// 100 products of 16 to 3000 rows with another schedule than before, by this or by uneven parts: 1.5 times as fast on average.
+// Second opinion for single products of more than 128 rows on fewer than 260 tiles of 256 x 256, where the estimates
+// above (fitted to matrices found in the caches, in equal K parts, and without the 64 x 64 tile) were on average 5.6 % behind the
+// best of the forced schedules and up to 47 %: fitted (4 to 12 % rms) to 2033 timings of forced (tile, split) pairs over 260
+// products of 129 to 3000 rows, weights streamed from memory.  A launch, then the larger of the K steps and of streaming B;
+// 64- and 128-wide tiles share a compute unit (the first at `step` a K step, each further one `more`), 256-wide ones come in
+// rounds (a step `step` on a quiet chip, `more` on a full one); a split adds its sum.  (The figures are a fit and not rates of the
+// part: 64-wide tiles hardly ever wait for B, hence their 14 TB/s.)
 struct MidTile { int tile_m, tile_n; double launch, step, more, tbs, sum, per_mega; };
 constexpr MidTile kMidTiles[4] = {{64, 64, 1.158, 0.4031, 0.1924, 14.09, 2.744, 1.677},
                                   {128, 128, 2.436, 0.5124, 0.5325, 2.914, 3.348, 1.262},
@@ -234,31 +234,38 @@ inline double est_mid_us(const MidTile& t, int M, int N, int K, int splits) {
   }
   return std::max(steps, stream) + (splits > 1 ? t.sum + (double)M * N * splits * t.per_mega * 1e-6 : 0.0);
 }
-// The schedule `first` or, where this estimate sees a tenth less time, its own choice.  (Over the 260 products 2.5 %
-// behind the best, and no product more than 5 % behind what it had before.)
-inline Gemm16Schedule second_opinion_mid(const Gemm16Schedule& first, int M, int N, int K) {
-  auto is = [&](const MidTile& t) { return t.tile_n == first.tile && t.tile_m == (first.tile_m ? first.tile_m : first.tile); };
-  double first_us = 0.0, best_us = 1e30, whole_us = 1e30;
-  Gemm16Schedule best = first, whole = first;           // whole: the best without a K split
+// The schedule `first` or, where this estimate sees a tenth less time, its own choice.  `equal` is what the first estimate chose
+// without K parts of unequal length, to which it was not fitted: where `first` has such parts, they are dropped unless this one, too,
+// sees them ahead, by a microsecond (1228 x 1112 x 1472 whole 27.8 us, in three parts 33.6; not for the best whole tile instead, whatever
+// the parts: 754 x 4376 x 11136 went from 96 us in three equal parts to 126 so, and takes 91 in four).  Over 592 products, each timed under its 20 schedules or so, the choice is 0.5 % behind the better of those
+// before and after unequal parts came in, on average, and 26 % at most.
+// Above 3000 rows, which it was not fitted to either, it is asked for unequal parts alone, and 5 % are enough, as the first
+// estimate is the more careful one with those (6782 x 768 x 13040 215 us whole, 135 in three parts).
+inline Gemm16Schedule second_opinion_mid(const Gemm16Schedule& first, const Gemm16Schedule& equal, int M, int N, int K) {
+  auto is = [](const MidTile& t, const Gemm16Schedule& s) { return t.tile_n == s.tile && t.tile_m == (s.tile_m ? s.tile_m : s.tile); };
+  auto unequal = [K](int splits) { return splits > 1 && K % (splits * G16_BK) != 0; };
+  const bool fitted = M <= 3000;
+  double first_us = 0.0, equal_us = 0.0, best_us = 1e30;
+  Gemm16Schedule best = first;
   for (const MidTile& t : kMidTiles) {
-    if (is(t)) first_us = est_mid_us(t, M, N, K, first.split_k);
+    if (is(t, first)) first_us = est_mid_us(t, M, N, K, first.split_k);
+    if (is(t, equal)) equal_us = est_mid_us(t, M, N, K, equal.split_k);
     if (t.tile_n == 64 && M > 512) continue;           // (not measured)
     for (int splits : {1, 2, 3, 4, 6, 8}) {
       if (splits > 1 && (!can_split(K, splits) || K / splits < 256)) continue;
+      if (!fitted && !unequal(splits)) continue;
       const double us = est_mid_us(t, M, N, K, splits);
-      const Gemm16Schedule sch = t.tile_m < t.tile_n ? Gemm16Schedule{256, splits, false, 1, 1, 128} : Gemm16Schedule{t.tile_n, splits, false};
-      if (us < best_us) { best_us = us; best = sch; }
-      if (splits == 1 && us < whole_us) { whole_us = us; whole = sch; }
+      if (us < best_us) {
+        best_us = us;
+        best = t.tile_m < t.tile_n ? Gemm16Schedule{256, splits, false, 1, 1, 128} : Gemm16Schedule{t.tile_n, splits, false};
+      }
     }
   }
   // (from a 256-wide tile to 128 x 128 ones, whose third and fourth on a unit cost more than the estimate has them, by a
   // fifth; to more parts by 2 us at least: 1052 x 704 x 1472 in four parts 14.9 us, whole 12.5)
-  const bool narrower = first.tile == 256 && best.tile < 256;
-  if (best_us < (narrower ? 0.8 : 0.9) * first_us && (best.split_k <= first.split_k || best_us + 2.0 < first_us)) return best;
-  // (a split into unequal parts that it sees nothing in is not taken: 1240 x 704 x 1368 whole / in two parts 13.1 / 14.8
-  // us, 2104 x 2560 x 4288 56 / 64)
-  if (first.split_k > 1 && K % (first.split_k * G16_BK) != 0 && whole_us < 1.05 * first_us) return whole;
-  return first;
+  const double margin = first.tile == 256 && best.tile < 256 ? 0.8 : fitted ? 0.9 : 0.95;
+  if (best_us < margin * first_us && (best.split_k <= first.split_k || best_us + 2.0 < first_us)) return best;
+  return fitted && unequal(first.split_k) && equal_us < first_us + 1.0 ? equal : first;
 }
 
 // Stacks of products whose 128 x 128 tiles leave half of the compute units idle go on 64 x 64 ones, while K is short: a
@@ -325,8 +332,7 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
   const long tiles256 = (long)ceil_div(M, 256) * ceil_div(N, 256) * batch;
   const long tiles128 = (long)ceil_div(M, 128) * ceil_div(N, 128) * batch;
   if (M > kWeightStreamMaxM && N >= 128) {
-    // the cheapest of: either tile, K in 1, 2, 3, 4 or 8 parts (a single product only; every
-    // part a whole number of K steps and at least 512 deep)
+    // the cheapest of: either tile, K in 1, 2, 3, 4 or 8 parts of at least 512 (a single product only)
     const int ksteps = ceil_div(K, G16_BK);
     Gemm16Schedule best{256, 1, false};
     double best_us = est_tiles256_us(tiles256, ksteps);
@@ -340,13 +346,32 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
       const double us = 1.06 * est_tiles128x256_us((long)ceil_div(M, 128) * ceil_div(N, 256) * batch, ksteps);
       if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, 1, 1, 128}; }
     }
+    Gemm16Schedule equal = best, uneven = best;
     if (batch == 1) {
+      double uneven_us = 1e30;
       for (int splits : {2, 3, 4, 8}) {
-        if (!can_split(K, splits) || K / splits < 512) continue;
+        const bool in_equal_parts = K % (splits * G16_BK) == 0;
+        if (!can_split(K, splits) || K / splits < (in_equal_parts || M <= 3000 ? 512 : 1024)) continue;
         const double sum_us = est_split_sum_us((long)M * N, splits);
-        consider(256, splits, est_tiles256_us(tiles256 * splits, split_steps(K, splits)) + sum_us);
-        consider(128, splits, est_tiles128_us(tiles128 * splits, split_steps(K, splits)) + sum_us);
+        const double us256 = est_tiles256_us(tiles256 * splits, split_steps(K, splits)) + sum_us;
+        const double us128 = est_tiles128_us(tiles128 * splits, split_steps(K, splits)) + sum_us;
+        if (in_equal_parts) {
+          consider(256, splits, us256);
+          consider(128, splits, us128);
+        } else {
+          if (us256 < uneven_us) { uneven_us = us256; uneven = {256, splits, false}; }
+          if (us128 < uneven_us) { uneven_us = us128; uneven = {128, splits, false}; }
+        }
       }
+      // The estimates were fitted without parts of unequal length.  Up to 3000 rows the second opinion below looks at these again;
+      // above, parts are at least 1024 deep (3077 x 640 x 1848 whole / in two parts 17.5 / 21.9 us) and have to win by half a
+      // microsecond, by 4 % against equal ones, and by 14 % against whole 128 x 256 tiles, whose estimate is 10 to 25 %
+      // high while they are one round of the chip (3170 x 1728 x 3520 whole / in two parts 46 / 56 us).  Over 380 products of
+      // more than 3000 rows, timed as those of the second opinion: 0.6 % behind on average, 15 % at most.
+      equal = best;
+      const bool take = M <= 3000 ? uneven_us < best_us
+                                  : (best.tile_m ? 1.14 : best.split_k > 1 ? 1.04 : 1.0) * uneven_us + 0.5 < best_us;
+      if (take) { best_us = uneven_us; best = uneven; }
     }
     // A tile count that is not a multiple of 256 leaves compute units idle in the last round: its tiles can be cut into
     // two or four pieces, or, where they are few and K is long, split along K among those units (one more launch and
@@ -373,8 +398,8 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
         if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, splits}; }
       }
     }
-    if (batch == 1 && M <= 3000 && tiles256 < 260 && best.rest_split == 1 && best.pieces == 1)
-      best = second_opinion_mid(best, M, N, K);
+    if (batch == 1 && tiles256 < 260 && best.rest_split == 1 && best.pieces == 1)
+      best = second_opinion_mid(best, equal, M, N, K);
     if (best.tile <= 128 && small_tiles_for_stack(tiles128, K, batch)) best.tile = 64;
     return best;
   }

@@ -347,6 +347,24 @@ def test_gemm_schedule_query_needs_no_device():
         sel(8, 8, 8, dtype="f64")
 
 
+def test_unequal_k_parts_only_where_they_were_timed_ahead():
+    """More than 128 rows, K in parts of unequal length or not: the schedule that was the fastest of the forced ones, or within
+    3 % of it (us: the other choice, a split into unequal parts or none).  In brackets: tile and parts."""
+    from tessera_amd.schedule import select_gfx950_gemm_schedule as sel
+    timed = {(3170, 1728, 3520): ((128, 256), 1),     # 46; 56 on 256 x 256 in two parts
+             (6506, 960, 4288): ((128, 256), 1),      # 56; 67
+             (3077, 640, 1848): ((128, 128), 1),      # 17.5; 21.9
+             (754, 4376, 11136): ((256, 256), 4),     # 91; 126 on 128 x 128 whole
+             (324, 7800, 11328): ((256, 256), 4),     # 92; 134
+             (1228, 1112, 1472): ((128, 128), 1),     # 27.8; 33.6
+             (6782, 768, 13040): ((256, 256), 3),     # 135; 215 whole
+             (4159, 640, 12160): ((128, 128), 3),     # 87; 129
+             (3015, 512, 6648): ((128, 128), 2)}      # 35; 51
+    for (m, n, k), (tile, parts) in timed.items():
+        sch = sel(m, n, k, dtype="bf16")
+        assert (sch.workgroup_tile[:2], sch.split_k) == (tile, parts), (m, n, k, sch.workgroup_tile, sch.split_k)
+
+
 def test_typed_descriptor_hook_validates_before_the_device():
     """The native-launcher hook refuses what its descriptor does not cover with RuntimeError,
     before any device call (nothing here needs a GPU)."""
