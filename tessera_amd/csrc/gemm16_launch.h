@@ -295,6 +295,24 @@ inline int skinny_loose_splits(int N, int K) {
   return best;
 }
 
+// A few rows (a B that streams from memory), K in `splits` parts of unequal length or in the `equal` ones that divide it.  Equal
+// ones where they are at least two thirds as many (21 x 10272 x 2816 in five / four parts 20.0 / 18.5 us), and short ones
+// that are 360 workgroups by themselves (27 x 10240 x 3264 in five / three 17.5 / 15.8; 16 x 8320 x 5952, three of 1984,
+// 22.2 / 27.0).  Whole instead of two parts that save less than their sum costs: 18 x 2176 x 1088 whole / in two 6.4 / 8.2, 12 x 640 x
+// 1344 7.2 / 8.6, 9 x 1728 x 1472 9.3 / 7.6; sooner over many columns, where a second workgroup on each unit streams B
+// faster (2 x 2952 x 1384 1.16 times as fast in two), and over more than 1100 off 128-byte lines (49 x 1128 x 1472 10.2 / 8.8, 17 x
+// 2120 x 1176 8.9 / 8.3).  Where 64-wide tiles fill the chip by themselves the lines count the other way (31 x
+// 13072 x 1368 13.3 / 14.1, 13 x 14704 x 1648 15.0, in three 16.8; 14 x 13504 x 1984 16.2, in three 13.6).
+// Drawn products of up to 64 rows, libraries with and without unequal parts in turn: with them 1.20 times as fast, 12 of 827 more than 3 %
+// slower.
+inline bool unequal_parts_pay(long tiles, int N, int K, int splits, int equal) {
+  const bool lines = N % 64 == 0;
+  if (3 * equal >= 2 * splits) return false;
+  if (equal > 1) return tiles * equal < 360 || K / equal >= 1536;
+  if (tiles >= 200) return K >= (lines ? 1200 : 2048);
+  return splits > 2 || K >= (!lines && tiles >= 18 ? 1160 : tiles < 24 ? 1480 : tiles < 40 ? 1400 : 1088);
+}
+
 inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
   if (batch == 1 && M <= kWeightStreamMaxM && N >= 128) {
     // Few rows under a very wide weight matrix (a vocabulary projection, a fused up projection):
@@ -429,29 +447,34 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
     // splits keep that under about 0.4 of the operand traffic
     splits = (int)std::min<long>(splits, std::max<long>(2, (long)K * (M + N) / (10L * M * N)));
     while (splits > 1 && !can_split(K, splits)) --splits;
-    // (equal parts where they are at least two thirds as many: 21 x 10272 x 2816 in 5 / 4 parts 20.0 / 18.5 us)
     int equal = splits;
     while (equal > 1 && K % (equal * G16_BK) != 0) --equal;
-    if (3 * equal >= 2 * splits) splits = equal;
+    if (splits > equal && !unequal_parts_pay(tiles, N, K, splits, equal)) splits = equal;
     // 9 to 32 rows: the streaming kernel on 128-column strips instead where it streams faster than the tiles: one
     // workgroup on every compute unit (16 x 8192 x 8192 31.4 -> 28.1 us, 4096 x 4096 12.7 -> 11.3, 8192 x 2048 10.4 ->
     // 9.4; two parts of a short K, 16320 x 2560, 18.2 against 17.3), or nearly so and a B that is read with the
     // non-temporal hint (7168 x 8192 29.4 -> 25.7, 14336 x 4096 28.5 -> 25.6).  Else the tiles: 7168 x 4096 15.4 against
     // 13.0, 8064 x 4096 (252 workgroups) 16.2 against 14.1, 6144 x 8192 23.0 against 21.2, 14656 x 2176 15.4 against 13.9; with K ranges
-    // under 512, 2048 x 7168, 11.5 against 12.2.  And where K has no even split that would give the tiles enough
-    // workgroups (27 x 3520 x 5312: 32.7 -> 13.7).  (The lines lie between those points, all but the last at 16 rows; 1.1e8 stands
+    // under 512, 2048 x 7168, 11.5 against 12.2.  And where the parts of K leave the tiles
+    // too few workgroups (9 x 3520 x 5312).  (The lines lie between those points, all but the last at 16 rows; 1.1e8 stands
     // above kStreamOnceBytes because 6144 x 8192, 1.007e8, gains nothing.  Over 16 weight shapes under 9 to 32 rows, several
     // matrices in turn, no choice is slower than the tiles by more than 1 %; a matrix alone in a loop: see kStreamOnceBytes.)
     // (Under 16 rows against the tiles' equal parts only: in unequal ones they lose there, 7 x 1280 x 2584 on strips 7.1 us, on tiles in five
-    // parts 8.3, and win above, 19 x 896 x 9280 13.2 and 10.9.)
+    // parts 8.3, and win above, 19 x 896 x 9280 13.2 and 10.9.  A large B, too, stays with the strips where its rows are off 128-byte
+    // lines, of which a 64-wide tile then reads one too many for every row, 30 x 6488 x 5384 21.0 us against 25.2, and from 9e7
+    // bytes on, 25 x 6720 x 10904 30.9 and 34.5, 17 x 4480 x 11680 23.0 and 24.9; on the lines tiles win, in parts for about two workgroups
+    // a unit, 20 x 3712 x 9528 17.9 and 15.5.)
     if (M <= kSkinnyWideMaxM && N >= 128) {
-      const int parts = M < 16 ? equal : splits;
       const int wide = skinny_wide_splits(N, K);
       const long wgs = (long)ceil_div(N, 128) * wide;
       const double bytes = 2.0 * K * N;
       const bool streams = bytes >= 1.1e8 ? wgs >= 216 : bytes >= 2.4e7 && wgs >= 256 && wide > 2;
-      if ((streams && wgs <= 256 && K >= 2048 && K / wide >= 512) || (K >= 2048 && tiles * parts < 128 && wgs > 2 * tiles * parts))
-        return {128, wide, true};
+      auto strips = [&](int parts) {
+        return (streams && wgs <= 256 && K >= 2048 && K / wide >= 512) || (K >= 2048 && tiles * parts < 128 && wgs > 2 * tiles * parts);
+      };
+      const bool equal_only = M < 16 || bytes >= 9e7 || (bytes >= 4.2e7 && N % 64 != 0);
+      if (strips(equal_only ? equal : splits)) return {128, wide, true};
+      if (splits > equal && strips(equal)) splits = std::max(equal, (int)std::min<long>(splits, 512 / tiles));
     }
   }
   return {t128 && !small_tiles_for_stack(tiles128, K, batch) ? 128 : 64, splits, false};

@@ -348,8 +348,7 @@ def test_gemm_schedule_query_needs_no_device():
 
 
 def test_unequal_k_parts_only_where_they_were_timed_ahead():
-    """More than 128 rows, K in parts of unequal length or not: the schedule that was the fastest of the forced ones, or within
-    3 % of it (us: the other choice, a split into unequal parts or none).  In brackets: tile and parts."""
+    """K in parts of unequal length or not: the schedule that was timed ahead of the other one (us of both beside it)."""
     from tessera_amd.schedule import select_gfx950_gemm_schedule as sel
     timed = {(3170, 1728, 3520): ((128, 256), 1),     # 46; 56 on 256 x 256 in two parts
              (6506, 960, 4288): ((128, 256), 1),      # 56; 67
@@ -359,7 +358,17 @@ def test_unequal_k_parts_only_where_they_were_timed_ahead():
              (1228, 1112, 1472): ((128, 128), 1),     # 27.8; 33.6
              (6782, 768, 13040): ((256, 256), 3),     # 135; 215 whole
              (4159, 640, 12160): ((128, 128), 3),     # 87; 129
-             (3015, 512, 6648): ((128, 128), 2)}      # 35; 51
+             (3015, 512, 6648): ((128, 128), 2),      # 35; 51
+             (18, 2176, 1088): ((64, 64), 1),         # 6.4; 8.2 in two parts
+             (12, 640, 1344): ((64, 64), 1),          # 7.2; 8.6
+             (9, 1728, 1472): ((64, 64), 2),          # 7.6; 9.3 whole
+             (2, 2952, 1384): ((64, 64), 2),          # in two parts 1.16 times as fast
+             (27, 10240, 3264): ((64, 64), 3),        # 15.8; 17.5 in five
+             (16, 8320, 5952): ((64, 64), 6),         # 22.2; 27.0 in three
+             (13, 14704, 1648): ((64, 64), 1),        # 15.0; 16.8 in three
+             (30, 6488, 5384): ((32, 128), 5),        # streaming strips 21.0; tiles in eight 25.2
+             (25, 6720, 10904): ((32, 128), 4),       # 30.9; 34.5
+             (20, 3712, 9528): ((64, 64), 8)}         # 15.5; 16.9 in fourteen, strips 17.9
     for (m, n, k), (tile, parts) in timed.items():
         sch = sel(m, n, k, dtype="bf16")
         assert (sch.workgroup_tile[:2], sch.split_k) == (tile, parts), (m, n, k, sch.workgroup_tile, sch.split_k)
