@@ -250,6 +250,11 @@ int tessera_gfx950_gemm_schedule(int M, int N, int K, int batch, int elem_bytes,
  * reference, whose schedule has no such step. */
 int tessera_gfx950_gemm_rest_split(int M, int N, int K, int batch, int* rest_tiles, int* rest_split);
 
+/* Which of the two it is: *pieces == *rest_split where the rest tiles are cut into pieces of the output (no partial
+ * sums, no workspace), 1 where they are split along K (*rest_split f32 partials for every value of a rest tile) or
+ * computed whole. */
+int tessera_gfx950_gemm_rest_pieces(int M, int N, int K, int batch, int* pieces);
+
 /* Kernel-only benchmark with resident, library-owned buffers: warm-up, `iters`
  * launches between HIP events, cross-checked against wall clock
  * (tessera_rocm_gemm.cpp:551-667).  *avg_ms = mean per-launch ms. */

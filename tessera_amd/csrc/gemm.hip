@@ -347,6 +347,13 @@ int tessera_gfx950_gemm_rest_split(int M, int N, int K, int batch, int* rest_til
   return kOk;
 }
 
+int tessera_gfx950_gemm_rest_pieces(int M, int N, int K, int batch, int* pieces) {
+  if (bad_dims(batch, M, N, K) || !pieces) return kBadShape;
+  const Gemm16Schedule sch = select_gemm16_schedule(M, N, K, batch);
+  *pieces = sch.tile == 256 && sch.split_k == 1 && !sch.skinny ? sch.pieces : 1;
+  return kOk;
+}
+
 int tessera_gfx950_gemm_bf16_bench(int M, int N, int K, int iters, double* avg_ms) {
   return bench_gemm16<BF16>(M, N, K, iters, 1, avg_ms);
 }

@@ -45,7 +45,8 @@ class Gfx950ScheduleDescriptor:
     raster_order: str = "xcd_banded"
     raster_group: int = 4
     rest_tiles: int = 0               # tiles beyond the last full round of 256 workgroups that are ...
-    rest_split_k: int = 1             # ... divided into this many parts, along K or in the output (1: none are)
+    rest_split_k: int = 1             # ... divided into this many parts (1: none are), along K, or ...
+    rest_pieces: int = 1              # ... where this is as many, in the output: no partial sums
 
     @property
     def mt(self) -> int:
@@ -69,6 +70,7 @@ class Gfx950ScheduleDescriptor:
             "schedule_split_k": self.split_k,
             "schedule_rest_tiles": self.rest_tiles,
             "schedule_rest_split_k": self.rest_split_k,
+            "schedule_rest_pieces": self.rest_pieces,
         }
 
     def cache_key(self) -> tuple:
@@ -89,10 +91,12 @@ def select_gfx950_gemm_schedule(m: int, n: int, k: int, *, dtype: str = "bf16", 
     _lane.check(_lane.load().tessera_gfx950_gemm_schedule(
         int(m), int(n), int(k), int(batch), nbytes, ctypes.byref(tm), ctypes.byref(tn), ctypes.byref(tk),
         ctypes.byref(sk)), "gemm_schedule")
-    rest_tiles, rest_split = ctypes.c_int(0), ctypes.c_int(1)
+    rest_tiles, rest_split, rest_pieces = ctypes.c_int(0), ctypes.c_int(1), ctypes.c_int(1)
     if nbytes == 2:
         _lane.check(_lane.load().tessera_gfx950_gemm_rest_split(
             int(m), int(n), int(k), int(batch), ctypes.byref(rest_tiles), ctypes.byref(rest_split)), "gemm_rest_split")
+        _lane.check(_lane.load().tessera_gfx950_gemm_rest_pieces(
+            int(m), int(n), int(k), int(batch), ctypes.byref(rest_pieces)), "gemm_rest_pieces")
     inst = _INSTRUCTION_TILE[name]
     if name in ("f16", "bf16") and max(tm.value, tn.value) == 256:
         inst = (16, 16, 32)       # the 256-wide tiles run v_mfma_f32_16x16x32 (less power per FLOP)
@@ -107,7 +111,7 @@ def select_gfx950_gemm_schedule(m: int, n: int, k: int, *, dtype: str = "bf16", 
                     if streaming else "A xor-swizzled 16B chunks; B natural [k][n] + transposing ds_read"),
         ownership="wave", vgpr_estimate=_VGPRS.get((tm.value, tn.value), 508), split_k=sk.value,
         source="tessera_gfx950_gemm_schedule (the launcher's own decision)",
-        rest_tiles=rest_tiles.value, rest_split_k=rest_split.value)
+        rest_tiles=rest_tiles.value, rest_split_k=rest_split.value, rest_pieces=rest_pieces.value)
 
 
 __all__ = ["Gfx950ScheduleDescriptor", "select_gfx950_gemm_schedule"]

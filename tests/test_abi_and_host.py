@@ -347,6 +347,19 @@ def test_gemm_schedule_query_needs_no_device():
         sel(8, 8, 8, dtype="f64")
 
 
+def test_schedule_tells_pieces_from_k_parts():
+    """The tiles beyond the last full round in four K parts (partial sums) or in four pieces of the output (none): the
+    queries, the attributes and the cache key differ."""
+    import dataclasses
+    from tessera_amd.schedule import select_gfx950_gemm_schedule as sel
+    pieces, parts, whole = sel(4100, 4104, 1096), sel(4096, 4104, 8192), sel(4096, 4096, 1096)
+    assert (pieces.rest_tiles, pieces.rest_split_k, pieces.rest_pieces) == (33, 4, 4)
+    assert parts.rest_tiles == 16 and parts.rest_split_k > 1 and parts.rest_pieces == 1
+    assert (whole.rest_tiles, whole.rest_split_k, whole.rest_pieces) == (0, 1, 1)
+    same = dataclasses.replace(pieces, rest_pieces=1)
+    assert same.cache_key() != pieces.cache_key() and pieces.target_ir_attrs()["schedule_rest_pieces"] == 4
+
+
 def test_unequal_k_parts_only_where_they_were_timed_ahead():
     """K in parts of unequal length or not: the schedule that was timed ahead of the other one (us of both beside it)."""
     from tessera_amd.schedule import select_gfx950_gemm_schedule as sel

@@ -302,7 +302,7 @@ def test_bad_shapes_rejected(lane):
 def test_rest_round_in_pieces(lane, M, N, K, parts):
     from tessera_amd.schedule import select_gfx950_gemm_schedule
     sch = select_gfx950_gemm_schedule(M, N, K, dtype="bf16")
-    assert sch.workgroup_tile[:2] == (256, 256) and sch.split_k == 1 and sch.rest_split_k == parts
+    assert sch.workgroup_tile[:2] == (256, 256) and sch.split_k == 1 and sch.rest_split_k == sch.rest_pieces == parts
     rng = np.random.default_rng(M + 2 * N + 3 * K)
     a = b16.from_float32((rng.standard_normal((M, K)) / np.sqrt(K)).astype(np.float32))
     b = b16.from_float32(rng.standard_normal((K, N)).astype(np.float32))
