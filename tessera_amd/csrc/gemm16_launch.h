@@ -405,14 +405,16 @@ inline Gemm16Schedule select_gemm16_schedule(int M, int N, int K, int batch) {
         us *= margin;
         if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, 1, pieces}; }
       };
-      cut(2, main_us + est_tiles128x256_us(2 * rest, ksteps));
+      // (128 x 256 pieces beside whole tiles: no less than 0.72 us a K step, on idle compute units too: 49 tiles left at K = 4832 in
+      // two / four pieces or four K parts 196 / 192 / 185 us; 0.60 sent 7521 x 2368 x 4824 from 172 us in K parts to 195 in two pieces)
+      cut(2, main_us + std::max(est_tiles128x256_us(2 * rest, ksteps), 7.0 + 0.72 * ksteps));
       // (128 x 128 pieces, alone on their compute units: 0.52 us a K step up to 64 of them, 0.65 from 192 on)
       if (rest <= 64) cut(4, main_us + 5.0 + ksteps * (0.52 + 0.13 * std::min(1.0, std::max(0.0, (4 * rest - 64) / 128.0))));
       for (int splits : {2, 3, 4, 6, 8, 12, 16}) {
         const int per = ceil_div(ksteps, splits);
         if (rest * splits > 256 || per < 2 || (long)per * (splits - 1) >= ksteps) continue;
-        const double us = main_us + 8.0 + est_tiles256_us(rest * splits, per) +
-                          est_split_sum_us(rest * 65536L, splits);
+        // (the partials of a few tiles are summed from the caches)
+        const double us = main_us + 8.0 + est_tiles256_us(rest * splits, per) + 0.9 * est_split_sum_us(rest * 65536L, splits);
         if (us < best_us) { best_us = us; best = Gemm16Schedule{256, 1, false, splits}; }
       }
     }

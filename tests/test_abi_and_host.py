@@ -360,6 +360,20 @@ def test_schedule_tells_pieces_from_k_parts():
     assert same.cache_key() != pieces.cache_key() and pieces.target_ir_attrs()["schedule_rest_pieces"] == 4
 
 
+def test_rest_tiles_in_pieces_or_k_parts_as_timed():
+    """The tiles beyond the last full round: K parts of a long K under 33 to 70 of them, pieces otherwise (us of both beside it)."""
+    from tessera_amd.schedule import select_gfx950_gemm_schedule as sel
+    timed = {(7521, 2368, 4824): (4, 1),        # 172 in four K parts; 195 in two pieces
+             (3438, 5760, 5880): (3, 1),        # 220; 239
+             (3176, 6656, 6256): (3, 1),        # 226; 242
+             (1531, 14336, 4096): (2, 2),       # 177 in two pieces; 206 in three K parts
+             (4655, 3520, 2560): (4, 4),        # 84 in four pieces; 88 in four K parts
+             (4159, 4416, 2112): (4, 4)}
+    for (m, n, k), want in timed.items():
+        sch = sel(m, n, k, dtype="bf16")
+        assert sch.workgroup_tile[:2] == (256, 256) and (sch.rest_split_k, sch.rest_pieces) == want, (m, n, k, sch)
+
+
 def test_unequal_k_parts_only_where_they_were_timed_ahead():
     """K in parts of unequal length or not: the schedule that was timed ahead of the other one (us of both beside it)."""
     from tessera_amd.schedule import select_gfx950_gemm_schedule as sel

@@ -294,6 +294,28 @@ def test_bad_shapes_rejected(lane):
     assert lib.tessera_gfx950_gemm_bf16(z.ctypes.data, z.ctypes.data, d.ctypes.data, 4, -1, 4) == 1
 
 
+# ... and where these are K parts (partial sums in the workspace, a second and a third launch), not pieces of the output: row tiles
+# and columns that end inside a tile, K steps that the parts do not divide, a last part of a single step, a K that ends
+# inside a step, the fused epilogue on both kinds of tile.  f32 sums: 1e-5; silu, whose slope is at most 1.1, 2e-5.
+@pytest.mark.parametrize("M,N,K,parts", [(1155, 13160, 2776, 8), (3206, 4912, 2840, 12), (1787, 9424, 3120, 6), (1426, 10760, 2912, 16),
+                                         (1035, 15016, 4776, 4)])
+def test_rest_round_in_unequal_k_parts(lane, M, N, K, parts):
+    from tessera_amd.schedule import select_gfx950_gemm_schedule
+    sch = select_gfx950_gemm_schedule(M, N, K, dtype="bf16")
+    assert sch.workgroup_tile[:2] == (256, 256) and sch.split_k == 1 and (sch.rest_split_k, sch.rest_pieces) == (parts, 1)
+    assert -(-K // 64) % parts and K % 64
+    rng = np.random.default_rng(M + 2 * N + 3 * K)
+    a = b16.from_float32((rng.standard_normal((M, K)) / np.sqrt(K)).astype(np.float32))
+    b = b16.from_float32(rng.standard_normal((K, N)).astype(np.float32))
+    ref = a.to_float32().astype(np.float64) @ b.to_float32().astype(np.float64)
+    acc = ops.gemm(a, b, out="f32")
+    assert orc.max_rel_err(acc, ref) <= 1e-5
+    assert np.array_equal(np.asarray(ops.gemm(a, b)).view(np.uint16), np.asarray(b16.from_float32(acc)).view(np.uint16))
+    bias = rng.standard_normal(N).astype(np.float32)
+    x = ref + bias
+    assert orc.max_rel_err(ops.fused_gemm(a, b, bias=bias, activation="silu"), x / (1 + np.exp(-x))) <= 2e-5
+
+
 # The last, mostly empty round in pieces of the output (two 128 x 256 or four 128 x 128 to a tile): row and column edges
 # inside a piece, pieces that lie past an edge altogether, last row tiles of at most 64 and 128 rows among the whole
 # tiles, a number of rest tiles that is not a multiple of 8, a K that ends inside a step.  f32 sums: 1e-5.
