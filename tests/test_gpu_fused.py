@@ -158,20 +158,16 @@ def test_gemm_epilogue_keyword(lane, act):
         ops.gemm(a, b, epilogue={"residual": np.zeros((3, 70, 136), np.float32)})
 
 
-# The activations themselves, through the epilogue of each product kernel: a zero product leaves the bias, here every binary
-# order of magnitude of either sign, zeros, infinities and a NaN.  Bound: the exponent -x log2(e) is off by at most its own
+# The activations themselves: a zero product leaves the bias, here every binary order of magnitude of either sign, zeros,
+# infinities and a NaN.  Bound: the exponent -x log2(e) is off by at most its own
 # rounding (|x| 2^-24 log2(e), as a relative error of the exponential |x| 2^-24) and the exponential, the sum, the reciprocal
 # and the last two products by an ulp each; gelu's cubic argument by three more.  Below the smallest normal number of f32
 # the exponential is flushed: an absolute 1.2e-38 (times |x| where x is a factor).
-@pytest.mark.parametrize("M,N,K", [(2, 640, 64), (64, 640, 64), (128, 2048, 64), (2048, 4096, 64)])
-@pytest.mark.parametrize("act", ["silu", "gelu", "sigmoid", "tanh"])
-def test_activation_values(lane, M, N, K, act):
-    x = np.array([s * m * 2.0 ** e for s in (1, -1) for m in (1.0, 1.37, 1.83) for e in range(-40, 7)] + [0.0, 86.9, 87.6, 88.3, -86.9, -87.6, -88.3])
-    bias = np.zeros(N, np.float32)
-    bias[:x.size] = x
-    bias[-3:] = [np.inf, -np.inf, np.nan]
-    got = ops.fused_gemm(np.zeros((M, K), np.float16), np.zeros((K, N), np.float16), bias=bias, activation=act)
-    assert np.array_equal(got[0], got[-1], equal_nan=True)
+_PROBES = np.array([s * m * 2.0 ** e for s in (1, -1) for m in (1.0, 1.37, 1.83) for e in range(-40, 7)] + [0.0, 86.9, 87.6, 88.3, -86.9, -87.6, -88.3])
+
+
+def _check_activation(got, bias, act):
+    """One row of results for a bias whose last three values are inf, -inf and NaN."""
     v = bias[:-3].astype(np.float64)
     with np.errstate(over="ignore"):
         arg = 2 * 0.7978845608028654 * (v + 0.044715 * v ** 3) if act == "gelu" else 2 * v if act == "tanh" else v
@@ -180,7 +176,46 @@ def test_activation_values(lane, M, N, K, act):
         ref = {"silu": v * sig, "gelu": v * sig, "sigmoid": sig, "tanh": np.tanh(v)}[act]
     rel = (8 + np.abs(arg)) * 2.0 ** -24 * (2 if act == "gelu" else 1)
     size = 2 * np.maximum(np.abs(ref), sig) if act == "tanh" else np.abs(ref)      # tanh = 2 sig - 1 cancels
-    assert np.all(np.abs(got[0, :-3] - ref) <= rel * size + 1.2e-38 * np.maximum(1, np.abs(v)))
-    inf, ninf, nan = got[0, -3:]
+    assert np.all(np.abs(got[:-3] - ref) <= rel * size + 1.2e-38 * np.maximum(1, np.abs(v)))
+    inf, ninf, nan = got[-3:]
     assert np.isnan(nan) and inf == (np.inf if act in ("silu", "gelu") else 1.0)
     assert {"silu": np.isnan(ninf), "gelu": ninf == -np.inf, "sigmoid": ninf == 0, "tanh": ninf == -1}[act]
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 640, 64), (64, 640, 64), (128, 2048, 64), (2048, 4096, 64)])
+@pytest.mark.parametrize("act", ["silu", "gelu", "sigmoid", "tanh"])
+def test_activation_values(lane, M, N, K, act):
+    """On the 64 x 64 and the 128 x 128 tile."""
+    bias = np.zeros(N, np.float32)
+    bias[:_PROBES.size] = _PROBES
+    bias[-3:] = [np.inf, -np.inf, np.nan]
+    got = ops.fused_gemm(np.zeros((M, K), np.float16), np.zeros((K, N), np.float16), bias=bias, activation=act)
+    assert np.array_equal(got[0], got[-1], equal_nan=True)
+    _check_activation(got[0], bias, act)
+
+
+# ... and through the other epilogues: the streaming kernels whole and the sum over their K parts, the sum over the K parts of
+# tiles, the 256-wide tiles, two and four pieces of a rest tile, the sum over a rest tile's K parts.  The values stand in the first
+# and in the last columns; every row is the same.
+_EPILOGUES = {"stream": (2, 640, 512), "stream_parts": (2, 640, 2048), "strip_parts": (7, 1280, 2584), "tile_parts": (100, 1024, 6472),
+              "tile128x256": (1280, 5120, 2000), "tile256": (3800, 4040, 520), "pieces4": (1100, 15400, 840),
+              "pieces2": (1430, 13960, 1032), "rest_parts": (1155, 13160, 2776)}
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu", "sigmoid", "tanh"])
+@pytest.mark.parametrize("route", list(_EPILOGUES))
+def test_activation_values_in_every_epilogue(lane, route, act):
+    from tessera_amd.schedule import select_gfx950_gemm_schedule
+    M, N, K = _EPILOGUES[route]
+    sch = select_gfx950_gemm_schedule(M, N, K, dtype="f16")
+    tile, rest = sch.workgroup_tile[:2], (sch.rest_split_k, sch.rest_pieces)
+    assert {"stream": tile == (32, 64) and sch.split_k == 1, "stream_parts": tile == (32, 64) and sch.split_k > 1,
+            "strip_parts": tile == (32, 128) and sch.split_k > 1, "tile_parts": tile == (128, 128) and sch.split_k > 1,
+            "tile128x256": tile == (128, 256) and sch.split_k == 1, "tile256": tile == (256, 256) and rest == (1, 1) and sch.split_k == 1,
+            "pieces4": rest == (4, 4), "pieces2": rest == (2, 2), "rest_parts": rest[0] > 1 and rest[1] == 1}[route], sch
+    bias = np.zeros(N, np.float32)
+    bias[:_PROBES.size] = bias[-3 - _PROBES.size:-3] = _PROBES
+    bias[-3:] = [np.inf, -np.inf, np.nan]
+    got = ops.fused_gemm(np.zeros((M, K), np.float16), np.zeros((K, N), np.float16), bias=bias, activation=act)
+    assert np.array_equal(got, np.broadcast_to(got[0], got.shape), equal_nan=True)
+    _check_activation(got[0], bias, act)

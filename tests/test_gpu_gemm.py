@@ -109,9 +109,9 @@ def test_mid_size_schedules(lane, M, N, K, tile, split):
     assert orc.max_rel_err(fused, np.maximum(ref + bias, 0.0)) <= 1e-5
 
 
-# Tile counts a little over a multiple of 256: the tiles beyond the last full round are split along
-# K by a second launch and summed by a third (ragged edges, K that the splits do not divide, the
-# fused epilogue on both kinds of tile).
+# Tile counts a little over a multiple of 256: the tiles beyond the last full round are divided among the idle compute
+# units, 16 of them under K = 4096 in eight K parts, the other shapes' in pieces of the output (ragged edges, a K that ends inside
+# a step, the fused epilogue on both kinds of tile; each way by itself in the two tests below).
 @pytest.mark.parametrize("M,N,K", [(4096, 4104, 4096), (4352, 4096, 1000), (4350, 4088, 2056), (4100, 4360, 2000), (6140, 6136, 2048)])
 def test_rest_round_split_along_k(lane, M, N, K):
     from tessera_amd.schedule import select_gfx950_gemm_schedule
