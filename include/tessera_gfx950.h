@@ -52,13 +52,16 @@
  * use.  tessera_gfx950_moe_layer_bf16_dev takes a caller-owned workspace instead: given the
  * router logits it uses no memory of the library's and has neither restriction (given a router
  * weight, the router product is a GEMM like any other and may split K through the stream's
- * workspace).  Calls that use the workspace: products that split K (few rows, or few tiles under a long K),
+ * workspace).  Calls that need the workspace: 8-bit products that split K on tiles (tile_m 128 or 256 by the query below),
  * attention that splits the keys (decode, and prefill with under 192 blocks of 256 query rows), routing,
- * combine and quantiser calls.  Three kinds use it where it is there and take a path without it
- * inside a capture on a stream that has none: single 16-bit products (K then stays whole), single 8-bit products of up to
- * 64 rows whose N, K or pointers are off the 16-byte grid, and attention of few query rows at head dimensions other than 64, 128 and 256 with 192 and
- * more (batch, head) pairs or under 1024 keys.  Any entry point (tessera_gfx950_probe is the cheapest) must have
- * been called once before the first capture: the first call initialises the device.
+ * combine and quantiser calls; recorded without one that is large enough they fail.  Three kinds use it where it
+ * is there and large enough and take a path without it inside a capture where it is not, on a stream that has run
+ * nothing eagerly as on one whose eager calls were smaller: single 16-bit products, single 8-bit products on the streaming kernel
+ * (up to 64 rows, tile_m 32 or 64), and attention of few query rows at head dimensions other than 64, 128 and 256 with 192 and
+ * more (batch, head) pairs or under 1024 keys.  The products then keep K whole: the f32 sums are added in another order
+ * than the eager call's, and few rows or few tiles under a long K take up to six times as long (64 x 896 x 14000: 82 us for
+ * 14).  Nothing reports it; the eager call with arguments as large avoids it.  Any entry point
+ * (tessera_gfx950_probe is the cheapest) must have been called once before the first capture: the first call initialises the device.
  */
 #ifndef TESSERA_GFX950_H
 #define TESSERA_GFX950_H

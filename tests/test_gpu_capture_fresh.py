@@ -59,7 +59,8 @@ def _attention(lane, rng, B, Hq, Hkv, Sq, Sk, D):
 CASES = {
     "gemm_copy_of_a": lambda lane, rng: _gemm16(lane, rng, 5, 131, 777),       # K off 8: A would be copied
     "gemm_split": lambda lane, rng: _gemm16(lane, rng, 33, 1003, 1024),        # N off 8: only the K split needs scratch
-    "gemm_strips": lambda lane, rng: _gemm16(lane, rng, 27, 3520, 5312),       # on the grid, 128-column strips
+    "gemm_strips": lambda lane, rng: _gemm16(lane, rng, 27, 3520, 5312),       # on the grid, few rows on tiles
+    "gemm_strips_9": lambda lane, rng: _gemm16(lane, rng, 9, 3520, 5312),      # on the grid, 128-column strips
     "gemm_tiles_split": lambda lane, rng: _gemm16(lane, rng, 150, 576, 5384),  # tiles, K in eight parts that are not equal
     "int8_copy_of_a": lambda lane, rng: _gemm8(lane, rng, 5, 131, 777, False),
     "int8_on_the_grid": lambda lane, rng: _gemm8(lane, rng, 16, 512, 1024, False),
@@ -71,12 +72,32 @@ CASES = {
 
 @pytest.mark.parametrize("case", CASES)
 def test_records_without_a_workspace(lane, hip, case):
+    _record_and_replay(lane, hip, *CASES[case](lane, np.random.default_rng(len(case))))
+
+
+@pytest.mark.parametrize("case", ["gemm_strips_9", "gemm_tiles_split"])
+def test_records_beside_a_smaller_workspace(lane, hip, case):
+    """The stream has the workspace of a smaller eager call (1 MiB, the smallest; these need 1.1 and 2.8 MB)."""
+    from tessera_amd.schedule import select_gfx950_gemm_schedule as sel
+    assert sel(9, 3520, 5312).workgroup_tile == (32, 128, 32) and 9 * 3520 * 4 * sel(9, 3520, 5312).split_k > 1 << 20
+    assert sel(150, 576, 5384).workgroup_tile[0] == 64 and 150 * 576 * 4 * sel(150, 576, 5384).split_k > 1 << 20
+    rng = np.random.default_rng(len(case))
+    small, run_small, *_ = _gemm16(lane, rng, 5, 131, 777)
+    try:
+        _record_and_replay(lane, hip, *CASES[case](lane, rng), before=run_small)
+    finally:
+        for x in small:
+            x.close()
+
+
+def _record_and_replay(lane, hip, d, enqueue, ref, dtype, tol, before=None):
     lane.load().tessera_gfx950_probe()
-    d, enqueue, ref, dtype, tol = CASES[case](lane, np.random.default_rng(len(case)))
     s, graph, exe = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
     assert hip.hipStreamCreate(ctypes.byref(s)) == 0
     lane.load().tessera_gfx950_stream_release(s)               # (a handle that an earlier test's stream had)
     try:
+        if before:
+            assert before(s) == 0 and hip.hipStreamSynchronize(s) == 0
         assert hip.hipStreamBeginCapture(s, 0) == 0
         rc = enqueue(s)
         ended = hip.hipStreamEndCapture(s, ctypes.byref(graph))
