@@ -303,11 +303,14 @@ inline int skinny_loose_splits(int N, int K) {
 // faster (2 x 2952 x 1384 1.16 times as fast in two), and over more than 1100 off 128-byte lines (49 x 1128 x 1472 10.2 / 8.8, 17 x
 // 2120 x 1176 8.9 / 8.3).  Where 64-wide tiles fill the chip by themselves the lines count the other way (31 x
 // 13072 x 1368 13.3 / 14.1, 13 x 14704 x 1648 15.0, in three 16.8; 14 x 13504 x 1984 16.2, in three 13.6).
+// Under 128 columns (router logits) always in parts: in a layer such a product's operands come from memory (762 x 32 x 1344 in front
+// of its experts 14 us whole, 11 in two parts; 2000 times the same one 7.3 and 8.6).
 // Drawn products of up to 64 rows, libraries with and without unequal parts in turn: with them 1.20 times as fast, 12 of 827 more than 3 %
 // slower.
 inline bool unequal_parts_pay(long tiles, int N, int K, int splits, int equal) {
   const bool lines = N % 64 == 0;
   if (3 * equal >= 2 * splits) return false;
+  if (N < 128) return true;
   if (equal > 1) return tiles * equal < 360 || K / equal >= 1536;
   if (tiles >= 200) return K >= (lines ? 1200 : 2048);
   return splits > 2 || K >= (!lines && tiles >= 18 ? 1160 : tiles < 24 ? 1480 : tiles < 40 ? 1400 : 1088);

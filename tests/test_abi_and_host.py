@@ -389,6 +389,7 @@ def test_unequal_k_parts_only_where_they_were_timed_ahead():
              (18, 2176, 1088): ((64, 64), 1),         # 6.4; 8.2 in two parts
              (12, 640, 1344): ((64, 64), 1),          # 7.2; 8.6
              (9, 1728, 1472): ((64, 64), 2),          # 7.6; 9.3 whole
+             (762, 32, 1344): ((64, 64), 2),          # 11; 14 whole, in front of an expert layer
              (2, 2952, 1384): ((64, 64), 2),          # in two parts 1.16 times as fast
              (27, 10240, 3264): ((64, 64), 3),        # 15.8; 17.5 in five
              (16, 8320, 5952): ((64, 64), 6),         # 22.2; 27.0 in three
