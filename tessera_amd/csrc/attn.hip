@@ -98,7 +98,7 @@ int launch_flash_for(const FlashParams& p, bool ext, hipStream_t s) {
 
 // Few query rows per KV head (decode, short speculative steps): the rows of a whole GQA group
 // share one MFMA tile and the key range is split over workgroups (flash_decode.h).  kNoScratch: padded head
-// dimensions, whose key splits found no workspace (a capture on a stream that has none); the general
+// dimensions, whose key splits found no workspace of their size (a capture on a stream with none or a smaller one); the general
 // kernel then serves them, which needs none from 192 blocks on and under 1024 keys.
 template <class T, int DP, int NQ, bool PAD, bool NT>
 int launch_decode_as(const FlashParams& p, hipStream_t s) {

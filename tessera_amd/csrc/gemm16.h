@@ -17,9 +17,10 @@
 // What follows describes the 32-wide step; the 16-wide one (kstep16) differs in how the
 // fragment reads are dealt out, see there.
 //
-// The tile body is a device function (gemm16_tile); the grouped kernel also holds a
-// 64 x BN instantiation of it with the four waves side by side along the columns, used
-// for a group's last row tile when at most 64 rows are left.
+// The tile body is a device function (gemm16_tile); the grouped kernel also holds shorter
+// instantiations of it for a group's last row tile: 128 x BN for at most 128 rows, and for at
+// most 64 rows one with the four waves side by side along the columns, 64 x 2 BN where groups
+// average more than a tile of rows and 64 x BN where they do not.
 //
 // LDS staging (double buffered, one barrier per K step).
 //   A tile  [BM][64] 16-bit, 128-byte rows, 16-byte chunks XOR-swizzled by

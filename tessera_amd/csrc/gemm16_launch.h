@@ -502,7 +502,7 @@ int launch_gemm16_skinny_as(const Gemm16Params& p, int kps, int splits, float* p
 
 // The few-row streaming kernel with K in `splits` parts.  loose: see the kernel; A is then copied into
 // rows padded with zeros to a multiple of 8 where its own cannot be read 16 bytes at a time.  Without a
-// workspace (a capture on a stream that has none) K stays whole; a copy of A that has no room is kNoScratch.
+// workspace that is large enough (a capture on a stream with none or a smaller one) K stays whole; a copy of A without room is kNoScratch.
 template <class T, int EPI>
 int launch_gemm16_skinny(Gemm16Params p, int splits, bool loose, hipStream_t s) {
   const int cols = p.M <= kSkinnyMaxM && !loose ? 64 : 128;
@@ -683,7 +683,7 @@ int launch_gemm16(Gemm16Params p, hipStream_t s) {
     return launch_status();
   }
   Gemm16Schedule sch = select_gemm16_schedule(p.M, p.N, p.K, p.groups);
-  // The f32 partials of a K split lie in the stream's workspace; without one (a capture on a stream that has none, a full
+  // The f32 partials of a K split lie in the stream's workspace; without one of their size (a capture on a stream with none or a smaller one, a full
   // device) K stays whole on the same tiles.
   float* ws = nullptr;
   if (!sch.skinny && (sch.split_k > 1 || sch.rest_split > 1)) {

@@ -100,7 +100,7 @@ inline bool gemm8_worth_copies(int M, int N, int K) {
 // The few-row streaming kernel with K in `splits` parts (more than one: then the sum).  loose: rows of B on any boundary; A is
 // then copied into rows padded with zeros to a multiple of 16 where its own cannot be read 16 bytes at a time, and
 // fp8 products that it takes over from the one-thread-per-element kernel keep that kernel's f32 sums (WIDEN).
-// Without a workspace (a capture on a stream that has none) K stays whole; a copy of A that has no room is kNoScratch.
+// Without a workspace that is large enough (a capture on a stream with none or a smaller one) K stays whole; a copy of A without room is kNoScratch.
 // (8 waves and about 256 workgroups measured best for up to 32 rows: 4-wave workgroups, two per
 // compute unit, and 384 or 512 workgroups were level or slower on M = 1 ... 32 against 4096 ...
 // 28672 columns.  33 to 64 rows double the accumulators: 4 waves, one per SIMD.)
