@@ -236,9 +236,10 @@ inline double est_mid_us(const MidTile& t, int M, int N, int K, int splits) {
 }
 // The schedule `first` or, where this estimate sees a tenth less time, its own choice.  `equal` is what the first estimate chose
 // without K parts of unequal length, to which it was not fitted: where `first` has such parts, they are dropped unless this one, too,
-// sees them ahead, by a microsecond (1228 x 1112 x 1472 whole 27.8 us, in three parts 33.6; not for the best whole tile instead, whatever
-// the parts: 754 x 4376 x 11136 went from 96 us in three equal parts to 126 so, and takes 91 in four).  Over 592 products, each timed under its 20 schedules or so, the choice is 0.5 % behind the better of those
-// before and after unequal parts came in, on average, and 26 % at most.
+// sees them ahead (1228 x 1112 x 1472 whole 27.8 us, in three parts 33.6; 255 x 3648 x 9792 in four unequal parts 37.9, in three equal
+// ones 43.6; not for the best whole tile instead, whatever the parts: 754 x 4376 x 11136 went from 96 us in three equal parts to 126 so, and takes
+// 91 in four).  4800 drawn products of 129 rows and more, each timed under all its schedules: where this check changes the choice, 124
+// times, 6 % faster on average, 23 of them more than 3 % slower.  (Asked for a microsecond's gain: 130, 5 %, 30.)
 // Above 3000 rows, which it was not fitted to either, it is asked for unequal parts alone, and 5 % are enough, as the first
 // estimate is the more careful one with those (6782 x 768 x 13040 215 us whole, 135 in three parts).
 inline Gemm16Schedule second_opinion_mid(const Gemm16Schedule& first, const Gemm16Schedule& equal, int M, int N, int K) {
@@ -265,7 +266,7 @@ inline Gemm16Schedule second_opinion_mid(const Gemm16Schedule& first, const Gemm
   // fifth; to more parts by 2 us at least: 1052 x 704 x 1472 in four parts 14.9 us, whole 12.5)
   const double margin = first.tile == 256 && best.tile < 256 ? 0.8 : fitted ? 0.9 : 0.95;
   if (best_us < margin * first_us && (best.split_k <= first.split_k || best_us + 2.0 < first_us)) return best;
-  return fitted && unequal(first.split_k) && equal_us < first_us + 1.0 ? equal : first;
+  return fitted && unequal(first.split_k) && equal_us < first_us ? equal : first;
 }
 
 // Stacks of products whose 128 x 128 tiles leave half of the compute units idle go on 64 x 64 ones, while K is short: a

@@ -383,6 +383,7 @@ def test_unequal_k_parts_only_where_they_were_timed_ahead():
              (754, 4376, 11136): ((256, 256), 4),     # 91; 126 on 128 x 128 whole
              (324, 7800, 11328): ((256, 256), 4),     # 92; 134
              (1228, 1112, 1472): ((128, 128), 1),     # 27.8; 33.6
+             (255, 3648, 9792): ((128, 128), 4),      # 37.9; 43.6 in three
              (6782, 768, 13040): ((256, 256), 3),     # 135; 215 whole
              (4159, 640, 12160): ((128, 128), 3),     # 87; 129
              (3015, 512, 6648): ((128, 128), 2),      # 35; 51
