@@ -922,8 +922,9 @@ __global__ __launch_bounds__(256) void gemm16_rest_sum_kernel(const float* __res
 // above pays for with a pass over the partial tiles, 3.7 TB/s to write and less to read).  The pieces of a tile run on
 // one XCD.  A tile's last rows run on a shorter body where 128 or 64 rows are enough.  f32 results, whole tiles / K
 // split of the last round / pieces: 1531 x 14336 x 4096 with gelu 206 / 206 / 177 us, 1100 x 16384 x 4096 181 / 158 /
-// 143, 2048 x 12288 x 4096 184 / 186 / 171, 6140 x 6136 x 2048 161 / 158 / 143; bound by the pieces' LDS traffic
-// (1125 of 1300 cycles a K step of a 128 x 256 piece).
+// 143, 2048 x 12288 x 4096 184 / 186 / 171, 6140 x 6136 x 2048 161 / 158 / 143.  By counters the pieces of the first keep neither unit full
+// (matrix pipes 41 % of the cycles, LDS 42 %): one wave on a SIMD with half of a tile's work between two barriers, and 96 idle
+// compute units.
 template <class T, int EPI>
 __global__ __launch_bounds__(256, 1) void gemm16_pieces_kernel(const Gemm16Params p, int main_tiles, int pieces) {
   extern __shared__ __attribute__((aligned(16))) char smem[];

@@ -272,7 +272,7 @@ inline Gemm16Schedule second_opinion_mid(const Gemm16Schedule& first, const Gemm
 // Stacks of products whose 128 x 128 tiles leave half of the compute units idle go on 64 x 64 ones, while K is short: a
 // step of those reads twice the operands per result, from the caches all of them share.  (90 stacks of 2 to 64 products of
 // 16 to 1024 rows, forced: on average 2 % behind the best tile instead of 12, none more than 4 % behind what it had; 4 of
-// 124 x 560 x 176 5.0 -> 3.4 us, 4 of 128 x 256 x 64 4.2 -> 3.4.  13 of 141 x 376 x 704 9.3 us on 128 x 128, 10.0 on 64 x 64; 25 of 384 x 256 x 448, 150 tiles, 8.8 and 10.9.)
+// 124 x 560 x 176 5.0 -> 3.4 us, 4 of 128 x 256 x 64 4.2 -> 3.4, on the device; a caller in Python sees 4.2 either way, the call's host path.  13 of 141 x 376 x 704 9.3 us on 128 x 128, 10.0 on 64 x 64; 25 of 384 x 256 x 448, 150 tiles, 8.8 and 10.9.)
 inline bool small_tiles_for_stack(long tiles128, int K, int batch) { return batch > 1 && tiles128 < 128 && K <= 640; }
 
 // Workgroups of the few-row kernel on 128-column strips with K in as many parts as keep it within one workgroup
@@ -308,6 +308,9 @@ inline int skinny_loose_splits(int N, int K) {
 // of its experts 14 us whole, 11 in two parts; 2000 times the same one 7.3 and 8.6).
 // Drawn products of up to 64 rows, libraries with and without unequal parts in turn: with them 1.20 times as fast, 12 of 827 more than 3 %
 // slower.
+// (These lines stand between times of calls repeated on one matrix, from the caches, where the second launch counts in full.  With weights
+// from memory and the launches queued up two parts are ahead below them too, 7 % on average over 41 drawn products, 18 x 2176 x
+// 1088 and its like by 0.5 us; with weights from memory called one by one, level over 43.)
 inline bool unequal_parts_pay(long tiles, int N, int K, int splits, int equal) {
   const bool lines = N % 64 == 0;
   if (3 * equal >= 2 * splits) return false;
